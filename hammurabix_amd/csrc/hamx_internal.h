@@ -96,6 +96,8 @@ enum Slot : int {
   kSlotSyncIO,    // hamx_sync_kernels staging (x, F, G)
   kSlotCreOut,    // hamx_cre_write_grid output staging
   kSlotFlag,      // hamx_los_forward's non-finite output flag
+  kSlotRndHalf,   // half spectra of the random-field generators
+  kSlotRndPart,   // partial sums of the generators' variance
   kSlotCount
 };
 static_assert(kSlotCount <= hamx_ctx::kSlots, "workspace slots");

@@ -1,14 +1,15 @@
 // Gaussian random fields on gfx950: Brnd_es::write_grid (brnd_es.cc:76-308)
 // and TErnd_dft::write_grid (ternd_dft.cc:35-128).
 //
-// Pipeline (every step a grid-stride elementwise kernel over the N vertices,
-// or the LDS Stockham FFT of hamx_fft.hip):
-//   ES : draw c0,c1 -> FFT(+) -> variance -> rescale+anisotropy -> FFT(-)
-//        -> Gram-Schmidt (b = sqrt2 * GS(Re part)) -> reassemble -> FFT(+)
-//        -> Hermitian extraction / N
-//   DFT: draw te_k -> FFT(+) -> variance -> rescale
-// The variance stays on the device (two-stage reduction), so the pipeline is
-// one stream of launches with no host round trip.
+// Steps (Brnd_es; Brnd_jf12 the same, TErnd_dft and Brnd_mhd a part of them):
+//   draw c0,c1 -> FFT(+) -> variance -> rescale+anisotropy -> FFT(-)
+//   -> Gram-Schmidt (b = sqrt2 * GS(Re part)) -> reassemble -> FFT(+)
+//   -> Hermitian extraction / N
+// Each elementwise step runs inside the axis pass beside it, and everything
+// after the rescale runs on half spectra of real even fields ("half-space
+// passes" below); boxes with an axis too long for those tiles take the
+// steps one by one on whole complex arrays.  The variance stays on the
+// device, so a realisation is one stream of launches with no host round trip.
 //
 // Gaussian variates: Philox4x32-10 (Salmon, Moraes, Dror, Shaw, SC'11)
 // keyed by the seed, counter = (pair index, stream), two 53-bit uniforms per
@@ -22,6 +23,7 @@
 
 #include "hamx.h"
 #include "hamx_cgs.h"
+#include "hamx_fft.h"
 #include "hamx_fields.h"
 #include "hamx_internal.h"
 #include "hamx_math.h"
@@ -140,6 +142,15 @@ __device__ inline double wavenum(uint64_t i, uint64_t n, double len) {
   return k;
 }
 
+// |k| of mode (i, j, l).  The bands compare it strictly with their edges,
+// which lattice modes can tie exactly: every path forms it in this order.
+__device__ inline double mode_k(double kx, double ky, double kz) {
+  return sqrt(kx * kx + ky * ky + kz * kz);
+}
+__device__ inline double mode_k(const BoxArgs &a, uint64_t i, uint64_t j, uint64_t l) {
+  return mode_k(wavenum(i, a.nx, a.lx), wavenum(j, a.ny, a.ly), wavenum(l, a.nz, a.lz));
+}
+
 // Vertex position (brnd_es.cc:165-173: vertex spacing L/(n-1)).
 __device__ inline Vec3 vertex_pos(const BoxArgs &a, uint64_t i, uint64_t j,
                                   uint64_t l) {
@@ -171,8 +182,10 @@ __device__ inline uint64_t sym_index(const BoxArgs &a, uint64_t idx) {
 // block combines the partials and writes the result to out[slot].
 constexpr int kRedBlocks = 1024;
 
+// The workgroup's sum, in every thread.
+template <uint32_t NT>
 __device__ inline double block_sum(double v) {
-  __shared__ double sm[4];
+  __shared__ double sm[NT / 64];
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1)
     v += __shfl_xor(v, o, 64);
@@ -181,8 +194,9 @@ __device__ inline double block_sum(double v) {
     sm[w] = v;
   __syncthreads();
   double t = 0.;
-  if (threadIdx.x == 0)
-    t = sm[0] + sm[1] + sm[2] + sm[3];
+#pragma unroll
+  for (uint32_t i = 0; i < NT / 64; ++i)
+    t += sm[i];
   __syncthreads();
   return t;
 }
@@ -198,7 +212,7 @@ __global__ __launch_bounds__(256) void k_partial(const double *x, uint64_t n,
     const double v = x[i];
     acc += mean ? (v - m) * (v - m) : v;
   }
-  const double t = block_sum(acc);
+  const double t = block_sum<256>(acc);
   if (threadIdx.x == 0)
     partials[blockIdx.x] = t;
 }
@@ -208,7 +222,7 @@ __global__ __launch_bounds__(256) void k_final(const double *partials, int np,
   double acc = 0.;
   for (int i = threadIdx.x; i < np; i += blockDim.x)
     acc += partials[i];
-  const double t = block_sum(acc);
+  const double t = block_sum<256>(acc);
   if (threadIdx.x == 0)
     out[0] = t / static_cast<double>(n);
 }
@@ -263,6 +277,11 @@ __device__ inline double es_spectrum(const EsArgs &a, double k) {
   return P * p0 * unit;
 }
 
+// The standard deviation of a mode's two components (brnd_es.cc:127-133).
+__device__ inline double es_sigma(const EsArgs &a, double k) {
+  return sqrt(a.third * es_spectrum(a, k) * a.b.dk3);
+}
+
 // Brnd_jf12::spatial_profile (brnd_jf12.cc:54-114): the squared disk (JF12
 // spiral regions as in the regular field, b0_int inside 5 kpc, Gaussian in
 // z) and halo amplitudes, in muG^2; 0 outside r < 20 kpc, |pos| > 1 kpc.
@@ -308,11 +327,7 @@ __global__ __launch_bounds__(256) void k_es_draw(double2 *c0, double2 *c1,
     }
     uint64_t i, j, l;
     box_ijl(a.b, idx, i, j, l);
-    const double kx = wavenum(i, a.b.nx, a.b.lx);
-    const double ky = wavenum(j, a.b.ny, a.b.ly);
-    const double kz = wavenum(l, a.b.nz, a.b.lz);
-    const double ks = sqrt(kx * kx + ky * ky + kz * kz);
-    const double sigma = sqrt(a.third * es_spectrum(a, ks) * a.b.dk3);
+    const double sigma = es_sigma(a, mode_k(a.b, i, j, l));
     double g0, g1, g2, g3;
     gauss_pair(seed, 0, 2 * idx, g0, g1);
     gauss_pair(seed, 0, 2 * idx + 1, g2, g3);
@@ -321,64 +336,81 @@ __global__ __launch_bounds__(256) void k_es_draw(double2 *c0, double2 *c1,
   }
 }
 
-// STEP II (brnd_es.cc:157-205).  HEAVY compiles in the JF12 energy profile,
-// the JF12 / Jaffe regular fields and the imported regular-field grid; the
-// light kernel (LSA, cartesian, uniform, helix fields and the ES profile)
-// then keeps few enough registers for several waves per SIMD.
+// STEP II (brnd_es.cc:157-205) at one vertex: v0 and v1 are the transformed
+// c0 and c1 there; false where the regular field is zero and the raw values
+// stay, else b is the rescaled field.  HEAVY compiles in the JF12 energy
+// profile, the JF12 / Jaffe regular fields and the imported regular-field
+// grid; the light form (LSA, cartesian, uniform, helix fields and the ES
+// profile) then keeps few enough registers for several waves per SIMD.
+struct EsScale {
+  double b_var_invsq, rho, inv_rho, rhonorm;
+};
+
+__device__ inline EsScale es_scale(const EsArgs &a, const double *var) {
+  const double rho2 = a.rho * a.rho;
+  return EsScale{1. / sqrt(3. * var[0]), a.rho, 1. / a.rho,
+                 1. / sqrt(a.third * rho2 + a.twothirds / rho2)};
+}
+
+template <bool HEAVY>
+__device__ inline bool es_rescale_at(const EsArgs &a, const EsScale &sc, uint64_t i, uint64_t j,
+                                     uint64_t l, const double2 &v0, const double2 &v1, Vec3 &b) {
+  const Vec3 pos = vertex_pos(a.b, i, j, l);
+  const double prof =
+      (HEAVY && a.jf12) ? jf12_profile(a.jp, pos) : profile(a.obs, a.r0, a.z0, pos);
+  const double ratio = sqrt(prof) * a.rms * sc.b_var_invsq;
+  b = Vec3{v0.x * ratio, v0.y * ratio, v1.y * ratio};
+  // anisotropy direction: versor of the regular field (brnd_es.cc:19-22)
+  Vec3 braw;
+  if (HEAVY && a.breg_model == HAMX_BREG_GRID) {
+    Cell c;
+    if (grid_cell(a.g_breg, pos, c)) {
+      const uint64_t sy = a.g_breg.nz, sx = a.g_breg.ny * a.g_breg.nz;
+      braw = Vec3{lerp_cell(a.bgx, c, sy, sx), lerp_cell(a.bgy, c, sy, sx),
+                  lerp_cell(a.bgz, c, sy, sx)};
+    } else {
+      braw = Vec3{0., 0., 0.};
+    }
+  } else {
+    braw = breg_eval<HEAVY>(a.breg_model, a.breg, pos);
+  }
+  Vec3 H{0., 0., 0.};
+  double l2 = 0.;
+  l2 += braw.x * braw.x;
+  l2 += braw.y * braw.y;
+  l2 += braw.z * braw.z;
+  if (l2 != 0) {
+    const double den = 1. / sqrt(l2);
+    H = Vec3{braw.x * den, braw.y * den, braw.z * den};
+  }
+  double h2 = 0.;
+  h2 += H.x * H.x;
+  h2 += H.y * H.y;
+  h2 += H.z * H.z;
+  if (h2 < 1e-10)
+    return false;
+  const double hb = dot0(H, b);
+  const Vec3 par{H.x * hb, H.y * hb, H.z * hb};
+  const Vec3 perp{b.x - par.x, b.y - par.y, b.z - par.z};
+  b = Vec3{(par.x * sc.rho + perp.x * sc.inv_rho) * sc.rhonorm,
+           (par.y * sc.rho + perp.y * sc.inv_rho) * sc.rhonorm,
+           (par.z * sc.rho + perp.z * sc.inv_rho) * sc.rhonorm};
+  return true;
+}
+
 template <bool HEAVY>
 __global__ __launch_bounds__(256) void k_es_rescale(double2 *c0, double2 *c1,
                                                     EsArgs a, const double *var) {
-  const double b_var_invsq = 1. / sqrt(3. * var[0]);
-  const double rho = a.rho;
-  const double rho2 = rho * rho;
-  const double rhonorm = 1. / sqrt(a.third * rho2 + a.twothirds / rho2);
-  const double inv_rho = 1. / rho;
+  const EsScale sc = es_scale(a, var);
   const uint64_t stride = static_cast<uint64_t>(gridDim.x) * blockDim.x;
   for (uint64_t idx = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
        idx < a.b.n; idx += stride) {
     uint64_t i, j, l;
     box_ijl(a.b, idx, i, j, l);
-    const Vec3 pos = vertex_pos(a.b, i, j, l);
-    const double prof =
-        (HEAVY && a.jf12) ? jf12_profile(a.jp, pos) : profile(a.obs, a.r0, a.z0, pos);
-    const double ratio = sqrt(prof) * a.rms * b_var_invsq;
     const double2 v0 = c0[idx], v1 = c1[idx];
-    Vec3 b{v0.x * ratio, v0.y * ratio, v1.y * ratio};
-    // anisotropy direction: versor of the regular field (brnd_es.cc:19-22)
-    Vec3 braw;
-    if (HEAVY && a.breg_model == HAMX_BREG_GRID) {
-      Cell c;
-      if (grid_cell(a.g_breg, pos, c)) {
-        const uint64_t sy = a.g_breg.nz, sx = a.g_breg.ny * a.g_breg.nz;
-        braw = Vec3{lerp_cell(a.bgx, c, sy, sx), lerp_cell(a.bgy, c, sy, sx),
-                    lerp_cell(a.bgz, c, sy, sx)};
-      } else {
-        braw = Vec3{0., 0., 0.};
-      }
-    } else {
-      braw = breg_eval<HEAVY>(a.breg_model, a.breg, pos);
-    }
-    Vec3 H{0., 0., 0.};
-    double l2 = 0.;
-    l2 += braw.x * braw.x;
-    l2 += braw.y * braw.y;
-    l2 += braw.z * braw.z;
-    if (l2 != 0) {
-      const double den = 1. / sqrt(l2);
-      H = Vec3{braw.x * den, braw.y * den, braw.z * den};
-    }
-    double h2 = 0.;
-    h2 += H.x * H.x;
-    h2 += H.y * H.y;
-    h2 += H.z * H.z;
-    if (h2 < 1e-10)
+    Vec3 b;
+    if (!es_rescale_at<HEAVY>(a, sc, i, j, l, v0, v1, b))
       continue; // zero regular field: the raw FFT values stay
-    const double hb = dot0(H, b);
-    const Vec3 par{H.x * hb, H.y * hb, H.z * hb};
-    const Vec3 perp{b.x - par.x, b.y - par.y, b.z - par.z};
-    b = Vec3{(par.x * rho + perp.x * inv_rho) * rhonorm,
-             (par.y * rho + perp.y * inv_rho) * rhonorm,
-             (par.z * rho + perp.z * inv_rho) * rhonorm};
     c0[idx] = make_double2(b.x, b.y);
     c1[idx] = make_double2(b.y, b.z);
   }
@@ -386,11 +418,7 @@ __global__ __launch_bounds__(256) void k_es_rescale(double2 *c0, double2 *c1,
 
 // STEP III Gram-Schmidt (brnd_es.cc:211-259) of the symmetrised vector b at
 // index idx: the part of b normal to the wave vector, times sqrt(3).
-__device__ inline Vec3 es_gs_at(const EsArgs &a, uint64_t idx, const Vec3 &b) {
-  uint64_t i, j, l;
-  box_ijl(a.b, idx, i, j, l);
-  const Vec3 k{wavenum(i, a.b.nx, a.b.lx), wavenum(j, a.b.ny, a.b.ly),
-               wavenum(l, a.b.nz, a.b.lz)};
+__device__ inline Vec3 es_gs(const EsArgs &a, const Vec3 &k, const Vec3 &b) {
   double k2 = 0.;
   k2 += k.x * k.x;
   k2 += k.y * k.y;
@@ -405,6 +433,15 @@ __device__ inline Vec3 es_gs_at(const EsArgs &a, uint64_t idx, const Vec3 &b) {
   const double kb = dot0(k, b);
   return Vec3{a.sqrt3 * (b.x - k.x * kb * inv), a.sqrt3 * (b.y - k.y * kb * inv),
               a.sqrt3 * (b.z - k.z * kb * inv)};
+}
+
+__device__ inline Vec3 es_gs_at(const EsArgs &a, uint64_t idx, const Vec3 &b) {
+  uint64_t i, j, l;
+  box_ijl(a.b, idx, i, j, l);
+  return es_gs(a,
+               Vec3{wavenum(i, a.b.nx, a.b.lx), wavenum(j, a.b.ny, a.b.ly),
+                    wavenum(l, a.b.nz, a.b.lz)},
+               b);
 }
 
 // STEP III and the reassembly c0 = bx + i by, c1 = by + i bz with
@@ -475,6 +512,10 @@ __device__ inline double dft_spectrum(const DftArgs &a, double k) {
   return a.rms * exp(a.a0 * log(k / a.k0)) / (4 * cgs::pi * k * k); // (k / k0)^a0
 }
 
+__device__ inline double dft_sigma(const DftArgs &a, double k) {
+  return sqrt(dft_spectrum(a, k) * a.b.dk3);
+}
+
 __global__ __launch_bounds__(256) void k_dft_draw(double2 *tk, DftArgs a,
                                                   uint64_t seed) {
   const uint64_t stride = static_cast<uint64_t>(gridDim.x) * blockDim.x;
@@ -486,15 +527,18 @@ __global__ __launch_bounds__(256) void k_dft_draw(double2 *tk, DftArgs a,
     }
     uint64_t i, j, l;
     box_ijl(a.b, idx, i, j, l);
-    const double kx = wavenum(i, a.b.nx, a.b.lx);
-    const double ky = wavenum(j, a.b.ny, a.b.ly);
-    const double kz = wavenum(l, a.b.nz, a.b.lz);
-    const double ks = sqrt(kx * kx + ky * ky + kz * kz);
-    const double sigma = sqrt(dft_spectrum(a, ks) * a.b.dk3);
+    const double sigma = dft_sigma(a, mode_k(a.b, i, j, l));
     double g0, g1;
     gauss_pair(seed, 1, idx, g0, g1);
     tk[idx] = make_double2(sigma * g0, sigma * g1);
   }
+}
+
+// The energy profile's factor at a vertex (ternd_dft.cc:117-125).
+__device__ inline double dft_ratio(const DftArgs &a, uint64_t i, uint64_t j, uint64_t l,
+                                   double te_var_invsq) {
+  const Vec3 pos = vertex_pos(a.b, i, j, l);
+  return sqrt(profile(a.obs, a.r0, a.z0, pos)) * a.rms * te_var_invsq;
 }
 
 __global__ __launch_bounds__(256) void k_dft_rescale(const double2 *tk, double *te,
@@ -505,11 +549,170 @@ __global__ __launch_bounds__(256) void k_dft_rescale(const double2 *tk, double *
        idx < a.b.n; idx += stride) {
     uint64_t i, j, l;
     box_ijl(a.b, idx, i, j, l);
-    const Vec3 pos = vertex_pos(a.b, i, j, l);
-    const double ratio = sqrt(profile(a.obs, a.r0, a.z0, pos)) * a.rms * te_var_invsq;
-    te[idx] = tk[idx].x * ratio;
+    te[idx] = tk[idx].x * dft_ratio(a, i, j, l, te_var_invsq);
   }
 }
+
+// -------------------------------------------------------------- Brnd_mhd --
+// Brnd_mhd::write_grid (brnd_mhd.cc:16-167): Alfven, fast and slow modes
+// about the regular field at the observer, drawn in k-space and brought back
+// by one backward transform per complex array; no energy-profile rescale.
+struct MhdArgs {
+  BoxArgs b;
+  double pa0, pf0, ps0, k0, k1, aa0, af0, as0, a1, beta, ma;
+};
+
+// Brnd_mhd::spectrum_a / _f / _s (brnd_mhd.cc:211-262): one form, the mode
+// choosing its index a0 and norm p0.
+__device__ inline double mhd_spectrum(const MhdArgs &a, double k, double a0, double p0) {
+  const double unit = 0.25 / (cgs::pi * k * k);
+  const double band1 = static_cast<double>(k < a.k1);
+  const double band2 = static_cast<double>(k > a.k1) * static_cast<double>(k < a.k0);
+  const double band3 = static_cast<double>(k > a.k0);
+  const double P = band1 * pow(a.k0 / a.k1, a.a1) * pow(k / a.k1, 6.0) +
+                   band2 / pow(k / a.k0, a.a1) + band3 / pow(k / a.k0, a0);
+  return P * p0 * unit;
+}
+
+// dynamo, h_s, h_f, F_a = F_s (bfield.h:388-412, brnd_mhd.cc:181-209)
+__device__ inline double mhd_dynamo(double beta, double c) {
+  return 1 + 0.25 * beta * beta + beta * (1. - 2. * c * c);
+}
+__device__ inline double mhd_h_s(double beta, double c) {
+  const double sq = sqrt(mhd_dynamo(beta, c));
+  const double dpp = 1 + sq + 0.5 * beta;
+  const double dmm = 1 - sq - 0.5 * beta;
+  const double dmp = 1 - sq + 0.5 * beta;
+  const double den = 1 / (dmp * (c * c + dpp * dpp * (1 - c * c) / (dmm * dmm)));
+  return isfinite(den) ? 2. * c * c * den * static_cast<double>(den > 0) : 0.;
+}
+__device__ inline double mhd_h_f(double beta, double c) {
+  if (c == 0)
+    return 0;
+  const double sq = sqrt(mhd_dynamo(beta, c));
+  const double dpp = 1 + sq + 0.5 * beta;
+  const double dpm = 1 + sq - 0.5 * beta;
+  const double dmp = 1 - sq + 0.5 * beta;
+  const double den = 1 / (dpp * (c * c + dmp * dmp * (1 - c * c) / (dpm * dpm)));
+  return isfinite(den) ? 2. * c * c * den : 0.;
+}
+__device__ inline double mhd_aniso(double ma, double c) {
+  return exp(-1. * pow(ma, -1.33333333) * fabs(c) / pow(1 - c * c, 0.33333333));
+}
+
+// Hamvec::versor and crossprod (hamvec.h:176-205)
+__device__ inline Vec3 versor3(const Vec3 &v) {
+  double l2 = 0.;
+  l2 += v.x * v.x;
+  l2 += v.y * v.y;
+  l2 += v.z * v.z;
+  if (l2 == 0)
+    return Vec3{0., 0., 0.};
+  const double den = 1. / sqrt(l2);
+  return Vec3{v.x * den, v.y * den, v.z * den};
+}
+__device__ inline Vec3 cross3(const Vec3 &a, const Vec3 &b) {
+  return Vec3{a.y * b.z - a.z * b.y, a.z * b.x - a.x * b.z, a.x * b.y - a.y * b.x};
+}
+// Brnd_mhd::e_plus / e_minus (brnd_mhd.cc:169-179): normalised unless
+// their squared length is below 1e-12
+__device__ inline Vec3 unit_or_small(const Vec3 &t) {
+  double l2 = 0.;
+  l2 += t.x * t.x;
+  l2 += t.y * t.y;
+  l2 += t.z * t.z;
+  if (l2 < 1e-12)
+    return t;
+  const double l = sqrt(l2);
+  return Vec3{t.x / l, t.y / l, t.z / l};
+}
+
+// The regular field at the observer (breg->read_field(observer)).
+__global__ void k_mhd_bobs(EsArgs a, double *out) {
+  if (blockIdx.x != 0 || threadIdx.x != 0)
+    return;
+  Vec3 b{0., 0., 0.};
+  if (a.breg_model == HAMX_BREG_GRID) {
+    Cell c;
+    if (grid_cell(a.g_breg, a.obs, c)) {
+      const uint64_t sy = a.g_breg.nz, sx = a.g_breg.ny * a.g_breg.nz;
+      b = Vec3{lerp_cell(a.bgx, c, sy, sx), lerp_cell(a.bgy, c, sy, sx),
+               lerp_cell(a.bgz, c, sy, sx)};
+    }
+  } else {
+    b = breg_eval(a.breg_model, a.breg, a.obs);
+  }
+  out[0] = b.x;
+  out[1] = b.y;
+  out[2] = b.z;
+}
+
+// Philox streams of the MHD draws: Gaussians (2 pairs per mode) and the
+// fast/slow power share of the modes along the field.
+constexpr uint32_t kMhdGaussStream = 3, kMhdShareStream = 4;
+
+// The field amplitude of mode (i, j, l), flat index idx (brnd_mhd.cc:54-137);
+// bh is the regular field's versor at the observer.
+__device__ inline Vec3 mhd_mode(const MhdArgs &a, uint64_t seed, const Vec3 &bh, uint64_t idx,
+                                uint64_t i, uint64_t j, uint64_t l) {
+  if (idx == 0)
+    return Vec3{0., 0., 0.};
+  const Vec3 k{wavenum(i, a.b.nx, a.b.lx), wavenum(j, a.b.ny, a.b.ly),
+               wavenum(l, a.b.nz, a.b.lz)};
+  const double ks = length0(k);
+  const Vec3 kh = versor3(k);
+  const Vec3 kxb = cross3(kh, bh);
+  Vec3 ep = unit_or_small(kxb);
+  Vec3 em = unit_or_small(cross3(kxb, kh));
+  const double dk3 = a.b.dk3;
+  double g0, g1, g2, g3;
+  gauss_pair(seed, kMhdGaussStream, 2 * idx, g0, g1);
+  if (dot0(ep, ep) > 1e-6) {
+    const double ang = dot0(bh, kh);
+    const double Pa = mhd_spectrum(a, ks, a.aa0, a.pa0) * mhd_aniso(a.ma, ang) * dk3;
+    const double Pf = mhd_spectrum(a, ks, a.af0, a.pf0) * mhd_h_f(a.beta, ang) * dk3;
+    const double Ps = mhd_spectrum(a, ks, a.as0, a.ps0) * mhd_aniso(a.ma, ang) *
+                      mhd_h_s(a.beta, ang) * dk3;
+    gauss_pair(seed, kMhdGaussStream, 2 * idx + 1, g2, g3);
+    const double Ap = g0 * sqrt(2. * Pa);
+    const double Am = g1 * sqrt(2. * Pf) + g2 * sqrt(2. * Ps);
+    return Vec3{ep.x * Ap + em.x * Am, ep.y * Ap + em.y * Am, ep.z * Ap + em.z * Am};
+  }
+  const double Pf = mhd_spectrum(a, ks, a.af0, a.pf0) * mhd_h_f(a.beta, 1) * dk3;
+  if (i == 0 && j == 0) {
+    ep.x = k.x;
+    em.y = k.y;
+  } else {
+    const double kp = sqrt(k.x * k.x + k.y * k.y);
+    ep = Vec3{k.x * k.z / (ks * kp), k.y * k.z / (ks * kp), -kp / ks};
+    em = Vec3{-k.y / kp, k.x / kp, 0.};
+  }
+  const double Af = g0 * sqrt(2. * Pf);
+  const double share = philox_uniform(seed, kMhdShareStream, idx);
+  return Vec3{ep.x * Af * share + em.x * Af * (1. - share),
+              ep.y * Af * share + em.y * Af * (1. - share),
+              ep.z * Af * share + em.z * Af * (1. - share)};
+}
+
+__global__ __launch_bounds__(256) void k_mhd_draw(double2 *c0, double2 *c1, MhdArgs a,
+                                                  uint64_t seed, const double *bobs) {
+  const uint64_t stride = static_cast<uint64_t>(gridDim.x) * blockDim.x;
+  const Vec3 bh = versor3(Vec3{bobs[0], bobs[1], bobs[2]});
+  for (uint64_t idx = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+       idx < a.b.n; idx += stride) {
+    uint64_t i, j, l;
+    box_ijl(a.b, idx, i, j, l);
+    const Vec3 bk = mhd_mode(a, seed, bh, idx, i, j, l);
+    c0[idx] = double2{bk.x, bk.y};
+    c1[idx] = double2{bk.y, bk.z};
+  }
+}
+
+} // namespace hamx
+
+#include "hamx_rnd_half.h"
+
+namespace hamx {
 
 // ------------------------------------------------------------------- host --
 static unsigned ew_blocks(uint64_t n) {
@@ -617,6 +820,10 @@ int brnd_generate(hamx_ctx *ctx, const hamx_es_desc *d, uint64_t seed, double *b
     a.g_breg = grid_geo(d->breg_box);
   }
   const uint64_t n = a.b.n;
+  HalfPlan hp;
+  int rc;
+  bool half = half_plan(ctx, a.b, &hp, &rc);
+  HAMX_TRY(rc);
   void *w;
   HAMX_TRY(ws_get(ctx, kSlotRndC0, n * sizeof(double2), &w));
   double2 *c0 = static_cast<double2 *>(w);
@@ -633,27 +840,45 @@ int brnd_generate(hamx_ctx *ctx, const hamx_es_desc *d, uint64_t seed, double *b
     HAMX_TRY(ws_get(ctx, kSlotRndOut2, n * sizeof(double), &w));
     oz = static_cast<double *>(w);
   }
-  const unsigned blocks = ew_blocks(n);
-  hipLaunchKernelGGL(k_es_draw, dim3(blocks), dim3(256), 0, ctx->stream, c0, c1, a, seed);
-  HAMX_HIP(ctx, hipGetLastError());
-  HAMX_TRY(fft3d_dev2(ctx, c0, c1, a.b.nx, a.b.ny, a.b.nz, +1));
-  HAMX_TRY(variance_dev(ctx, reinterpret_cast<const double *>(c0), n, red));
   const bool heavy = a.jf12 || a.breg_model == HAMX_BREG_GRID ||
                      a.breg_model == HAMX_BREG_JF12 || a.breg_model == HAMX_BREG_JAFFE;
-  if (heavy)
-    hipLaunchKernelGGL(k_es_rescale<true>, dim3(blocks), dim3(256), 0, ctx->stream, c0, c1, a,
-                       static_cast<const double *>(red + 1));
+  const double inv_n = 1. / static_cast<double>(n);
+  // without room for the half arrays beside c0 and c1: the whole-array steps
+  void *hw = nullptr;
+  if (half && (rc = ws_get(ctx, kSlotRndHalf, half_bytes(hp), &hw)) == HAMX_ERR_NOMEM)
+    half = false;
   else
-    hipLaunchKernelGGL(k_es_rescale<false>, dim3(blocks), dim3(256), 0, ctx->stream, c0, c1,
-                       a, static_cast<const double *>(red + 1));
-  HAMX_HIP(ctx, hipGetLastError());
-  HAMX_TRY(fft3d_dev2(ctx, c0, c1, a.b.nx, a.b.ny, a.b.nz, -1));
-  hipLaunchKernelGGL(k_es_gs_pairs, dim3(blocks), dim3(256), 0, ctx->stream, c0, c1, a);
-  HAMX_HIP(ctx, hipGetLastError());
-  HAMX_TRY(fft3d_dev2(ctx, c0, c1, a.b.nx, a.b.ny, a.b.nz, +1));
-  hipLaunchKernelGGL(k_es_final, dim3(blocks), dim3(256), 0, ctx->stream, c0, c1, ox,
-                     oy, oz, a.b, 1. / static_cast<double>(n));
-  HAMX_HIP(ctx, hipGetLastError());
+    HAMX_TRY(rc);
+  if (half) {
+    const HalfArrays H = half_arrays(hp, hw);
+    HAMX_TRY(half_draw(ctx, hp, EsDraw{a}, seed, c0, c1, red));
+    HAMX_TRY(heavy ? half_mid<true>(ctx, hp, c0, c1, H, a, red + 1)
+                   : half_mid<false>(ctx, hp, c0, c1, H, a, red + 1));
+    HAMX_TRY(half_y(ctx, hp, H, -1));
+    HAMX_TRY(half_gs_x(ctx, hp, H, a));
+    HAMX_TRY(half_y(ctx, hp, H, +1));
+    HAMX_TRY(half_out(ctx, hp, H, ox, oy, oz, inv_n));
+  } else {
+    const unsigned blocks = ew_blocks(n);
+    hipLaunchKernelGGL(k_es_draw, dim3(blocks), dim3(256), 0, ctx->stream, c0, c1, a, seed);
+    HAMX_HIP(ctx, hipGetLastError());
+    HAMX_TRY(fft3d_dev2(ctx, c0, c1, a.b.nx, a.b.ny, a.b.nz, +1));
+    HAMX_TRY(variance_dev(ctx, reinterpret_cast<const double *>(c0), n, red));
+    if (heavy)
+      hipLaunchKernelGGL(k_es_rescale<true>, dim3(blocks), dim3(256), 0, ctx->stream, c0, c1, a,
+                         static_cast<const double *>(red + 1));
+    else
+      hipLaunchKernelGGL(k_es_rescale<false>, dim3(blocks), dim3(256), 0, ctx->stream, c0, c1,
+                         a, static_cast<const double *>(red + 1));
+    HAMX_HIP(ctx, hipGetLastError());
+    HAMX_TRY(fft3d_dev2(ctx, c0, c1, a.b.nx, a.b.ny, a.b.nz, -1));
+    hipLaunchKernelGGL(k_es_gs_pairs, dim3(blocks), dim3(256), 0, ctx->stream, c0, c1, a);
+    HAMX_HIP(ctx, hipGetLastError());
+    HAMX_TRY(fft3d_dev2(ctx, c0, c1, a.b.nx, a.b.ny, a.b.nz, +1));
+    hipLaunchKernelGGL(k_es_final, dim3(blocks), dim3(256), 0, ctx->stream, c0, c1, ox,
+                       oy, oz, a.b, inv_n);
+    HAMX_HIP(ctx, hipGetLastError());
+  }
   if (!out_dev) {
     HAMX_HIP(ctx, hipMemcpyAsync(bx, ox, n * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
     HAMX_HIP(ctx, hipMemcpyAsync(by, oy, n * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
@@ -661,159 +886,6 @@ int brnd_generate(hamx_ctx *ctx, const hamx_es_desc *d, uint64_t seed, double *b
   }
   HAMX_HIP(ctx, hipStreamSynchronize(ctx->stream));
   return HAMX_OK;
-}
-// -------------------------------------------------------------- Brnd_mhd --
-// Brnd_mhd::write_grid (brnd_mhd.cc:16-167): Alfven, fast and slow modes
-// about the regular field at the observer, drawn in k-space and brought back
-// by one backward transform per complex array; no energy-profile rescale.
-struct MhdArgs {
-  BoxArgs b;
-  double pa0, pf0, ps0, k0, k1, aa0, af0, as0, a1, beta, ma;
-};
-
-// Brnd_mhd::spectrum_a / _f / _s (brnd_mhd.cc:211-262): one form, the mode
-// choosing its index a0 and norm p0.
-__device__ inline double mhd_spectrum(const MhdArgs &a, double k, double a0, double p0) {
-  const double unit = 0.25 / (cgs::pi * k * k);
-  const double band1 = static_cast<double>(k < a.k1);
-  const double band2 = static_cast<double>(k > a.k1) * static_cast<double>(k < a.k0);
-  const double band3 = static_cast<double>(k > a.k0);
-  const double P = band1 * pow(a.k0 / a.k1, a.a1) * pow(k / a.k1, 6.0) +
-                   band2 / pow(k / a.k0, a.a1) + band3 / pow(k / a.k0, a0);
-  return P * p0 * unit;
-}
-
-// dynamo, h_s, h_f, F_a = F_s (bfield.h:388-412, brnd_mhd.cc:181-209)
-__device__ inline double mhd_dynamo(double beta, double c) {
-  return 1 + 0.25 * beta * beta + beta * (1. - 2. * c * c);
-}
-__device__ inline double mhd_h_s(double beta, double c) {
-  const double sq = sqrt(mhd_dynamo(beta, c));
-  const double dpp = 1 + sq + 0.5 * beta;
-  const double dmm = 1 - sq - 0.5 * beta;
-  const double dmp = 1 - sq + 0.5 * beta;
-  const double den = 1 / (dmp * (c * c + dpp * dpp * (1 - c * c) / (dmm * dmm)));
-  return isfinite(den) ? 2. * c * c * den * static_cast<double>(den > 0) : 0.;
-}
-__device__ inline double mhd_h_f(double beta, double c) {
-  if (c == 0)
-    return 0;
-  const double sq = sqrt(mhd_dynamo(beta, c));
-  const double dpp = 1 + sq + 0.5 * beta;
-  const double dpm = 1 + sq - 0.5 * beta;
-  const double dmp = 1 - sq + 0.5 * beta;
-  const double den = 1 / (dpp * (c * c + dmp * dmp * (1 - c * c) / (dpm * dpm)));
-  return isfinite(den) ? 2. * c * c * den : 0.;
-}
-__device__ inline double mhd_aniso(double ma, double c) {
-  return exp(-1. * pow(ma, -1.33333333) * fabs(c) / pow(1 - c * c, 0.33333333));
-}
-
-// Hamvec::versor and crossprod (hamvec.h:176-205)
-__device__ inline Vec3 versor3(const Vec3 &v) {
-  double l2 = 0.;
-  l2 += v.x * v.x;
-  l2 += v.y * v.y;
-  l2 += v.z * v.z;
-  if (l2 == 0)
-    return Vec3{0., 0., 0.};
-  const double den = 1. / sqrt(l2);
-  return Vec3{v.x * den, v.y * den, v.z * den};
-}
-__device__ inline Vec3 cross3(const Vec3 &a, const Vec3 &b) {
-  return Vec3{a.y * b.z - a.z * b.y, a.z * b.x - a.x * b.z, a.x * b.y - a.y * b.x};
-}
-// Brnd_mhd::e_plus / e_minus (brnd_mhd.cc:169-179): normalised unless
-// their squared length is below 1e-12
-__device__ inline Vec3 unit_or_small(const Vec3 &t) {
-  double l2 = 0.;
-  l2 += t.x * t.x;
-  l2 += t.y * t.y;
-  l2 += t.z * t.z;
-  if (l2 < 1e-12)
-    return t;
-  const double l = sqrt(l2);
-  return Vec3{t.x / l, t.y / l, t.z / l};
-}
-
-// The regular field at the observer (breg->read_field(observer)).
-__global__ void k_mhd_bobs(EsArgs a, double *out) {
-  if (blockIdx.x != 0 || threadIdx.x != 0)
-    return;
-  Vec3 b{0., 0., 0.};
-  if (a.breg_model == HAMX_BREG_GRID) {
-    Cell c;
-    if (grid_cell(a.g_breg, a.obs, c)) {
-      const uint64_t sy = a.g_breg.nz, sx = a.g_breg.ny * a.g_breg.nz;
-      b = Vec3{lerp_cell(a.bgx, c, sy, sx), lerp_cell(a.bgy, c, sy, sx),
-               lerp_cell(a.bgz, c, sy, sx)};
-    }
-  } else {
-    b = breg_eval(a.breg_model, a.breg, a.obs);
-  }
-  out[0] = b.x;
-  out[1] = b.y;
-  out[2] = b.z;
-}
-
-// Philox streams of the MHD draws: Gaussians (2 pairs per mode) and the
-// fast/slow power share of the modes along the field.
-constexpr uint32_t kMhdGaussStream = 3, kMhdShareStream = 4;
-
-__global__ __launch_bounds__(256) void k_mhd_draw(double2 *c0, double2 *c1, MhdArgs a,
-                                                  uint64_t seed, const double *bobs) {
-  const uint64_t stride = static_cast<uint64_t>(gridDim.x) * blockDim.x;
-  const Vec3 B{bobs[0], bobs[1], bobs[2]};
-  const Vec3 bh = versor3(B);
-  for (uint64_t idx = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-       idx < a.b.n; idx += stride) {
-    if (idx == 0) {
-      c0[0] = double2{0., 0.};
-      c1[0] = double2{0., 0.};
-      continue;
-    }
-    uint64_t i, j, l;
-    box_ijl(a.b, idx, i, j, l);
-    const Vec3 k{wavenum(i, a.b.nx, a.b.lx), wavenum(j, a.b.ny, a.b.ly),
-                 wavenum(l, a.b.nz, a.b.lz)};
-    const double ks = length0(k);
-    const Vec3 kh = versor3(k);
-    const Vec3 kxb = cross3(kh, bh);
-    Vec3 ep = unit_or_small(kxb);
-    Vec3 em = unit_or_small(cross3(kxb, kh));
-    const double dk3 = a.b.dk3;
-    double g0, g1, g2, g3;
-    gauss_pair(seed, kMhdGaussStream, 2 * idx, g0, g1);
-    Vec3 bk;
-    if (dot0(ep, ep) > 1e-6) {
-      const double ang = dot0(bh, kh);
-      const double Pa = mhd_spectrum(a, ks, a.aa0, a.pa0) * mhd_aniso(a.ma, ang) * dk3;
-      const double Pf = mhd_spectrum(a, ks, a.af0, a.pf0) * mhd_h_f(a.beta, ang) * dk3;
-      const double Ps = mhd_spectrum(a, ks, a.as0, a.ps0) * mhd_aniso(a.ma, ang) *
-                        mhd_h_s(a.beta, ang) * dk3;
-      gauss_pair(seed, kMhdGaussStream, 2 * idx + 1, g2, g3);
-      const double Ap = g0 * sqrt(2. * Pa);
-      const double Am = g1 * sqrt(2. * Pf) + g2 * sqrt(2. * Ps);
-      bk = Vec3{ep.x * Ap + em.x * Am, ep.y * Ap + em.y * Am, ep.z * Ap + em.z * Am};
-    } else {
-      const double Pf = mhd_spectrum(a, ks, a.af0, a.pf0) * mhd_h_f(a.beta, 1) * dk3;
-      if (i == 0 && j == 0) {
-        ep.x = k.x;
-        em.y = k.y;
-      } else {
-        const double kp = sqrt(k.x * k.x + k.y * k.y);
-        ep = Vec3{k.x * k.z / (ks * kp), k.y * k.z / (ks * kp), -kp / ks};
-        em = Vec3{-k.y / kp, k.x / kp, 0.};
-      }
-      const double Af = g0 * sqrt(2. * Pf);
-      const double share = philox_uniform(seed, kMhdShareStream, idx);
-      bk = Vec3{ep.x * Af * share + em.x * Af * (1. - share),
-                ep.y * Af * share + em.y * Af * (1. - share),
-                ep.z * Af * share + em.z * Af * (1. - share)};
-    }
-    c0[idx] = double2{bk.x, bk.y};
-    c1[idx] = double2{bk.y, bk.z};
-  }
 }
 
 int brnd_mhd(hamx_ctx *ctx, const hamx_mhd_desc *d, uint64_t seed, double *bx, double *by,
@@ -863,11 +935,11 @@ int brnd_mhd(hamx_ctx *ctx, const hamx_mhd_desc *d, uint64_t seed, double *bx, d
   a.beta = d->beta;
   a.ma = d->ma;
   const uint64_t n = a.b.n;
+  HalfPlan hp;
+  int rc;
+  const bool half = half_plan(ctx, a.b, &hp, &rc);
+  HAMX_TRY(rc);
   void *w;
-  HAMX_TRY(ws_get(ctx, kSlotRndC0, n * sizeof(double2), &w));
-  double2 *c0 = static_cast<double2 *>(w);
-  HAMX_TRY(ws_get(ctx, kSlotRndC1, n * sizeof(double2), &w));
-  double2 *c1 = static_cast<double2 *>(w);
   HAMX_TRY(ws_get(ctx, kSlotReduce, (16 + kRedBlocks) * sizeof(double), &w));
   double *bobs = static_cast<double *>(w);
   double *ox = bx, *oy = by, *oz = bz;
@@ -881,14 +953,26 @@ int brnd_mhd(hamx_ctx *ctx, const hamx_mhd_desc *d, uint64_t seed, double *bx, d
   }
   hipLaunchKernelGGL(k_mhd_bobs, dim3(1), dim3(64), 0, ctx->stream, e, bobs);
   HAMX_HIP(ctx, hipGetLastError());
-  const unsigned blocks = ew_blocks(n);
-  hipLaunchKernelGGL(k_mhd_draw, dim3(blocks), dim3(256), 0, ctx->stream, c0, c1, a, seed,
-                     static_cast<const double *>(bobs));
-  HAMX_HIP(ctx, hipGetLastError());
-  HAMX_TRY(fft3d_dev2(ctx, c0, c1, a.b.nx, a.b.ny, a.b.nz, +1));
-  hipLaunchKernelGGL(k_es_final, dim3(blocks), dim3(256), 0, ctx->stream, c0, c1, ox, oy, oz,
-                     a.b, 1.);
-  HAMX_HIP(ctx, hipGetLastError());
+  if (half) {
+    HAMX_TRY(ws_get(ctx, kSlotRndHalf, half_bytes(hp), &w));
+    const HalfArrays H = half_arrays(hp, w);
+    HAMX_TRY(half_mhd_x(ctx, hp, H, a, seed, bobs));
+    HAMX_TRY(half_y(ctx, hp, H, +1));
+    HAMX_TRY(half_out(ctx, hp, H, ox, oy, oz, 1.));
+  } else {
+    HAMX_TRY(ws_get(ctx, kSlotRndC0, n * sizeof(double2), &w));
+    double2 *c0 = static_cast<double2 *>(w);
+    HAMX_TRY(ws_get(ctx, kSlotRndC1, n * sizeof(double2), &w));
+    double2 *c1 = static_cast<double2 *>(w);
+    const unsigned blocks = ew_blocks(n);
+    hipLaunchKernelGGL(k_mhd_draw, dim3(blocks), dim3(256), 0, ctx->stream, c0, c1, a, seed,
+                       static_cast<const double *>(bobs));
+    HAMX_HIP(ctx, hipGetLastError());
+    HAMX_TRY(fft3d_dev2(ctx, c0, c1, a.b.nx, a.b.ny, a.b.nz, +1));
+    hipLaunchKernelGGL(k_es_final, dim3(blocks), dim3(256), 0, ctx->stream, c0, c1, ox, oy, oz,
+                       a.b, 1.);
+    HAMX_HIP(ctx, hipGetLastError());
+  }
   if (!out_dev) {
     HAMX_HIP(ctx, hipMemcpyAsync(bx, ox, n * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
     HAMX_HIP(ctx, hipMemcpyAsync(by, oy, n * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
@@ -938,14 +1022,23 @@ extern "C" int hamx_ternd_dft(hamx_ctx *ctx, const hamx_dft_desc *d, uint64_t se
     HAMX_TRY(ws_get(ctx, kSlotRndOut0, n * sizeof(double), &w));
     ot = static_cast<double *>(w);
   }
-  const unsigned blocks = ew_blocks(n);
-  hipLaunchKernelGGL(k_dft_draw, dim3(blocks), dim3(256), 0, ctx->stream, tk, a, seed);
-  HAMX_HIP(ctx, hipGetLastError());
-  HAMX_TRY(fft3d_dev(ctx, tk, a.b.nx, a.b.ny, a.b.nz, +1));
-  HAMX_TRY(variance_dev(ctx, reinterpret_cast<const double *>(tk), n, red));
-  hipLaunchKernelGGL(k_dft_rescale, dim3(blocks), dim3(256), 0, ctx->stream, tk, ot, a,
-                     static_cast<const double *>(red + 1));
-  HAMX_HIP(ctx, hipGetLastError());
+  HalfPlan hp;
+  int rc;
+  const bool half = half_plan(ctx, a.b, &hp, &rc);
+  HAMX_TRY(rc);
+  if (half) {
+    HAMX_TRY(half_draw(ctx, hp, DftDraw{a}, seed, tk, static_cast<double2 *>(nullptr), red));
+    HAMX_TRY(half_te_out(ctx, hp, tk, ot, a, red + 1));
+  } else {
+    const unsigned blocks = ew_blocks(n);
+    hipLaunchKernelGGL(k_dft_draw, dim3(blocks), dim3(256), 0, ctx->stream, tk, a, seed);
+    HAMX_HIP(ctx, hipGetLastError());
+    HAMX_TRY(fft3d_dev(ctx, tk, a.b.nx, a.b.ny, a.b.nz, +1));
+    HAMX_TRY(variance_dev(ctx, reinterpret_cast<const double *>(tk), n, red));
+    hipLaunchKernelGGL(k_dft_rescale, dim3(blocks), dim3(256), 0, ctx->stream, tk, ot, a,
+                       static_cast<const double *>(red + 1));
+    HAMX_HIP(ctx, hipGetLastError());
+  }
   if (!out_dev)
     HAMX_HIP(ctx, hipMemcpyAsync(te, ot, n * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
   HAMX_HIP(ctx, hipStreamSynchronize(ctx->stream));

@@ -1,0 +1,75 @@
+"""The generators' half-space passes at the sizes where they can go wrong --
+the smallest box, odd numbers of z lines (the variance ends inside a line),
+axes at and beyond the passes' LDS bounds, mixed-radix and Bluestein lengths
+on each axis -- element-wise against the CPU oracle on the same Philox
+stream.  The bound is the generators' own 1e-11 relative L2: the passes sum
+in another order than the oracle, FP64 throughout (1e-15 to 1e-14 seen)."""
+import numpy as np
+import pytest
+
+from hammurabix_amd import _capi as capi
+from hammurabix_amd.units import CGS
+from oracle_lib import load_oracle, ptr, rel_l2
+import ctypes as C
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(2, 2, 2), (3, 5, 7), (16, 8, 4), (33, 17, 9), (64, 48, 128), (11, 26, 13),
+          (5, 3, 37),
+          (4, 6, 1024), (3, 2, 512),    # z at the passes' bound
+          (4, 3, 1100), (2, 2, 1031),   # ... and beyond it: whole-array steps
+          (2100, 3, 2), (4096, 2, 3),   # x in the largest tile
+          (1031, 3, 2),                 # Bluestein x of 4096 points
+          (4116, 2, 2), (2053, 2, 2)]   # x beyond the bound
+
+
+def box(shape):
+    return capi.HamxBox(*shape, -20 * CGS.kpc, 20 * CGS.kpc, -20 * CGS.kpc, 20 * CGS.kpc,
+                        -4 * CGS.kpc, 4 * CGS.kpc)
+
+
+def fill(d, shape):
+    d.box = box(shape)
+    d.observer[:] = [-8.3 * CGS.kpc, 0.0, 0.006 * CGS.kpc]
+    if hasattr(d, "breg_model"):
+        d.breg_model = capi.HAMX_BREG_LSA
+        d.breg[0:4] = [6e-6, 27 * CGS.rad, 0.9 * CGS.rad, 25 * CGS.rad]
+    return d
+
+
+def compare(gpu, oracle, d, seed, shape, outs):
+    n = int(np.prod(shape))
+    g = [np.full(n, np.nan) for _ in range(outs)]
+    r = [np.zeros(n) for _ in range(outs)]
+    gpu(d, seed, *g)
+    assert oracle(C.byref(d), seed, *[ptr(a) for a in r]) == 0
+    for a, b in zip(g, r):
+        assert np.all(np.isfinite(a))
+        assert rel_l2(a, b) < 1e-11
+
+
+def es(shape, rho):
+    d = fill(capi.HamxEsDesc(), shape)
+    d.rms, d.k0, d.k1, d.a0, d.a1, d.rho = 2e-6, 0.12, 0.06, 1.7, 0.5, rho
+    d.r0, d.z0 = 8 * CGS.kpc, 1 * CGS.kpc
+    return d
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+def test_es(ctx, shape):
+    compare(ctx.brnd_es, load_oracle().orc_brnd_es, es(shape, 0.7), 5, shape, 3)
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+def test_dft(ctx, shape):
+    d = fill(capi.HamxDftDesc(), shape)
+    d.rms, d.k0, d.a0, d.r0, d.z0 = 1e-3, 0.02, -1.7, 8 * CGS.kpc, 1 * CGS.kpc
+    compare(ctx.ternd_dft, load_oracle().orc_ternd_dft, d, 6, shape, 1)
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+def test_mhd(ctx, shape):
+    d = fill(capi.HamxMhdDesc(), shape)
+    d.pa0 = d.pf0 = d.ps0 = 1e-12
+    d.k0, d.k1, d.aa0, d.af0, d.as0, d.a1, d.beta, d.ma = 0.3, 0.1, 1.7, 1.5, 1.7, 0.0, 0.1, 0.5
+    compare(ctx.brnd_mhd, load_oracle().orc_brnd_mhd, d, 7, shape, 3)
