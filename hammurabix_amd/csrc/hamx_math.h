@@ -156,4 +156,29 @@ __device__ inline void sincos_fast(double x, double &s, double &c) {
   }
 }
 
+// sqrt(x) for x >= 0 below 2^1000, within 1 ulp: the v_rsq_f64 estimate and
+// two coupled Newton steps for the root and half its reciprocal, without the
+// library's scaling of tiny arguments (below 2^-1000 the result is 2^-500).
+__device__ inline double sqrt_pos(double x) {
+  x = fmax(x, 0x1p-1000);
+  const double y = __builtin_amdgcn_rsq(x);
+  double g = x * y, h = 0.5 * y;
+  const double e = fma(-h, g, 0.5);
+  g = fma(g, e, g);
+  h = fma(h, e, h);
+  return fma(fma(-g, g, x), h, g);
+}
+
+// sin and cos of 2 pi u for 0 <= u < 1: the quadrant and the angle within it
+// are exact in 4 u, and pi/2 in two parts keeps the product's error below the
+// series'.
+__device__ inline void sincos_turn(double u, double &s, double &c) {
+  const double v = 4.0 * u, k = rint(v), r = v - k;
+  double sr, cr;
+  sincos_series(fma(r, 1.5707963267948966, r * 6.123233995736766e-17), sr, cr);
+  const int q = static_cast<int>(k) & 3;
+  s = (q == 0) ? sr : (q == 1) ? cr : (q == 2) ? -sr : -cr;
+  c = (q == 0) ? cr : (q == 1) ? -sr : (q == 2) ? -cr : sr;
+}
+
 } // namespace hamx

@@ -61,9 +61,9 @@ __device__ inline void gauss_pair(uint64_t seed, uint32_t stream, uint64_t m,
   const uint64_t b = (static_cast<uint64_t>(c[3]) << 32) | c[2];
   const double u1 = (static_cast<double>(a >> 11) + 1.0) * 0x1.0p-53;
   const double u2 = static_cast<double>(b >> 11) * 0x1.0p-53;
-  const double r = sqrt(-2.0 * log_pos(u1));
+  const double r = sqrt_pos(-2.0 * log_pos(u1));
   double s, co;
-  sincos_fast(cgs::twopi * u2, s, co);
+  sincos_turn(u2, s, co);
   g0 = r * co;
   g1 = r * s;
 }
@@ -142,14 +142,45 @@ __device__ inline double wavenum(uint64_t i, uint64_t n, double len) {
   return k;
 }
 
-// |k| of mode (i, j, l).  The bands compare it strictly with their edges,
-// which lattice modes can tie exactly: every path forms it in this order.
-__device__ inline double mode_k(double kx, double ky, double kz) {
-  return sqrt(kx * kx + ky * ky + kz * kz);
+// |k|^2 of a mode.  The bands compare |k| strictly with their edges, which
+// lattice modes can tie exactly: every path forms it in this order.
+__device__ inline double mode_k2(double kx2, double ky, double kz) {
+  return kx2 + ky * ky + kz * kz;
 }
-__device__ inline double mode_k(const BoxArgs &a, uint64_t i, uint64_t j, uint64_t l) {
-  return mode_k(wavenum(i, a.nx, a.lx), wavenum(j, a.ny, a.ly), wavenum(l, a.nz, a.lz));
+__device__ inline double mode_k2(const BoxArgs &a, uint64_t i, uint64_t j, uint64_t l) {
+  const double kx = wavenum(i, a.nx, a.lx);
+  return mode_k2(kx * kx, wavenum(j, a.ny, a.ly), wavenum(l, a.nz, a.lz));
 }
+
+// A band edge k as bounds on x = |k|^2, so that the kernels take no square
+// root to decide: sqrt(x) < k exactly where x <= lt, sqrt(x) > k exactly
+// where x > le (correctly rounded square roots, x >= 0).
+struct KEdge {
+  double lt, le;
+};
+
+static KEdge k_edge(double k) {
+  if (std::isnan(k))
+    return KEdge{-1., INFINITY}; // neither below nor above
+  auto last = [k](bool strict) { // the largest x whose root is below k (or equal)
+    auto in = [&](double x) { return strict ? std::sqrt(x) < k : std::sqrt(x) <= k; };
+    if (!in(0.))
+      return -1.;
+    double x = std::fmin(k * k, 1.7976931348623157e308);
+    while (!in(x))
+      x = std::nextafter(x, 0.);
+    for (double y; x < 1.7976931348623157e308 && in(y = std::nextafter(x, INFINITY));)
+      x = y;
+    return x;
+  };
+  return KEdge{last(true), std::isinf(k) && k > 0 ? INFINITY : last(false)};
+}
+
+// A power of |k| as coef * x^e, x = |k|^2: one logarithm and one exponential.
+struct KPower {
+  double coef, e;
+  __device__ double at(double lnx) const { return coef * exp_fast(e * lnx); }
+};
 
 // Vertex position (brnd_es.cc:165-173: vertex spacing L/(n-1)).
 __device__ inline Vec3 vertex_pos(const BoxArgs &a, uint64_t i, uint64_t j,
@@ -247,8 +278,12 @@ static int variance_dev(hamx_ctx *ctx, const double *x, uint64_t n,
 struct EsArgs {
   BoxArgs b;
   Vec3 obs;
-  double rms, k0, k1, a0, a1, rho, r0, z0;
-  double c01; // (k0 / k1)^a1, the low band's constant factor
+  double rms, rho, r0, z0;
+  // Brnd_es::spectrum (brnd_es.cc:34-49) as amplitudes of a mode's components:
+  // low x below k1, mid between k1 and k0, high above k0
+  KEdge k0, k1;
+  double low;
+  KPower mid, high;
   int breg_model;
   int jf12; // Brnd_jf12: its energy profile and literal constants
   double jp[13];
@@ -258,28 +293,27 @@ struct EsArgs {
   GridGeo g_breg;
 };
 
-// Brnd_es::spectrum (brnd_es.cc:34-49)
-__device__ inline double es_spectrum(const EsArgs &a, double k) {
-  const double p0 = a.rms * a.rms;
-  const double unit = 1. / (4. * cgs::pi * k * k);
-  // the reference's sum of band-masked terms, with each power evaluated only
-  // where its band is on (a masked-off term adds an exact zero)
-  double P = 0.;
-  if (k < a.k1) {
-    const double x = k / a.k1, x3 = x * x * x;
-    P += a.c01 * (x3 * x3); // (k0 / k1)^a1 (k / k1)^6
-  }
-  // 1 / (k / k0)^a as exp(-a ln(k / k0)): within a few ulp of the power
-  if (k > a.k1 && k < a.k0)
-    P += exp_fast(-a.a1 * log_pos(k / a.k0));
-  if (k > a.k0)
-    P += exp_fast(-a.a0 * log_pos(k / a.k0));
-  return P * p0 * unit;
+// The standard deviation of the components of a mode at x = |k|^2
+// (brnd_es.cc:34-49,127-133): the square root of the band's power
+//   third rms^2 dk3 / (4 pi k^2) {(k0/k1)^a1 (k/k1)^6, (k/k0)^-a1, (k/k0)^-a0}
+// with the constants folded on the host (es_bands).  With k1 > k0 the low and
+// the high band overlap and their powers add.
+__device__ inline double es_sigma(const EsArgs &a, double x) {
+  const double lo = x <= a.k1.lt ? a.low * x : 0.;
+  const bool hi = x > a.k0.le, mid = x > a.k1.le && x <= a.k0.lt;
+  double v = 0.;
+  if (hi || mid)
+    v = (hi ? a.high : a.mid).at(log_pos(x));
+  return lo != 0. && v != 0. ? sqrt(lo * lo + v * v) : lo + v;
 }
 
-// The standard deviation of a mode's two components (brnd_es.cc:127-133).
-__device__ inline double es_sigma(const EsArgs &a, double k) {
-  return sqrt(a.third * es_spectrum(a, k) * a.b.dk3);
+static void es_bands(EsArgs &a, const hamx_es_desc *d) {
+  const double p = a.third * d->rms * d->rms * a.b.dk3 / (4. * cgs::pi);
+  a.k0 = k_edge(d->k0);
+  a.k1 = k_edge(d->k1);
+  a.low = std::sqrt(p * std::pow(d->k0 / d->k1, d->a1)) / (d->k1 * d->k1 * d->k1);
+  a.mid = KPower{std::sqrt(p) * std::pow(d->k0, 0.5 * d->a1), -0.25 * (d->a1 + 2.)};
+  a.high = KPower{std::sqrt(p) * std::pow(d->k0, 0.5 * d->a0), -0.25 * (d->a0 + 2.)};
 }
 
 // Brnd_jf12::spatial_profile (brnd_jf12.cc:54-114): the squared disk (JF12
@@ -327,7 +361,7 @@ __global__ __launch_bounds__(256) void k_es_draw(double2 *c0, double2 *c1,
     }
     uint64_t i, j, l;
     box_ijl(a.b, idx, i, j, l);
-    const double sigma = es_sigma(a, mode_k(a.b, i, j, l));
+    const double sigma = es_sigma(a, mode_k2(a.b, i, j, l));
     double g0, g1, g2, g3;
     gauss_pair(seed, 0, 2 * idx, g0, g1);
     gauss_pair(seed, 0, 2 * idx + 1, g2, g3);
@@ -502,18 +536,15 @@ __global__ __launch_bounds__(256) void k_es_final(const double2 *c0, const doubl
 struct DftArgs {
   BoxArgs b;
   Vec3 obs;
-  double rms, k0, a0, r0, z0;
+  double rms, r0, z0;
+  KEdge k0;
+  KPower amp; // above k0
 };
 
-// TErnd_dft::spectrum (ternd_dft.cc:17-24)
-__device__ inline double dft_spectrum(const DftArgs &a, double k) {
-  if (k < a.k0)
-    return 0.;
-  return a.rms * exp(a.a0 * log(k / a.k0)) / (4 * cgs::pi * k * k); // (k / k0)^a0
-}
-
-__device__ inline double dft_sigma(const DftArgs &a, double k) {
-  return sqrt(dft_spectrum(a, k) * a.b.dk3);
+// The standard deviation of the components of a mode at x = |k|^2, the
+// square root of rms (k / k0)^a0 dk3 / (4 pi k^2) (ternd_dft.cc:17-24,71-78).
+__device__ inline double dft_sigma(const DftArgs &a, double x) {
+  return x <= a.k0.lt ? 0. : a.amp.at(log_pos(x));
 }
 
 __global__ __launch_bounds__(256) void k_dft_draw(double2 *tk, DftArgs a,
@@ -527,7 +558,7 @@ __global__ __launch_bounds__(256) void k_dft_draw(double2 *tk, DftArgs a,
     }
     uint64_t i, j, l;
     box_ijl(a.b, idx, i, j, l);
-    const double sigma = dft_sigma(a, mode_k(a.b, i, j, l));
+    const double sigma = dft_sigma(a, mode_k2(a.b, i, j, l));
     double g0, g1;
     gauss_pair(seed, 1, idx, g0, g1);
     tk[idx] = make_double2(sigma * g0, sigma * g1);
@@ -788,11 +819,6 @@ int brnd_generate(hamx_ctx *ctx, const hamx_es_desc *d, uint64_t seed, double *b
   a.b = box_args(d->box);
   a.obs = Vec3{d->observer[0], d->observer[1], d->observer[2]};
   a.rms = d->rms;
-  a.k0 = d->k0;
-  a.k1 = d->k1;
-  a.a0 = d->a0;
-  a.a1 = d->a1;
-  a.c01 = std::pow(d->k0 / d->k1, d->a1);
   a.rho = d->rho;
   a.r0 = d->r0;
   a.z0 = d->z0;
@@ -804,6 +830,7 @@ int brnd_generate(hamx_ctx *ctx, const hamx_es_desc *d, uint64_t seed, double *b
   a.third = jf12 ? 0.33333333 : cgs::onethird;
   a.twothirds = jf12 ? 0.66666667 : cgs::twothirds;
   a.sqrt3 = jf12 ? 1.73205081 : cgs::sqrthree;
+  es_bands(a, d);
   if (d->breg_model == HAMX_BREG_GRID) {
     if (!(d->breg_x && d->breg_y && d->breg_z))
       return set_err(ctx, HAMX_ERR_ARG, "breg grid model without breg grid arrays");
@@ -1007,8 +1034,9 @@ extern "C" int hamx_ternd_dft(hamx_ctx *ctx, const hamx_dft_desc *d, uint64_t se
   a.b = box_args(d->box);
   a.obs = Vec3{d->observer[0], d->observer[1], d->observer[2]};
   a.rms = d->rms;
-  a.k0 = d->k0;
-  a.a0 = d->a0;
+  a.k0 = k_edge(d->k0);
+  a.amp = KPower{std::sqrt(d->rms * a.b.dk3 / (4. * cgs::pi)) * std::pow(d->k0, -0.5 * d->a0),
+                 0.25 * (d->a0 - 2.)};
   a.r0 = d->r0;
   a.z0 = d->z0;
   const uint64_t n = a.b.n;
