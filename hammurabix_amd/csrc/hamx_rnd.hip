@@ -432,6 +432,87 @@ __device__ inline bool es_rescale_at(const EsArgs &a, const EsScale &sc, uint64_
   return true;
 }
 
+// The same step split for the light models: the energy profile's square root
+// is a product of a factor of (x, y) and one of z, and the regular field's
+// versor is (cz ux, cz uy, sz uz) with (ux, uy, uz) a function of (x, y) and
+// (cz, sz) of z (LSA: cos chi and sin chi; the others: 1), so a tile of z
+// lines evaluates models and profile once per line and once per z.
+struct EsLine {
+  double ux, uy, uz; // 0, 0, 0: the regular field is zero on the line
+  double ratio;
+};
+struct EsZ {
+  double cz, sz, ratio;
+};
+
+__device__ inline double axis_pos(uint64_t i, uint64_t n, double len, double lo) {
+  return static_cast<double>(i) * len / static_cast<double>(n - 1) + lo; // as vertex_pos
+}
+
+__device__ inline EsLine es_line(const EsArgs &a, const EsScale &sc, uint32_t i, uint32_t j) {
+  const Vec3 pos{axis_pos(i, a.b.nx, a.b.lx, a.b.x_min), axis_pos(j, a.b.ny, a.b.ly, a.b.y_min),
+                 0.};
+  const double r = sqrt(pos.x * pos.x + pos.y * pos.y);
+  EsLine o{0., 0., 0.,
+           exp_fast(-0.5 * ((r - fabs(a.obs.x)) / a.r0)) * a.rms * sc.b_var_invsq};
+  if (a.breg_model == HAMX_BREG_LSA) {
+    // breg_eval's LSA (breg_lsa.cc:9-26) without chi and the strength
+    if (a.breg[0] == 0. || r > (20. * cgs::kpc) || r < (3. * cgs::kpc))
+      return o;
+    double s, c;
+    sincos_fast(a.breg[1] + a.breg[2] * log_pos(r / (8. * cgs::kpc)), s, c);
+    const double cos_p = pos.x / r, sin_p = pos.y / r;
+    o.ux = s * cos_p - c * sin_p;
+    o.uy = s * sin_p + c * cos_p;
+    o.uz = 1.;
+    return o;
+  }
+  const Vec3 b = breg_eval<false>(a.breg_model, a.breg, pos);
+  const double l2 = b.x * b.x + b.y * b.y + b.z * b.z;
+  if (l2 != 0.) {
+    const double den = 1. / sqrt(l2);
+    o.ux = b.x * den;
+    o.uy = b.y * den;
+    o.uz = b.z * den;
+  }
+  return o;
+}
+
+__device__ inline EsZ es_z(const EsArgs &a, uint32_t l) {
+  const double z = axis_pos(l, a.b.nz, a.b.lz, a.b.z_min);
+  EsZ o{1., 1., exp_fast(-0.5 * ((fabs(z) - fabs(a.obs.z)) / a.z0))};
+  if (a.breg_model == HAMX_BREG_LSA) {
+    const double u = z / (1. * cgs::kpc), e = exp_fast(-2. * fabs(u));
+    sincos_fast(a.breg[3] * copysign((1. - e) * rcp_f64(1. + e), u), o.sz, o.cz);
+  }
+  return o;
+}
+
+__device__ inline Vec3 es_rescale_split(const EsLine &ln, const EsZ &zt, const EsScale &sc,
+                                        const double2 &v0, const double2 &v1) {
+  if (ln.ux == 0. && ln.uy == 0. && ln.uz == 0.)
+    return Vec3{v0.x, v1.x, v1.y}; // zero regular field: the raw FFT values stay
+  const double ratio = ln.ratio * zt.ratio;
+  const Vec3 b{v0.x * ratio, v0.y * ratio, v1.y * ratio};
+  const Vec3 H{zt.cz * ln.ux, zt.cz * ln.uy, zt.sz * ln.uz};
+  const double hb = dot0(H, b);
+  const Vec3 par{H.x * hb, H.y * hb, H.z * hb};
+  const Vec3 perp{b.x - par.x, b.y - par.y, b.z - par.z};
+  return Vec3{(par.x * sc.rho + perp.x * sc.inv_rho) * sc.rhonorm,
+              (par.y * sc.rho + perp.y * sc.inv_rho) * sc.rhonorm,
+              (par.z * sc.rho + perp.z * sc.inv_rho) * sc.rhonorm};
+}
+
+// The profile's two factors stay far from overflow and underflow over the
+// whole box (a scale height of a few parsec would not).
+static bool profile_splits(const hamx_box &b, const double *obs, double r0, double z0) {
+  const double r = std::hypot(std::fmax(std::fabs(b.x_min), std::fabs(b.x_max)),
+                              std::fmax(std::fabs(b.y_min), std::fabs(b.y_max)));
+  const double z = std::fmax(std::fabs(b.z_min), std::fabs(b.z_max));
+  return (r + std::fabs(obs[0])) / std::fabs(r0) < 400. &&
+         (z + std::fabs(obs[2])) / std::fabs(z0) < 400.;
+}
+
 template <bool HEAVY>
 __global__ __launch_bounds__(256) void k_es_rescale(double2 *c0, double2 *c1,
                                                     EsArgs a, const double *var) {
@@ -570,6 +651,17 @@ __device__ inline double dft_ratio(const DftArgs &a, uint64_t i, uint64_t j, uin
                                    double te_var_invsq) {
   const Vec3 pos = vertex_pos(a.b, i, j, l);
   return sqrt(profile(a.obs, a.r0, a.z0, pos)) * a.rms * te_var_invsq;
+}
+
+// ... as a factor of (x, y) and one of z.
+__device__ inline double dft_line(const DftArgs &a, uint32_t i, uint32_t j, double te_var_invsq) {
+  const double x = axis_pos(i, a.b.nx, a.b.lx, a.b.x_min);
+  const double y = axis_pos(j, a.b.ny, a.b.ly, a.b.y_min);
+  return exp_fast(-0.5 * ((sqrt(x * x + y * y) - fabs(a.obs.x)) / a.r0)) * a.rms * te_var_invsq;
+}
+__device__ inline double dft_z(const DftArgs &a, uint32_t l) {
+  const double z = axis_pos(l, a.b.nz, a.b.lz, a.b.z_min);
+  return exp_fast(-0.5 * ((fabs(z) - fabs(a.obs.z)) / a.z0));
 }
 
 __global__ __launch_bounds__(256) void k_dft_rescale(const double2 *tk, double *te,
@@ -879,7 +971,8 @@ int brnd_generate(hamx_ctx *ctx, const hamx_es_desc *d, uint64_t seed, double *b
   if (half) {
     const HalfArrays H = half_arrays(hp, hw);
     HAMX_TRY(half_draw(ctx, hp, EsDraw{a}, seed, c0, c1, red));
-    HAMX_TRY(heavy ? half_mid<true>(ctx, hp, c0, c1, H, a, red + 1)
+    const bool split = !heavy && profile_splits(d->box, d->observer, d->r0, d->z0);
+    HAMX_TRY(split ? half_mid<true>(ctx, hp, c0, c1, H, a, red + 1)
                    : half_mid<false>(ctx, hp, c0, c1, H, a, red + 1));
     HAMX_TRY(half_y(ctx, hp, H, -1));
     HAMX_TRY(half_gs_x(ctx, hp, H, a));
@@ -1056,7 +1149,8 @@ extern "C" int hamx_ternd_dft(hamx_ctx *ctx, const hamx_dft_desc *d, uint64_t se
   HAMX_TRY(rc);
   if (half) {
     HAMX_TRY(half_draw(ctx, hp, DftDraw{a}, seed, tk, static_cast<double2 *>(nullptr), red));
-    HAMX_TRY(half_te_out(ctx, hp, tk, ot, a, red + 1));
+    HAMX_TRY(half_te_out(ctx, hp, tk, ot, a, profile_splits(d->box, d->observer, d->r0, d->z0),
+                         red + 1));
   } else {
     const unsigned blocks = ew_blocks(n);
     hipLaunchKernelGGL(k_dft_draw, dim3(blocks), dim3(256), 0, ctx->stream, tk, a, seed);

@@ -207,8 +207,10 @@ __global__ __launch_bounds__(1024) void k_var_half(const double *part, uint32_t 
 // CL stored z lines (i, j) and their mirrors (-i, -j): lines c0 and c1 of
 // the former in LDS, then those of the latter.  A thread's vertex l of a
 // line and vertex -l of its mirror are read by no other thread, so the even
-// parts go straight back into the two lines' places.
-template <bool HEAVY, uint32_t TILE, uint32_t NT, int MODE>
+// parts go straight back into the two lines' places.  SPLIT takes the
+// rescale's factors from tables of the tile's 2 CL lines and of z in LDS: the
+// kernel was bound by the per-vertex models (es 256x256x64 106 -> 62 us).
+template <bool SPLIT, uint32_t TILE, uint32_t NT, int MODE>
 __global__ __launch_bounds__(NT) void k_es_mid(const double2 *__restrict__ c0,
                                                const double2 *__restrict__ c1, HalfArrays H,
                                                EsArgs a, const double *__restrict__ var,
@@ -246,25 +248,47 @@ __global__ __launch_bounds__(NT) void k_es_mid(const double2 *__restrict__ c0,
         lds[(e - q * n) * P + m * CL + q] = r[k][m];
     }
   }
+  const EsScale sc = es_scale(a, var);
+  EsZ *zt = reinterpret_cast<EsZ *>(lds + L.len * P + (fft_lds_tw<TILE, MODE>() ? L.len : 0));
+  EsLine *lt = reinterpret_cast<EsLine *>(zt + n);
+  if constexpr (SPLIT) {
+    for (uint32_t e = threadIdx.x; e < n + 2 * nl; e += NT) {
+      if (e < n) {
+        zt[e] = es_z(a, e);
+      } else {
+        const bool mir = e - n >= nl;
+        const uint32_t q = e - n - (mir ? nl : 0), line = L0 + q;
+        const uint32_t i = line / h.ny, j = line - i * h.ny;
+        lt[mir ? CL + q : q] = mir ? es_line(a, sc, mirror_of(i, h.nx), mirror_of(j, h.ny))
+                                   : es_line(a, sc, i, j);
+      }
+    }
+  }
   __syncthreads();
   fft_lines<1, TILE, NT, MODE>(lds, twl, L, cl + 2, P);
-  const EsScale sc = es_scale(a, var);
 #pragma unroll 1
   for (uint32_t e = threadIdx.x; e < nl * n; e += NT) {
     const uint32_t q = fast_quot(h.dz, e), l = e - q * n, lm = mirror_of(l, n);
-    const uint32_t line = L0 + q, i = line / h.ny, j = line - i * h.ny;
     Vec3 f{0., 0., 0.};
+    if constexpr (SPLIT) {
+      const Vec3 b = es_rescale_split(lt[q], zt[l], sc, lds[l * P + q], lds[l * P + CL + q]);
+      const Vec3 m = es_rescale_split(lt[CL + q], zt[lm], sc, lds[lm * P + 2 * CL + q],
+                                      lds[lm * P + 3 * CL + q]);
+      f = Vec3{b.x + m.x, b.y + m.y, b.z + m.z};
+    } else {
+      const uint32_t line = L0 + q, i = line / h.ny, j = line - i * h.ny;
 #pragma unroll 1
-    for (int m = 0; m < 2; ++m) {
-      const uint32_t vi = m ? mirror_of(i, h.nx) : i, vj = m ? mirror_of(j, h.ny) : j;
-      const uint32_t vl = m ? lm : l;
-      const double2 v0 = lds[vl * P + 2 * m * CL + q], v1 = lds[vl * P + (2 * m + 1) * CL + q];
-      Vec3 b;
-      if (!es_rescale_at<HEAVY>(a, sc, vi, vj, vl, v0, v1, b))
-        b = Vec3{v0.x, v1.x, v1.y};
-      f.x += b.x;
-      f.y += b.y;
-      f.z += b.z;
+      for (int m = 0; m < 2; ++m) {
+        const uint32_t vi = m ? mirror_of(i, h.nx) : i, vj = m ? mirror_of(j, h.ny) : j;
+        const uint32_t vl = m ? lm : l;
+        const double2 v0 = lds[vl * P + 2 * m * CL + q], v1 = lds[vl * P + (2 * m + 1) * CL + q];
+        Vec3 b;
+        if (!es_rescale_at<true>(a, sc, vi, vj, vl, v0, v1, b))
+          b = Vec3{v0.x, v1.x, v1.y};
+        f.x += b.x;
+        f.y += b.y;
+        f.z += b.z;
+      }
     }
     lds[l * P + q] = make_double2(0.5 * f.x, 0.5 * f.y);
     lds[l * P + CL + q] = make_double2(0.5 * f.z, 0.);
@@ -457,8 +481,9 @@ __global__ __launch_bounds__(NT) void k_half_out(HalfArrays H, double *__restric
 }
 
 // z(+) and the energy profile of TErnd_dft (ternd_dft.cc:109-128): CL z lines
-// of the whole box.
-template <uint32_t TILE, uint32_t NT, int MODE>
+// of the whole box.  SPLIT takes the profile's factors from tables in LDS (te
+// 800x800x160 1072 -> 727 us).
+template <bool SPLIT, uint32_t TILE, uint32_t NT, int MODE>
 __global__ __launch_bounds__(NT) void k_te_out(const double2 *__restrict__ tk,
                                                double *__restrict__ te, DftArgs a,
                                                const double *__restrict__ var, HalfArgs h,
@@ -482,14 +507,26 @@ __global__ __launch_bounds__(NT) void k_te_out(const double2 *__restrict__ tk,
     if (q < CL)
       lds[(e - q * n) * P + q] = r[k];
   }
+  const double te_var_invsq = 1. / sqrt(var[0]);
+  double *zt = reinterpret_cast<double *>(lds + L.len * P +
+                                          (fft_lds_tw<TILE, MODE>() ? L.len : 0));
+  if constexpr (SPLIT) {
+    for (uint32_t e = threadIdx.x; e < n + nl; e += NT) {
+      const uint32_t line = L0 + e - n, i = line / h.ny;
+      zt[e] = e < n ? dft_z(a, e) : dft_line(a, i, line - i * h.ny, te_var_invsq);
+    }
+  }
   __syncthreads();
   fft_lines<1, TILE, NT, MODE>(lds, twl, L, cl, P);
-  const double te_var_invsq = 1. / sqrt(var[0]);
 #pragma unroll 1
   for (uint32_t e = threadIdx.x; e < nl * n; e += NT) {
     const uint32_t q = fast_quot(h.dz, e), l = e - q * n;
-    const uint32_t line = L0 + q, i = line / h.ny, j = line - i * h.ny;
-    te[at0 + e] = lds[l * P + q].x * dft_ratio(a, i, j, l, te_var_invsq);
+    if constexpr (SPLIT) {
+      te[at0 + e] = lds[l * P + q].x * (zt[n + q] * zt[l]);
+    } else {
+      const uint32_t line = L0 + q, i = line / h.ny, j = line - i * h.ny;
+      te[at0 + e] = lds[l * P + q].x * dft_ratio(a, i, j, l, te_var_invsq);
+    }
   }
 }
 
@@ -632,16 +669,18 @@ int half_draw(hamx_ctx *ctx, const HalfPlan &p, const Draw &dr, uint64_t seed, d
 }
 
 // z(+), rescale, even part, z(-) of Brnd_es.
-template <bool HEAVY>
+template <bool SPLIT>
 int half_mid(hamx_ctx *ctx, const HalfPlan &p, const double2 *c0, const double2 *c1,
              const HalfArrays &H, const EsArgs &a, const double *var) {
   uint32_t cl;
   const uint32_t tile = p.z_tile(4, p.h.lines, &cl);
+  const uint32_t tables = SPLIT ? p.lz.n * sizeof(EsZ) + (2u << cl) * sizeof(EsLine) : 0;
   with_tile(tile, p.lz.mode, [&](auto T, auto NT, auto M) {
-    hipLaunchKernelGGL((k_es_mid<HEAVY, decltype(T)::value, decltype(NT)::value,
+    hipLaunchKernelGGL((k_es_mid<SPLIT, decltype(T)::value, decltype(NT)::value,
                                  decltype(M)::value>),
                        dim3((p.h.lines + (1u << cl) - 1) >> cl), dim3(decltype(NT)::value),
-                       fft_lds_bytes(p.lz, (4u << cl) + 1, tile), ctx->stream, c0, c1, H, a, var,
+                       fft_lds_bytes(p.lz, (4u << cl) + 1, tile) + tables, ctx->stream, c0, c1,
+                       H, a, var,
                        p.h, p.lz, cl);
   });
   HAMX_HIP(ctx, hipGetLastError());
@@ -681,15 +720,23 @@ inline int half_mhd_x(hamx_ctx *ctx, const HalfPlan &p, const HalfArrays &H, con
 
 // z(+) and rescale of TErnd_dft.
 inline int half_te_out(hamx_ctx *ctx, const HalfPlan &p, const double2 *tk, double *te,
-                       const DftArgs &a, const double *var) {
+                       const DftArgs &a, bool split, const double *var) {
   const uint32_t lines = p.h.nx * p.h.ny;
   uint32_t cl;
   const uint32_t tile = p.z_tile(1, lines, &cl);
+  const uint32_t tables = split ? (p.lz.n + (1u << cl)) * sizeof(double) : 0;
   with_tile(tile, p.lz.mode, [&](auto T, auto NT, auto M) {
-    hipLaunchKernelGGL((k_te_out<decltype(T)::value, decltype(NT)::value, decltype(M)::value>),
-                       dim3((lines + (1u << cl) - 1) >> cl), dim3(decltype(NT)::value),
-                       fft_lds_bytes(p.lz, (1u << cl) + 1, tile), ctx->stream, tk, te, a, var,
-                       p.h, lines, p.lz, cl);
+    auto launch = [&](auto S) {
+      hipLaunchKernelGGL((k_te_out<decltype(S)::value, decltype(T)::value, decltype(NT)::value,
+                                   decltype(M)::value>),
+                         dim3((lines + (1u << cl) - 1) >> cl), dim3(decltype(NT)::value),
+                         fft_lds_bytes(p.lz, (1u << cl) + 1, tile) + tables, ctx->stream, tk, te,
+                         a, var, p.h, lines, p.lz, cl);
+    };
+    if (split)
+      launch(std::true_type{});
+    else
+      launch(std::false_type{});
   });
   HAMX_HIP(ctx, hipGetLastError());
   return HAMX_OK;

@@ -67,6 +67,38 @@ def test_dft(ctx, shape):
     compare(ctx.ternd_dft, load_oracle().orc_ternd_dft, d, 6, shape, 1)
 
 
+@pytest.mark.parametrize("z0", [1.0, 0.009])  # 0.009 kpc: the profile is not split
+@pytest.mark.parametrize("model", ["helix", "none", "lsa_off", "jf12_profile"])
+def test_rescale_routes(ctx, model, z0):
+    shape = (20, 18, 12)
+    d = es(shape, 1.6)
+    d.z0 = z0 * CGS.kpc
+    orc = load_oracle()
+    if model == "helix":  # zero field outside 5-15 kpc: raw values there
+        d.breg_model = capi.HAMX_BREG_HELIX
+        d.breg[0:5] = [1e-6, 2e-6, 0.5e-6, 5 * CGS.kpc, 15 * CGS.kpc]
+    elif model == "none":
+        d.breg_model = capi.HAMX_BREG_NONE
+    elif model == "lsa_off":
+        d.breg[0] = 0.0
+    if model == "jf12_profile":
+        mu, kpc = 1e-6, CGS.kpc
+        d.jf12[:] = [10.81 * mu, 6.96 * mu, 9.59 * mu, 6.96 * mu, 1.96 * mu, 16.34 * mu,
+                     37.29 * mu, 10.35 * mu, 7.63 * mu, 0.61 * kpc, 4.68 * mu, 10.97 * kpc,
+                     2.84 * kpc]
+        compare(ctx.brnd_jf12, orc.orc_brnd_jf12, d, 5, shape, 3)
+    else:
+        compare(ctx.brnd_es, orc.orc_brnd_es, d, 5, shape, 3)
+
+
+@pytest.mark.parametrize("z0", [1.0, 0.009])
+def test_dft_profile_routes(ctx, z0):
+    shape = (20, 18, 12)
+    d = fill(capi.HamxDftDesc(), shape)
+    d.rms, d.k0, d.a0, d.r0, d.z0 = 1e-3, 0.02, -1.7, 8 * CGS.kpc, z0 * CGS.kpc
+    compare(ctx.ternd_dft, load_oracle().orc_ternd_dft, d, 6, shape, 1)
+
+
 @pytest.mark.parametrize("shape", SHAPES)
 def test_mhd(ctx, shape):
     d = fill(capi.HamxMhdDesc(), shape)
