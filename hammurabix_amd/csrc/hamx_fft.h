@@ -4,8 +4,8 @@
 // random-field kernels that fuse their elementwise steps into an axis pass
 // (hamx_rnd.hip).
 //
-// * n = 2^a 3^b 5^c 7^d <= 8192: mixed-radix Stockham autosort passes (radix
-//   4 while 4 divides what is left, then 2, 3, 5, 7).  A pass of radix R
+// * n = 2^a 3^b 5^c 7^d <= 8192: mixed-radix Stockham autosort passes (the
+//   power of two in radix 8 and 4, then 3, 5, 7).  A pass of radix R
 //   stages its inputs in registers, synchronises, then writes its outputs, so
 //   one LDS buffer suffices.
 // * any other n <= 4096: Bluestein's algorithm.  With c_j = exp(sign i pi j^2 / n),
@@ -14,6 +14,12 @@
 //   M-point forward transform, a product with the transform of conj(c), and
 //   an M-point inverse transform; the outputs are multiplied by the chirp
 //   and 1/M.
+//
+// A pass over memory is bound by HBM only while the LDS passes hide behind
+// it, so there are few of them: with radix 8 (and the odd radices in their
+// real-factor form, fused multiply-adds throughout) the axis passes of es
+// 256x256x64 took 5 to 12% less time than with radix 4 and 2, te 800x800x160's
+// 12 to 20% less.
 //
 // Layout: point t of line c at lds[t P + c].  C is a power of two and
 // consecutive threads take consecutive lines, so a pass's reads are
@@ -70,7 +76,7 @@ inline FastDiv fast_div(uint32_t d) {
 __device__ inline uint32_t fast_quot(const FastDiv &f, uint32_t e) { return __umulhi(e, f.m); }
 
 __device__ inline double2 cmul(double2 a, double2 b) {
-  return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
+  return make_double2(fma(a.x, b.x, -(a.y * b.y)), fma(a.x, b.y, a.y * b.x));
 }
 __device__ inline double2 cadd(double2 a, double2 b) { return make_double2(a.x + b.x, a.y + b.y); }
 __device__ inline double2 csub(double2 a, double2 b) { return make_double2(a.x - b.x, a.y - b.y); }
@@ -82,30 +88,90 @@ __device__ inline double2 with_sign(double2 w) {
     w.y = -w.y;
   return w;
 }
+// SIGN * i * v
+template <int SIGN>
+__device__ inline double2 times_i(double2 v) {
+  return SIGN > 0 ? make_double2(-v.y, v.x) : make_double2(v.y, -v.x);
+}
 
-// y_t = sum_m x_m W^(t m), W = exp(SIGN 2 pi i / R); w[t] = W^t.
+// cos and sin of 2 pi t m / R for the odd radices
+template <int R>
+__device__ constexpr double odd_cos(int j) {
+  constexpr double c3[2] = {1., -0.5};
+  constexpr double c5[3] = {1., 0.30901699437494742410, -0.80901699437494742410};
+  constexpr double c7[4] = {1., 0.62348980185873353053, -0.22252093395631440429,
+                            -0.90096886790241912624};
+  const int k = j % R, h = 2 * k > R ? R - k : k;
+  return R == 3 ? c3[h] : R == 5 ? c5[h] : c7[h];
+}
+template <int R>
+__device__ constexpr double odd_sin(int j) {
+  constexpr double s3[2] = {0., 0.86602540378443864676};
+  constexpr double s5[3] = {0., 0.95105651629515357212, 0.58778525229247312917};
+  constexpr double s7[4] = {0., 0.78183148246802980871, 0.97492791218182360702,
+                            0.43388373911755812048};
+  const int k = j % R, h = 2 * k > R ? R - k : k;
+  const double s = R == 3 ? s3[h] : R == 5 ? s5[h] : s7[h];
+  return 2 * k > R ? -s : s;
+}
+
+template <int SIGN>
+__device__ inline void dft4(double2 x0, double2 x1, double2 x2, double2 x3, double2 &y0,
+                            double2 &y1, double2 &y2, double2 &y3) {
+  const double2 a0 = cadd(x0, x2), a1 = csub(x0, x2), a2 = cadd(x1, x3);
+  const double2 a3 = times_i<SIGN>(csub(x1, x3));
+  y0 = cadd(a0, a2);
+  y1 = cadd(a1, a3);
+  y2 = csub(a0, a2);
+  y3 = csub(a1, a3);
+}
+
+// y_t = sum_m x_m W^(t m), W = exp(SIGN 2 pi i / R).  Odd R by the pairs
+// x_m + x_{R-m}, x_m - x_{R-m}: real factors only.
 template <int R, int SIGN>
-__device__ inline void small_dft(const double2 (&x)[R], const double2 (&w)[R], double2 (&y)[R]) {
+__device__ inline void small_dft(const double2 (&x)[R], double2 (&y)[R]) {
   if constexpr (R == 2) {
     y[0] = cadd(x[0], x[1]);
     y[1] = csub(x[0], x[1]);
   } else if constexpr (R == 4) {
-    const double2 a0 = cadd(x[0], x[2]), a1 = csub(x[0], x[2]), a2 = cadd(x[1], x[3]);
-    const double2 d13 = csub(x[1], x[3]);
-    // (x1 - x3) * SIGN * i
-    const double2 a3 = SIGN > 0 ? make_double2(-d13.y, d13.x) : make_double2(d13.y, -d13.x);
-    y[0] = cadd(a0, a2);
-    y[1] = cadd(a1, a3);
-    y[2] = csub(a0, a2);
-    y[3] = csub(a1, a3);
+    dft4<SIGN>(x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]);
+  } else if constexpr (R == 8) {
+    // even and odd points by dft4, the odd ones times W^t
+    constexpr double h = 0.70710678118654752440;
+    double2 e[4], o[4];
+    dft4<SIGN>(x[0], x[2], x[4], x[6], e[0], e[1], e[2], e[3]);
+    dft4<SIGN>(x[1], x[3], x[5], x[7], o[0], o[1], o[2], o[3]);
+    const double2 i1 = times_i<SIGN>(o[1]), i3 = times_i<SIGN>(o[3]);
+    o[1] = make_double2(h * (o[1].x + i1.x), h * (o[1].y + i1.y));
+    o[2] = times_i<SIGN>(o[2]);
+    o[3] = make_double2(h * (i3.x - o[3].x), h * (i3.y - o[3].y));
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      y[t] = cadd(e[t], o[t]);
+      y[t + 4] = csub(e[t], o[t]);
+    }
   } else {
+    constexpr int H = R / 2;
+    double2 s[H], d[H];
+    y[0] = x[0];
 #pragma unroll
-    for (int t = 0; t < R; ++t) {
-      double2 acc = x[0];
+    for (int m = 0; m < H; ++m) {
+      s[m] = cadd(x[m + 1], x[R - 1 - m]);
+      d[m] = csub(x[m + 1], x[R - 1 - m]);
+      y[0] = cadd(y[0], s[m]);
+    }
 #pragma unroll
-      for (int m = 1; m < R; ++m)
-        acc = cadd(acc, cmul(x[m], w[(t * m) % R]));
-      y[t] = acc;
+    for (int t = 1; t <= H; ++t) {
+      double2 a = x[0], b = make_double2(0., 0.);
+#pragma unroll
+      for (int m = 0; m < H; ++m) {
+        const double c = odd_cos<R>(t * (m + 1)), q = odd_sin<R>(t * (m + 1));
+        a = make_double2(fma(c, s[m].x, a.x), fma(c, s[m].y, a.y));
+        b = make_double2(fma(q, d[m].x, b.x), fma(q, d[m].y, b.y));
+      }
+      b = times_i<SIGN>(b);
+      y[t] = cadd(a, b);
+      y[R - t] = csub(a, b);
     }
   }
 }
@@ -128,12 +194,6 @@ __device__ inline void stockham_pass(double2 *lds, uint32_t n, uint32_t cshift, 
     }
   }
   __syncthreads();
-  double2 w[R];
-  if constexpr (R != 2 && R != 4) {
-#pragma unroll
-    for (int t = 0; t < R; ++t)
-      w[t] = with_sign<SIGN>(tw[t * q]); // exp(SIGN 2 pi i t / R)
-  }
   const uint32_t p = ps.p;
 #pragma unroll
   for (uint32_t u = 0; u < NB; ++u) {
@@ -150,7 +210,7 @@ __device__ inline void stockham_pass(double2 *lds, uint32_t n, uint32_t cshift, 
         for (int m = 1; m < R; ++m)
           x[u][m] = cmul(x[u][m], with_sign<SIGN>(tw[m * k * ps.tstep]));
       }
-      small_dft<R, SIGN>(x[u], w, y);
+      small_dft<R, SIGN>(x[u], y);
       double2 *at = lds + ((i - k) * R + k) * P + (b & cmask);
 #pragma unroll
       for (int m = 0; m < R; ++m)
@@ -161,14 +221,16 @@ __device__ inline void stockham_pass(double2 *lds, uint32_t n, uint32_t cshift, 
 }
 
 // Every pass of a plan, in order.  Entered and left with LDS synchronised.
-// POW2 instances (plans of radix 4 and 2 only) leave the odd radices out, so
-// their register staging stays at the radix-4 / radix-2 size.
+// POW2 instances (plans of radix 8, 4 and 2) leave the odd radices out, whose
+// register staging is larger.
 template <int SIGN, uint32_t TILE, uint32_t NT, bool POW2>
 __device__ inline void run_plan(double2 *lds, const FftPlan &pl, uint32_t cshift, uint32_t P,
                                 const double2 *tw) {
   for (uint32_t s = 0; s < pl.npass; ++s) {
     const FftPass ps = pl.pass[s];
-    if (ps.radix == 4) {
+    if (ps.radix == 8) {
+      stockham_pass<8, SIGN, TILE, NT, POW2>(lds, pl.n, cshift, P, ps, tw);
+    } else if (ps.radix == 4) {
       stockham_pass<4, SIGN, TILE, NT, POW2>(lds, pl.n, cshift, P, ps, tw);
     } else if (ps.radix == 2) {
       stockham_pass<2, SIGN, TILE, NT, POW2>(lds, pl.n, cshift, P, ps, tw);
@@ -251,6 +313,15 @@ struct FftAxis {
   uint64_t s, inner, outer, lines;
   uint32_t cshift, P;
 };
+
+// The tile of workgroup b of g (g a multiple of 8): the eight XCDs take
+// workgroups in turn, and this gives each of them a contiguous run of tiles,
+// so that neighbouring columns meet in one L2.  Columns rarely start on a
+// cache line (H's rows are nz/2 + 1 long), and a tile's rows are a line or
+// less: both tiles that touch a line then read it from memory once (y passes
+// of es 512x512x128: 280 -> 204 us; with eight columns a tile, 172 us).
+__device__ inline uint32_t xcd_tile(uint32_t b, uint32_t g) { return (b & 7) * (g >> 3) + (b >> 3); }
+inline unsigned xcd_grid(uint64_t tiles) { return static_cast<unsigned>((tiles + 7) / 8 * 8); }
 
 __device__ inline uint64_t line_base(const FftAxis &ax, uint64_t L) {
   if (ax.lines <= 0xffffffffull) { // uniform: 32-bit software division

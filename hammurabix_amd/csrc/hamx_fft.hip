@@ -74,7 +74,10 @@ __global__ __launch_bounds__(NT) void k_fft_axis(FftArrays arr, FftAxis ax, FftL
   constexpr uint32_t K = TILE / NT;
   double2 *__restrict__ data = arr.p[blockIdx.y];
   const uint32_t n = L.n, cs = ax.cshift, C = 1u << cs, P = ax.P;
-  const uint64_t L0 = static_cast<uint64_t>(blockIdx.x) << cs;
+  const uint32_t tile = CONTIG ? blockIdx.x : xcd_tile(blockIdx.x, gridDim.x);
+  const uint64_t L0 = static_cast<uint64_t>(tile) << cs;
+  if (L0 >= ax.lines)
+    return; // uniform: the grid's last few workgroups
   const double2 *twl = fft_tables<TILE, NT, MODE>(lds, L, P);
   const uint64_t left = ax.lines - L0; // lines of this tile that exist (>= 1)
   const uint32_t total = C * n;
@@ -160,7 +163,7 @@ __global__ __launch_bounds__(NT) void k_fft_axis(FftArrays arr, FftAxis ax, FftL
         block_sums<NT>(m2, z0, z1);
       }
       if (threadIdx.x == 0) {
-        double *p = var.part + 4 * static_cast<uint64_t>(blockIdx.x);
+        double *p = var.part + 4 * static_cast<uint64_t>(tile);
         p[0] = mean;
         p[1] = cnt;
         p[2] = m2;
@@ -176,7 +179,7 @@ namespace {
 using cld = std::complex<long double>;
 const long double kTwoPiL = 6.283185307179586476925286766559005768394L;
 
-// Stockham plan of n: radix 4 while 4 divides, then 2, 3, 5, 7.
+// Stockham plan of n: radix 4 and 8, then 3, 5, 7.
 bool make_plan(uint32_t n, FftPlan &pl) {
   std::memset(&pl, 0, sizeof(pl));
   pl.n = n;
@@ -194,11 +197,18 @@ bool make_plan(uint32_t n, FftPlan &pl) {
     p *= r;
     return true;
   };
-  while (m % 4 == 0)
-    if (!push(4))
-      return false;
-  if (m % 2 == 0 && !push(2))
+  // the power of two in the fewest passes of radix 8 and 4 (2 alone as 2)
+  int e = 0;
+  while (m % (2u << e) == 0)
+    ++e;
+  if (e == 1 && !push(2))
     return false;
+  for (int fours = (3 - e % 3) % 3; e > 1; --fours) {
+    const bool four = fours > 0;
+    if (!push(four ? 4u : 8u))
+      return false;
+    e -= four ? 2 : 3;
+  }
   for (uint32_t r : {3u, 5u, 7u})
     while (m % r == 0)
       if (!push(r))
@@ -345,9 +355,9 @@ namespace {
 template <int SIGN, uint32_t TILE, uint32_t NT, int MODE, bool CONTIG, bool VAR>
 int launch_axis(hamx_ctx *ctx, const FftArrays &arr, unsigned arrays, const FftLine &L,
                 const FftAxis &ax, const FftVar &var) {
-  const uint64_t C = 1ull << ax.cshift;
+  const uint64_t tiles = (ax.lines + (1ull << ax.cshift) - 1) >> ax.cshift;
   hipLaunchKernelGGL((k_fft_axis<SIGN, TILE, NT, MODE, CONTIG, VAR>),
-                     dim3(static_cast<unsigned>((ax.lines + C - 1) / C), arrays), dim3(NT),
+                     dim3(CONTIG ? static_cast<unsigned>(tiles) : xcd_grid(tiles), arrays), dim3(NT),
                      fft_lds_bytes(L, ax.P, TILE), ctx->stream, arr, ax, L, fast_div(L.n), var);
   HAMX_HIP(ctx, hipGetLastError());
   return HAMX_OK;
@@ -367,10 +377,10 @@ int launch_mode(hamx_ctx *ctx, const FftArrays &arr, unsigned arrays, const FftL
 }
 
 // The tile: 2048 values (32 KB of LDS) for lines of up to 2048 points along
-// the contiguous axis; along the strided axes the smallest one that holds
-// four columns (64-byte rows), where there is one.
+// the contiguous axis; along the strided axes the smallest one up to 4096
+// values that holds eight columns (128-byte rows), else four, else what fits.
 uint32_t axis_tile(const FftLine &L, bool contig, FftAxis &ax) {
-  const uint32_t want = contig ? L.len : 4 * L.len;
+  const uint32_t want = contig ? L.len : (8 * L.len <= 4096 ? 8 : 4) * L.len;
   uint32_t tile = want <= 2048 ? 2048 : 4096;
   if (L.len > tile || (!contig && 2 * L.len > tile))
     tile = kTileMax;

@@ -26,9 +26,9 @@
 //
 // 248 bytes per vertex for es instead of 808 (one elementwise or axis pass
 // at a time over two complex arrays), 72 instead of 280 for mhd, 72 instead of
-// 144 for te.  Measured per realisation, whole-array steps -> these: es
-// 256x256x64 726 -> 398 us, es 512x512x128 7.03 -> 3.19 ms, te 800x800x160
-// 7.89 -> 4.77 ms, mhd 135x121x98 343 -> 210 us.  Distance from a 64-bit
+// 144 for te.  Measured per realisation, whole-array steps -> these (with the
+// engine and table work below): es 256x256x64 726 -> 304 us, es 512x512x128
+// 7.05 -> 2.24 ms, te 800x800x160 7.90 -> 2.71 ms, mhd 135x121x98 344 -> 197 us.  Distance from a 64-bit
 // reference 1.0e-15 -> 1.2e-15 to 3e-15: the rounding errors of a vertex and
 // its mirror now coincide instead of averaging in the extraction.
 //
@@ -108,7 +108,7 @@ struct DftDraw {
 // engine's tables).  Bound by the FP64 and integer instructions of the draws:
 // with the band decided on |k|^2, the spectrum as one power of it and the
 // square roots and angles without the library's special cases, te 800x800x160
-// 2633 -> 1416 us, es 256x256x64 94 -> 82 us.
+// 2633 -> 1416 us, es 256x256x64 94 -> 82 us (1207 and 78 with radix 8).
 template <typename Draw, uint32_t TILE, uint32_t NT, int MODE>
 __global__ __launch_bounds__(NT) void k_draw_axis(double2 *__restrict__ o0,
                                                   double2 *__restrict__ o1, Draw dr,
@@ -209,7 +209,7 @@ __global__ __launch_bounds__(1024) void k_var_half(const double *part, uint32_t 
 // line and vertex -l of its mirror are read by no other thread, so the even
 // parts go straight back into the two lines' places.  SPLIT takes the
 // rescale's factors from tables of the tile's 2 CL lines and of z in LDS: the
-// kernel was bound by the per-vertex models (es 256x256x64 106 -> 62 us).
+// kernel was bound by the per-vertex models (es 256x256x64 106 -> 62 us, 55 with radix 8).
 template <bool SPLIT, uint32_t TILE, uint32_t NT, int MODE>
 __global__ __launch_bounds__(NT) void k_es_mid(const double2 *__restrict__ c0,
                                                const double2 *__restrict__ c1, HalfArrays H,
@@ -361,9 +361,12 @@ __global__ __launch_bounds__(NT) void k_es_gs_x(HalfArrays H, EsArgs a, HalfArgs
                                                 uint32_t cs) {
   extern __shared__ double2 lds[];
   const uint32_t n = h.nx, C = 1u << cs, P = 2 * C;
+  const uint32_t col0 = xcd_tile(blockIdx.x, gridDim.x) << cs;
+  if (col0 >= h.ncol)
+    return; // uniform: the grid's last few workgroups
   const double2 *twl = fft_tables<TILE, NT, MODE>(lds, L, P);
   const uint32_t c = threadIdx.x & (C - 1), t0 = threadIdx.x >> cs, dt = NT >> cs;
-  const uint32_t col = (blockIdx.x << cs) + c;
+  const uint32_t col = col0 + c;
   const bool on = col < h.ncol;
   load_half_columns<TILE, NT>(lds, H, h, cs, col, on);
   __syncthreads();
@@ -400,10 +403,13 @@ __global__ __launch_bounds__(NT) void k_mhd_x(HalfArrays H, MhdArgs a, uint64_t 
                                               FftLine L, uint32_t cs) {
   extern __shared__ double2 lds[];
   const uint32_t n = h.nx, C = 1u << cs, P = 2 * C;
+  const uint32_t col0 = xcd_tile(blockIdx.x, gridDim.x) << cs;
+  if (col0 >= h.ncol)
+    return; // uniform: the grid's last few workgroups
   const double2 *twl = fft_tables<TILE, NT, MODE>(lds, L, P);
   const Vec3 bh = versor3(Vec3{bobs[0], bobs[1], bobs[2]});
   const uint32_t c = threadIdx.x & (C - 1), t0 = threadIdx.x >> cs, dt = NT >> cs;
-  const uint32_t col = (blockIdx.x << cs) + c;
+  const uint32_t col = col0 + c;
   const bool on = col < h.ncol;
   const uint32_t j = col / h.nh, l = col - j * h.nh;
 #pragma unroll 1
@@ -482,7 +488,7 @@ __global__ __launch_bounds__(NT) void k_half_out(HalfArrays H, double *__restric
 
 // z(+) and the energy profile of TErnd_dft (ternd_dft.cc:109-128): CL z lines
 // of the whole box.  SPLIT takes the profile's factors from tables in LDS (te
-// 800x800x160 1072 -> 727 us).
+// 800x800x160 1072 -> 727 us, 579 with radix 8).
 template <bool SPLIT, uint32_t TILE, uint32_t NT, int MODE>
 __global__ __launch_bounds__(NT) void k_te_out(const double2 *__restrict__ tk,
                                                double *__restrict__ te, DftArgs a,
@@ -695,7 +701,7 @@ inline int half_gs_x(hamx_ctx *ctx, const HalfPlan &p, const HalfArrays &H, cons
   const uint32_t tile = p.x_tile(2, h.ncol, &cs);
   with_tile(tile, p.lx.mode, [&](auto T, auto NT, auto M) {
     hipLaunchKernelGGL((k_es_gs_x<decltype(T)::value, decltype(NT)::value, decltype(M)::value>),
-                       dim3((h.ncol + (1u << cs) - 1) >> cs), dim3(decltype(NT)::value),
+                       dim3(xcd_grid((h.ncol + (1u << cs) - 1) >> cs)), dim3(decltype(NT)::value),
                        fft_lds_bytes(p.lx, 2u << cs, tile), ctx->stream, H, a, h, p.lx, cs);
   });
   HAMX_HIP(ctx, hipGetLastError());
@@ -710,7 +716,7 @@ inline int half_mhd_x(hamx_ctx *ctx, const HalfPlan &p, const HalfArrays &H, con
   const uint32_t tile = p.x_tile(2, h.ncol, &cs);
   with_tile(tile, p.lx.mode, [&](auto T, auto NT, auto M) {
     hipLaunchKernelGGL((k_mhd_x<decltype(T)::value, decltype(NT)::value, decltype(M)::value>),
-                       dim3((h.ncol + (1u << cs) - 1) >> cs), dim3(decltype(NT)::value),
+                       dim3(xcd_grid((h.ncol + (1u << cs) - 1) >> cs)), dim3(decltype(NT)::value),
                        fft_lds_bytes(p.lx, 2u << cs, tile), ctx->stream, H, a, seed, bobs, h,
                        p.lx, cs);
   });
