@@ -175,8 +175,10 @@ __device__ inline bool eval_sample(const Phys &ph, const Grids &gr,
   double te = 0.;
   if (ph.tereg_model == HAMX_TEREG_UNIF)
     te = tereg_unif(ph.tereg, pos, ph.obs);
-  else if (HEAVY && ph.tereg_model == HAMX_TEREG_YMW16)
-    te = tereg_ymw16_eval(ph.tereg, pos.x, pos.y, pos.z);
+  else if (HEAVY && ph.tereg_model == HAMX_TEREG_YMW16) {
+    const double r2 = pos.x * pos.x + pos.y * pos.y, inv_r = r2 > 0. ? rsqrt_f64(r2) : 0.;
+    te = ymw16_density(ph.ymw, pos.x, pos.y, pos.z, r2 * inv_r, inv_r);
+  }
   else if (ph.tereg_model == HAMX_TEREG_GRID)
     te = gather1(gr.tereg, gr.g_tereg, pos);
   if (PACKED) {
@@ -336,11 +338,13 @@ k_los_wave(Phys ph, Grids gr, ShellArgs sa) {
 }
 
 // ---------------------------------------------------- specialised march --
-// The common model set -- WMAP-LSA regular B, uniform-sphere thermal
-// electrons, a CRE model with a constant spectral index, random grids (if
-// any) packed in one box, synchrotron on -- with the per-sample arithmetic
-// rewritten into fewer, cheaper operations that agree with the reference to
-// rounding:
+// A CRE model with a constant spectral index, random grids (if any) packed in
+// one box, synchrotron on -- above all with WMAP-LSA regular B and uniform-
+// sphere thermal electrons, and (MODELS) with any other regular models, which
+// then took 1.6 to 2.6 times less than the generic march (cartesian B 3.32 ->
+// 1.56 ms, JF12 6.5 -> 4.0, LSA with YMW16 12.75 -> 4.8 on 3 shells up to nside
+// 128) -- with the per-sample arithmetic rewritten into fewer, cheaper
+// operations that agree with the reference to rounding:
 //   * the IAU angle enters only through cos/sin(2 ipa), formed from the two
 //     projections x = -e_phi.B, y = -e_theta.B as ((x^2 - y^2), 2xy)/(x^2+y^2)
 //     instead of atan2, so one sincos of the Faraday phase gives
@@ -353,13 +357,16 @@ k_los_wave(Phys ph, Grids gr, ShellArgs sa) {
 //     TE sphere test, the te > 0 clamp and the grid-cell lookup (divisions
 //     kept) decide exactly as in the reference.
 
-template <bool GRIDS, bool PW1>
 // Four waves per SIMD (at most 128 VGPRs; the allocator moves ~90 scalar
 // values into a 96-byte private segment) measured 4% faster than three
 // (7.30 -> 7.01 ms per pass on the random_forward workload), which in turn
-// measured 8% faster than the unconstrained choice of two.
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_los_fast(
-    Phys ph, FastConst fc, Grids gr, ShellArgs sa) {
+// measured 8% faster than the unconstrained choice of two.  With YMW16 two /
+// three / four waves measured 5.68 / 4.98 / 4.80 ms per march (3 shells up to
+// nside 128); JF12 4.7 / 4.0 ms with two / three.
+template <bool GRIDS, bool PW1, int MODELS>
+__global__ __launch_bounds__(256) __attribute__((
+    amdgpu_waves_per_eu(MODELS == kAllModels ? 3 : 4))) void
+k_los_fast(Phys ph, FastConst fc, Grids gr, ShellArgs sa) {
   // kFastRays consecutive rays per wavefront: their set-up (pointing,
   // versors, FD cache, culled step range) runs one ray per lane into LDS,
   // then the rays are marched one after another, 64 samples per step
@@ -386,7 +393,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
       FastSample o;
       bool valid = false;
       if (k < r.k_hi)
-        valid = eval_fast<GRIDS, PW1>(ph, fc, gr, sa, r, k, o);
+        valid = eval_fast<GRIDS, PW1, MODELS>(ph, fc, gr, sa, r, k, o);
       const double fdk = valid ? o.fdk : 0.;
       const double incl = wave_incl_scan(fdk, lane);
       const double fd_here = fd_carry + incl;
@@ -606,6 +613,8 @@ Phys make_phys(const hamx_los_desc *d) {
   std::memcpy(ph.breg, d->breg, sizeof(ph.breg));
   std::memcpy(ph.tereg, d->tereg, sizeof(ph.tereg));
   std::memcpy(ph.cre, d->cre, sizeof(ph.cre));
+  if (d->tereg_model == HAMX_TEREG_YMW16)
+    ph.ymw = ymw16_fold(d->tereg);
   ph.fd_fore = -(cgs::qe * cgs::qe * cgs::qe) / (2. * cgs::pi * cgs::mec2 * cgs::mec2);
   ph.qe3 = cgs::qe * cgs::qe * cgs::qe;
   ph.three_qe = 3. * cgs::qe;
@@ -981,12 +990,12 @@ int los_forward_impl(hamx_ctx *ctx, const hamx_los_desc *d, const hamx_fields *f
     HAMX_TRY(fill_f64(ctx, o_fd, h_fd.npix, 0.));
 
   const int sched = d->schedule == HAMX_SCHED_THREAD ? HAMX_SCHED_THREAD : HAMX_SCHED_WAVE;
-  // the specialised kernel covers LSA + uniform TE + constant-index CRE with
-  // synchrotron on and the random grids (if any) packed in one box
-  const bool fast = d->schedule == HAMX_SCHED_AUTO && d->breg_model == HAMX_BREG_LSA &&
-                    d->tereg_model == HAMX_TEREG_UNIF && ph.idx_const && d->do_sync &&
+  // the specialised kernel covers a constant-index CRE with synchrotron on
+  // and the random grids (if any) packed in one box
+  const bool fast = d->schedule == HAMX_SCHED_AUTO && ph.idx_const && d->do_sync &&
                     (d->cre_model == HAMX_CRE_ANA || d->cre_model == HAMX_CRE_UNIF) &&
                     (packed || !grids_any);
+  const FastModels models = fast_models(d);
   const bool pw1 = fast && 0.5 * (ph.idx + 1) == -1.0;
   const bool creg = d->cre_model == HAMX_CRE_GRID && d->do_sync;
   // models with large evaluators get kernels of their own (register use)
@@ -1022,18 +1031,30 @@ int los_forward_impl(hamx_ctx *ctx, const hamx_los_desc *d, const hamx_fields *f
       const FastConst fc = make_fast(d, ph, sa.delta, pw1);
       const unsigned blocks =
           static_cast<unsigned>((npix + 4 * kFastRays - 1) / (4 * kFastRays));
+#define HAMX_LAUNCH_FAST(G, P, M)                                                          \
+  hipLaunchKernelGGL((k_los_fast<G, P, M>), dim3(blocks), dim3(256), 0, ctx->stream, ph, fc, gr, \
+                     sa)
+#define HAMX_LAUNCH_FAST_M(G, P)                                                           \
+  do {                                                                                     \
+    if (models == kLsaUnif)                                                                \
+      HAMX_LAUNCH_FAST(G, P, kLsaUnif);                                                    \
+    else if (models == kLightModels)                                                       \
+      HAMX_LAUNCH_FAST(G, P, kLightModels);                                                \
+    else if (models == kYmw16Models)                                                       \
+      HAMX_LAUNCH_FAST(G, P, kYmw16Models);                                                \
+    else                                                                                   \
+      HAMX_LAUNCH_FAST(G, P, kAllModels);                                                  \
+  } while (0)
       if (packed && pw1)
-        hipLaunchKernelGGL((k_los_fast<true, true>), dim3(blocks), dim3(256), 0, ctx->stream,
-                           ph, fc, gr, sa);
+        HAMX_LAUNCH_FAST_M(true, true);
       else if (packed)
-        hipLaunchKernelGGL((k_los_fast<true, false>), dim3(blocks), dim3(256), 0,
-                           ctx->stream, ph, fc, gr, sa);
+        HAMX_LAUNCH_FAST_M(true, false);
       else if (pw1)
-        hipLaunchKernelGGL((k_los_fast<false, true>), dim3(blocks), dim3(256), 0,
-                           ctx->stream, ph, fc, gr, sa);
+        HAMX_LAUNCH_FAST_M(false, true);
       else
-        hipLaunchKernelGGL((k_los_fast<false, false>), dim3(blocks), dim3(256), 0,
-                           ctx->stream, ph, fc, gr, sa);
+        HAMX_LAUNCH_FAST_M(false, false);
+#undef HAMX_LAUNCH_FAST_M
+#undef HAMX_LAUNCH_FAST
     } else if (sched == HAMX_SCHED_WAVE) {
       const unsigned blocks = static_cast<unsigned>((npix + 3) / 4);
 #define HAMX_LAUNCH_WAVE(P, C, H)                                                          \

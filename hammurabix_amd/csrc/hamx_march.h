@@ -16,6 +16,7 @@
 #include "hamx_math.h"
 #include "hamx_healpix.h"
 #include "hamx_internal.h"
+#include "hamx_ymw16.h"
 
 namespace hamx {
 
@@ -45,6 +46,7 @@ struct Phys {
   // the x_fact numerators of J_tot and J_pol in their own operation orders,
   // and the fore factor's 1.73205081 qe^3 and denominator.
   double xft_num, xfp_num, fore_num, fore_den;
+  Ymw16 ymw; // HAMX_TEREG_YMW16
 };
 
 struct Grids {
@@ -505,10 +507,21 @@ struct FastSample {
   double fdk, jt, jp, c2i, s2i;
 };
 
-// MODELS: the regular B and TE come from the descriptor's models (any of
-// them, an LSA field with its parameter partials; a uniform TE sphere with
-// n0's) instead of being LSA and the uniform sphere.
-template <bool GRIDS, bool PW1, bool MODELS = false>
+// MODELS other than kLsaUnif: the regular B and TE come from the descriptor's
+// models (an LSA field with its parameter partials; a uniform TE sphere with
+// n0's) instead of being LSA and the uniform sphere.  JF12, Jaffe and YMW16,
+// whose evaluators take many registers, are compiled in only where the pass
+// has them: kYmw16Models adds YMW16 to the light models, kAllModels all three.
+enum FastModels { kLsaUnif = 0, kLightModels = 1, kYmw16Models = 2, kAllModels = 3 };
+inline FastModels fast_models(const hamx_los_desc *d) {
+  if (d->breg_model == HAMX_BREG_LSA && d->tereg_model == HAMX_TEREG_UNIF)
+    return kLsaUnif;
+  if (d->breg_model == HAMX_BREG_JF12 || d->breg_model == HAMX_BREG_JAFFE)
+    return kAllModels;
+  return d->tereg_model == HAMX_TEREG_YMW16 ? kYmw16Models : kLightModels;
+}
+
+template <bool GRIDS, bool PW1, int MODELS = kLsaUnif>
 __device__ inline bool eval_fast(const Phys &ph, const FastConst &fc, const Grids &gr,
                                  const ShellArgs &sa, const RayGeo &r, uint64_t k,
                                  FastSample &o) {
@@ -527,13 +540,13 @@ __device__ inline bool eval_fast(const Phys &ph, const FastConst &fc, const Grid
   const double rr2 = pos.x * pos.x + pos.y * pos.y;
   const double inv_r = rr2 > 0. ? rsqrt_f64(rr2) : 0.;
   o.rr = rr2 * inv_r;
-  const bool lsa = !MODELS || ph.breg_model == HAMX_BREG_LSA;
+  const bool lsa = MODELS == kLsaUnif || ph.breg_model == HAMX_BREG_LSA;
   o.lsa_in = lsa && !(rr2 > (400. * cgs::kpc * cgs::kpc) || rr2 < (9. * cgs::kpc * cgs::kpc));
-  if (MODELS && !lsa) {
+  if (MODELS != kLsaUnif && !lsa) {
     if (ph.breg_model == HAMX_BREG_GRID)
       B = gather3(gr.breg_x, gr.breg_y, gr.breg_z, gr.g_breg, pos);
     else
-      B = breg_eval<true>(ph.breg_model, ph.breg, pos);
+      B = breg_eval<MODELS == kAllModels>(ph.breg_model, ph.breg, pos);
   }
   // exp(-2|z| / kpc): the LSA's tanh(z / kpc) and, when the CRE scale
   // height is 1 kpc, the CRE's sech^2(z / z0)
@@ -562,15 +575,15 @@ __device__ inline bool eval_fast(const Phys &ph, const FastConst &fc, const Grid
   }
   // uniform TE sphere (tereg_unif.cc:6-12)
   double te = 0.;
-  if (!MODELS || ph.tereg_model == HAMX_TEREG_UNIF) {
+  if (MODELS == kLsaUnif || ph.tereg_model == HAMX_TEREG_UNIF) {
     const Vec3 d{pos.x - ph.obs.x, pos.y - ph.obs.y, pos.z - ph.obs.z};
     o.te_in = !(d.x * d.x + d.y * d.y + d.z * d.z > fc.te_r02);
     if (o.te_in)
       te = fc.n0;
   } else {
     o.te_in = false; // no n0 partial
-    if (ph.tereg_model == HAMX_TEREG_YMW16)
-      te = tereg_ymw16_eval(ph.tereg, pos.x, pos.y, pos.z);
+    if (MODELS >= kYmw16Models && ph.tereg_model == HAMX_TEREG_YMW16)
+      te = ymw16_density(ph.ymw, pos.x, pos.y, pos.z, o.rr, inv_r);
     else if (ph.tereg_model == HAMX_TEREG_GRID)
       te = gather1(gr.tereg, gr.g_tereg, pos);
   }

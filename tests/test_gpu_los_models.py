@@ -1,0 +1,73 @@
+"""The specialised march with every regular-field and electron model, with
+and without packed random grids, for a spectral index of 3 (emissivity as a
+product) and 2.8 (as a power), on the default schedule against the CPU
+oracle: FP64 maps within 1e-10 relative L2 (the plain-path bar)."""
+import numpy as np
+import pytest
+
+from hammurabix_amd import Param, _capi as capi, configs
+from hammurabix_amd.units import CGS
+from oracle_lib import write_grid
+from test_gpu_los import assert_parity, gpu_maps, random_grids
+from test_oracle_models import jf12_params
+
+pytestmark = pytest.mark.gpu
+
+
+def set_breg(d, name):
+    mu, kpc = 1e-6, CGS.kpc
+    if name == "none":
+        d.breg_model = capi.HAMX_BREG_NONE
+    elif name == "cart":
+        d.breg_model = capi.HAMX_BREG_CART
+        d.breg[0:3] = [1 * mu, 2 * mu, 0.5 * mu]
+    elif name == "helix":
+        d.breg_model = capi.HAMX_BREG_HELIX
+        d.breg[0:5] = [1 * mu, 2 * mu, 0.5 * mu, 3 * kpc, 12 * kpc]
+    elif name == "jf12":
+        d.breg_model = capi.HAMX_BREG_JF12
+        d.breg[0:20] = list(jf12_params())
+    elif name == "grid":
+        d.breg_model = capi.HAMX_BREG_GRID
+
+
+@pytest.mark.parametrize("alpha", [3.0, 2.8])
+@pytest.mark.parametrize("random", [True, False])
+@pytest.mark.parametrize("breg,tereg", [("none", "unif"), ("cart", "none"), ("helix", "unif"),
+                                        ("grid", "grid"), ("lsa", "none"), ("lsa", "ymw16"),
+                                        ("cart", "ymw16"), ("jf12", "unif"), ("jf12", "ymw16")])
+def test_models(ctx, breg, tereg, random, alpha):
+    print("case:", breg, tereg, random, alpha, flush=True)
+    par = Param(text=configs.random_forward(
+        nside_sim=2, nside_out=8, oc_r_res=0.043, grid=(16, 16, 8),
+        tereg="ymw16" if tereg == "ymw16" else "unif"))
+    d = par.los_desc()
+    d.cre[0] = alpha
+    set_breg(d, breg)
+    grids = {}
+    b, te, box = random_grids((16, 16, 8), seed=3, te_scale=0.002)
+    if random:
+        grids.update(brnd=b, brnd_box=box, ternd=te, ternd_box=box)
+    if breg == "grid":
+        g, t, gbox = random_grids((9, 11, 7), seed=4)
+        grids.update(breg=g, breg_box=gbox, tereg=np.abs(t), tereg_box=gbox)
+    if tereg == "grid":
+        d.tereg_model = capi.HAMX_TEREG_GRID
+    elif tereg == "none":
+        d.tereg_model = capi.HAMX_TEREG_NONE
+    if (breg, random) == ("none", False):
+        return  # no field at all: nothing to compare
+    if tereg == "none" and not random:
+        d.do_dm = d.do_fd = 0  # zero maps
+    ref = {k: v for k, v in write_grid(d, **grids).items() if np.any(v)}
+    got = gpu_maps(ctx, d, **grids)
+    assert_parity({k: got[k] for k in ref}, ref, label=f"{breg}/{tereg}")
+
+
+def test_ymw16_through_its_nebulae(ctx):
+    """A short, finely sampled shell about the Sun: the Local Bubble, Loop I
+    and the Gum shell, whose shortened forms are this march's own."""
+    par = Param(text=configs.plain_forward(tereg="ymw16", nside_sim=8, nside_out=8,
+                                           oc_r_max=1.5, oc_r_res=0.002))
+    d = par.los_desc()
+    assert_parity(gpu_maps(ctx, d), write_grid(d), label="ymw16 nebulae")
