@@ -41,6 +41,7 @@
 #include "hamx_healpix.h"
 #include "hamx_internal.h"
 #include "hamx_march.h"
+#include "hamx_cre_grid.h"
 #include "hamx_sync.h"
 
 namespace hamx {
@@ -73,84 +74,10 @@ __device__ inline double cre_index(const Phys &ph, const Vec3 &pos) {
   return -ph.cre[0] + ph.cre[1] * r + ph.cre[2] * z;
 }
 
-// CREfield::read_grid_num (cre.cc:144-199) of energy bin e in a cell found by
-// grid_cell on the CRE box: the same z, y, x interpolation order over the
-// [x][y][z][E] layout (z neighbours nE apart).
-__device__ inline double lerp_cell_e(const double *f, const Cell &c, uint64_t nE,
-                                     uint64_t sy, uint64_t sx, uint64_t e) {
-  const uint64_t i00 = c.idx * nE + e, i01 = i00 + sy, i10 = i00 + sx, i11 = i00 + sx + sy;
-  const double i1 = f[i00] * (1. - c.zd) + f[i00 + nE] * c.zd;
-  const double i2 = f[i01] * (1 - c.zd) + f[i01 + nE] * c.zd;
-  const double j1 = f[i10] * (1 - c.zd) + f[i10 + nE] * c.zd;
-  const double j2 = f[i11] * (1 - c.zd) + f[i11 + nE] * c.zd;
-  const double w1 = i1 * (1 - c.yd) + i2 * c.yd;
-  const double w2 = j1 * (1 - c.yd) + j2 * c.yd;
-  return w1 * (1 - c.xd) + w2 * c.xd;
-}
-
-// sync_emissivity_t and _p with the CRE grid (integrator.cc:286-325 and
-// 355-394) for one sample: the midpoint rule over the energy bins of
-// F(x) resp. G(x) times the bin-mean flux / beta, bins whose mean x exceeds
-// 100 skipped, then the fore factor.  Each bin's gather is shared by J_tot
-// and J_pol and reused by the next bin.  Outside the grid every gathered
-// flux is 0 and so are both sums.
-// The kernels of one bin come from one evaluation: u = ln(x_fact) +
-// ln((1/E_{i+1}^2 + 1/E_i^2) / 2) (the second term tabulated per bin) in
-// place of ln(xv), and G at the J_pol mean xvp, which may differ from the
-// J_tot mean xvt in the last bits (the two x_fact products round
-// differently), as G(xvt) (1 + xvt - xvp), exact to first order.
-__device__ inline void cre_grid_emissivity(const Phys &ph, const Grids &gr, const Vec3 &pos,
-                                           double b_per, const double *stab, double &jt,
-                                           double &jp) {
-  jt = 0.;
-  jp = 0.;
-  Cell c;
-  if (!grid_cell(gr.g_cre, pos, c))
-    return;
-  const double ab = fabs(b_per);
-  const double den = ph.three_qe * ab;
-  const double xft = ph.xft_num / den;
-  const double xfp = ph.xfp_num / den;
-  const uint64_t nE = gr.cre_nE;
-  const uint64_t sy = gr.g_cre.nz * nE, sx = gr.g_cre.ny * sy;
-  const double *ke2 = gr.cre_tab, *beta = ke2 + nE, *dE = beta + nE, *lnc = dE + nE;
-  const double lxt = log(xft);
-  double xt0 = xft / ke2[0], xp0 = xfp / ke2[0];
-  double g0 = 0.;
-  bool have0 = false;
-  double Jt = 0., Jp = 0.;
-  for (uint64_t i = 0; i + 1 < nE; ++i) {
-    const double xt1 = xft / ke2[i + 1], xp1 = xfp / ke2[i + 1];
-    const double xvt = 0.5 * (xt1 + xt0), xvp = 0.5 * (xp1 + xp0);
-    const bool on_t = !(xvt > 100), on_p = !(xvp > 100);
-    if (on_t || on_p) {
-      if (!have0)
-        g0 = lerp_cell_e(gr.cre, c, nE, sy, sx, i) / beta[i];
-      const double g1 = lerp_cell_e(gr.cre, c, nE, sy, sx, i + 1) / beta[i + 1];
-      const double flux = 0.5 * (g1 + g0);
-      double F, G;
-      sync_fg(stab, lxt + lnc[i], xvt, F, G);
-      if (on_t)
-        Jt += F * flux * dE[i];
-      if (on_p)
-        Jp += G * (1. + (xvt - xvp)) * flux * dE[i];
-      g0 = g1;
-      have0 = true;
-    } else {
-      have0 = false;
-    }
-    xt0 = xt1;
-    xp0 = xp1;
-  }
-  const double fore = ph.fore_num * ab / ph.fore_den;
-  jt = Jt * fore;
-  jp = Jp * fore;
-}
-
 template <bool PACKED, bool CREG, bool HEAVY>
 __device__ inline bool eval_sample(const Phys &ph, const Grids &gr,
                                    const ShellArgs &sa, const RayGeo &r,
-                                   uint64_t k, SampleOut &s, const double *stab) {
+                                   uint64_t k, SampleOut &s, const double2 *stab) {
   const double dist =
       sa.d_start + (static_cast<double>(static_cast<uint32_t>(k)) + 0.5) * sa.delta;
   const Vec3 pos{r.l.x * dist + ph.obs.x, r.l.y * dist + ph.obs.y,
@@ -288,7 +215,7 @@ template <bool PACKED, bool CREG, bool HEAVY>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CREG ? 3 : 2))) void
 k_los_wave(Phys ph, Grids gr, ShellArgs sa) {
   // the synchrotron kernel tables of the CRE grid emissivities, in LDS
-  __shared__ double stab[CREG ? kSyncTab : 1];
+  __shared__ double2 stab[CREG ? kSyncTab : 1];
   if (CREG) {
     load_sync_tab(stab);
     __syncthreads();
@@ -363,10 +290,16 @@ k_los_wave(Phys ph, Grids gr, ShellArgs sa) {
 // measured 8% faster than the unconstrained choice of two.  With YMW16 two /
 // three / four waves measured 5.68 / 4.98 / 4.80 ms per march (3 shells up to
 // nside 128); JF12 4.7 / 4.0 ms with two / three.
-template <bool GRIDS, bool PW1, int MODELS>
+template <bool GRIDS, bool PW1, int MODELS, bool CREG>
 __global__ __launch_bounds__(256) __attribute__((
-    amdgpu_waves_per_eu(MODELS == kAllModels ? 3 : 4))) void
+    amdgpu_waves_per_eu(MODELS == kAllModels || CREG ? 3 : 4))) void
 k_los_fast(Phys ph, FastConst fc, Grids gr, ShellArgs sa) {
+  // the synchrotron kernels' table of the CRE grid emissivities
+  __shared__ double2 stab[CREG ? kSyncTab : 1];
+  if constexpr (CREG) {
+    load_sync_tab(stab);
+    __syncthreads();
+  }
   // kFastRays consecutive rays per wavefront: their set-up (pointing,
   // versors, FD cache, culled step range) runs one ray per lane into LDS,
   // then the rays are marched one after another, 64 samples per step
@@ -393,7 +326,7 @@ k_los_fast(Phys ph, FastConst fc, Grids gr, ShellArgs sa) {
       FastSample o;
       bool valid = false;
       if (k < r.k_hi)
-        valid = eval_fast<GRIDS, PW1, MODELS>(ph, fc, gr, sa, r, k, o);
+        valid = eval_fast<GRIDS, PW1, MODELS, CREG>(ph, fc, gr, sa, r, k, o, stab);
       const double fdk = valid ? o.fdk : 0.;
       const double incl = wave_incl_scan(fdk, lane);
       const double fd_here = fd_carry + incl;
@@ -420,7 +353,7 @@ k_los_fast(Phys ph, FastConst fc, Grids gr, ShellArgs sa) {
 template <bool PACKED, bool CREG, bool HEAVY>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CREG ? 3 : 2))) void
 k_los_thread(Phys ph, Grids gr, ShellArgs sa) {
-  __shared__ double stab[CREG ? kSyncTab : 1];
+  __shared__ double2 stab[CREG ? kSyncTab : 1];
   if (CREG) {
     load_sync_tab(stab);
     __syncthreads();
@@ -673,6 +606,7 @@ Phys make_phys(const hamx_los_desc *d) {
 FastConst make_fast(const hamx_los_desc *d, const Phys &ph, double delta, bool pw1) {
   FastConst fc;
   std::memset(&fc, 0, sizeof(fc));
+  const bool creg = d->cre_model == HAMX_CRE_GRID;
   fc.b0 = d->breg[0];
   fc.psi0 = d->breg[1];
   fc.psi1 = d->breg[2];
@@ -688,6 +622,11 @@ FastConst make_fast(const hamx_los_desc *d, const Phys &ph, double delta, bool p
   fc.te_r0 = d->tereg[1];
   fc.te_r02 = d->tereg[1] * d->tereg[1];
   fc.cre_unif = d->cre_model == HAMX_CRE_UNIF;
+  if (creg) { // the flux grid's emissivities take delta i2bt alone
+    fc.kt = fc.kp = delta * ph.i2bt;
+    fc.fd_scale = ph.fd_fore * delta;
+    return fc;
+  }
   if (fc.cre_unif) {
     fc.cre_r0 = d->cre[1];
     fc.cre_r02 = d->cre[1] * d->cre[1];
@@ -792,18 +731,19 @@ int stage_fields(hamx_ctx *ctx, const hamx_los_desc *d, const hamx_fields &f,
     gr.cre = static_cast<const double *>(p);
     gr.g_cre = grid_geo(f.cre_box);
     gr.cre_nE = nE;
-    // E_i, x denominators and beta as integrator.cc:300-304 forms them
+    // the energies and beta as integrator.cc:300-304 forms them
     std::vector<double> &tab = ctx->host_tab;
     tab.assign(4 * nE, 0.);
     std::vector<double> KE(nE);
     for (uint64_t i = 0; i != nE; ++i) {
       KE[i] = f.cre_E_min * std::exp(i * f.cre_E_fact);
-      tab[i] = KE[i] * KE[i];
-      tab[nE + i] = std::sqrt(1 - cgs::mec2 / KE[i]);
+      tab[kCreInvBeta * nE + i] = 1. / std::sqrt(1 - cgs::mec2 / KE[i]);
     }
     for (uint64_t i = 0; i + 1 < nE; ++i) {
-      tab[2 * nE + i] = std::fabs(KE[i + 1] - KE[i]);
-      tab[3 * nE + i] = std::log(0.5 * (1. / tab[i + 1] + 1. / tab[i]));
+      const double c = 0.5 * (1. / (KE[i + 1] * KE[i + 1]) + 1. / (KE[i] * KE[i]));
+      tab[kCreC * nE + i] = c;
+      tab[kCreLnC * nE + i] = std::log(c);
+      tab[kCreHalfDE * nE + i] = 0.5 * std::fabs(KE[i + 1] - KE[i]);
     }
     if (ar)
       return set_err(ctx, HAMX_ERR_UNSUPPORTED,
@@ -817,7 +757,10 @@ int stage_fields(hamx_ctx *ctx, const hamx_los_desc *d, const hamx_fields &f,
   // Pack the random B components and TE density into one record per vertex
   // when they share a box: 64 B contiguous per z-pair of corners.
   packed = false;
-  if (!ar && d->cre_model != HAMX_CRE_GRID && has_brnd &&
+  // (the generic march over a CRE flux grid gathers them where they lie)
+  const bool pack = d->cre_model != HAMX_CRE_GRID ||
+                    (d->schedule == HAMX_SCHED_AUTO && d->do_sync);
+  if (!ar && pack && has_brnd &&
       (!f.ternd || same_box(f.brnd_box, f.ternd_box))) {
     const uint64_t n = box_size(f.brnd_box);
     void *pk;
@@ -990,14 +933,15 @@ int los_forward_impl(hamx_ctx *ctx, const hamx_los_desc *d, const hamx_fields *f
     HAMX_TRY(fill_f64(ctx, o_fd, h_fd.npix, 0.));
 
   const int sched = d->schedule == HAMX_SCHED_THREAD ? HAMX_SCHED_THREAD : HAMX_SCHED_WAVE;
-  // the specialised kernel covers a constant-index CRE with synchrotron on
-  // and the random grids (if any) packed in one box
-  const bool fast = d->schedule == HAMX_SCHED_AUTO && ph.idx_const && d->do_sync &&
-                    (d->cre_model == HAMX_CRE_ANA || d->cre_model == HAMX_CRE_UNIF) &&
+  // the specialised kernel covers a constant-index CRE or an imported flux
+  // grid, with synchrotron on and the random grids (if any) packed in one box
+  const bool creg = d->cre_model == HAMX_CRE_GRID && d->do_sync;
+  const bool fast = d->schedule == HAMX_SCHED_AUTO && d->do_sync &&
+                    (creg || (ph.idx_const && (d->cre_model == HAMX_CRE_ANA ||
+                                               d->cre_model == HAMX_CRE_UNIF))) &&
                     (packed || !grids_any);
   const FastModels models = fast_models(d);
-  const bool pw1 = fast && 0.5 * (ph.idx + 1) == -1.0;
-  const bool creg = d->cre_model == HAMX_CRE_GRID && d->do_sync;
+  const bool pw1 = fast && (creg || 0.5 * (ph.idx + 1) == -1.0);
   // models with large evaluators get kernels of their own (register use)
   const bool heavy = d->breg_model == HAMX_BREG_JF12 || d->breg_model == HAMX_BREG_JAFFE ||
                      d->tereg_model == HAMX_TEREG_YMW16;
@@ -1031,21 +975,34 @@ int los_forward_impl(hamx_ctx *ctx, const hamx_los_desc *d, const hamx_fields *f
       const FastConst fc = make_fast(d, ph, sa.delta, pw1);
       const unsigned blocks =
           static_cast<unsigned>((npix + 4 * kFastRays - 1) / (4 * kFastRays));
-#define HAMX_LAUNCH_FAST(G, P, M)                                                          \
-  hipLaunchKernelGGL((k_los_fast<G, P, M>), dim3(blocks), dim3(256), 0, ctx->stream, ph, fc, gr, \
-                     sa)
+#define HAMX_LAUNCH_FAST(G, P, M, C)                                                       \
+  hipLaunchKernelGGL((k_los_fast<G, P, M, C>), dim3(blocks), dim3(256), 0, ctx->stream, ph, fc, \
+                     gr, sa)
 #define HAMX_LAUNCH_FAST_M(G, P)                                                           \
   do {                                                                                     \
     if (models == kLsaUnif)                                                                \
-      HAMX_LAUNCH_FAST(G, P, kLsaUnif);                                                    \
+      HAMX_LAUNCH_FAST(G, P, kLsaUnif, false);                                             \
     else if (models == kLightModels)                                                       \
-      HAMX_LAUNCH_FAST(G, P, kLightModels);                                                \
+      HAMX_LAUNCH_FAST(G, P, kLightModels, false);                                         \
     else if (models == kYmw16Models)                                                       \
-      HAMX_LAUNCH_FAST(G, P, kYmw16Models);                                                \
+      HAMX_LAUNCH_FAST(G, P, kYmw16Models, false);                                         \
     else                                                                                   \
-      HAMX_LAUNCH_FAST(G, P, kAllModels);                                                  \
+      HAMX_LAUNCH_FAST(G, P, kAllModels, false);                                           \
   } while (0)
-      if (packed && pw1)
+#define HAMX_LAUNCH_FAST_CREG(G)                                                           \
+  do {                                                                                     \
+    if (models == kLsaUnif)                                                                \
+      HAMX_LAUNCH_FAST(G, true, kLsaUnif, true);                                           \
+    else if (models == kLightModels)                                                       \
+      HAMX_LAUNCH_FAST(G, true, kLightModels, true);                                       \
+    else                                                                                   \
+      HAMX_LAUNCH_FAST(G, true, kAllModels, true);                                         \
+  } while (0)
+      if (creg && packed)
+        HAMX_LAUNCH_FAST_CREG(true);
+      else if (creg)
+        HAMX_LAUNCH_FAST_CREG(false);
+      else if (packed && pw1)
         HAMX_LAUNCH_FAST_M(true, true);
       else if (packed)
         HAMX_LAUNCH_FAST_M(true, false);
@@ -1053,6 +1010,7 @@ int los_forward_impl(hamx_ctx *ctx, const hamx_los_desc *d, const hamx_fields *f
         HAMX_LAUNCH_FAST_M(false, true);
       else
         HAMX_LAUNCH_FAST_M(false, false);
+#undef HAMX_LAUNCH_FAST_CREG
 #undef HAMX_LAUNCH_FAST_M
 #undef HAMX_LAUNCH_FAST
     } else if (sched == HAMX_SCHED_WAVE) {
@@ -1333,7 +1291,7 @@ __global__ __launch_bounds__(256) void k_cre_write(Phys ph, CreWriteArgs a, doub
 
 __global__ __launch_bounds__(256) void k_sync_fg(const double *x, uint64_t n, double *F,
                                                  double *G) {
-  __shared__ double tab[kSyncTab];
+  __shared__ double2 tab[kSyncTab];
   load_sync_tab(tab);
   __syncthreads();
   const uint64_t stride = static_cast<uint64_t>(gridDim.x) * blockDim.x;

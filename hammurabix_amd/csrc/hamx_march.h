@@ -60,9 +60,8 @@ struct Grids {
   GridGeo g_breg;
   const double *tereg;
   GridGeo g_tereg;
-  // CRE_num grid [x][y][z][E] and its energy tables: E_i^2, beta_i,
-  // |E_{i+1} - E_i| and ln((1/E_{i+1}^2 + 1/E_i^2) / 2), cre_nE doubles
-  // each from cre_tab
+  // CRE_num grid [x][y][z][E] and its energy tables (hamx_cre_grid.h),
+  // cre_nE doubles each from cre_tab
   const double *cre;
   GridGeo g_cre;
   uint64_t cre_nE;
@@ -464,6 +463,11 @@ __device__ inline void scatter_staged(const StagedCache &c, double *__restrict__
   wave_lds_sync();
 }
 
+// hamx_cre_grid.h
+__device__ inline void cre_grid_emissivity(const Phys &ph, const Grids &gr, const Vec3 &pos,
+                                           double b_per, const double2 *stab, double &jt,
+                                           double &jp);
+
 // Per-shell constants of the specialised march (see make_fast).
 struct FastConst {
   double psi0, psi1, chi0, b0;
@@ -521,10 +525,12 @@ inline FastModels fast_models(const hamx_los_desc *d) {
   return d->tereg_model == HAMX_TEREG_YMW16 ? kYmw16Models : kLightModels;
 }
 
-template <bool GRIDS, bool PW1, int MODELS = kLsaUnif>
+// CREG: the emissivities of an imported CRE flux grid (stab: the synchrotron
+// kernels' table in LDS) instead of the constant-index model's.
+template <bool GRIDS, bool PW1, int MODELS = kLsaUnif, bool CREG = false>
 __device__ inline bool eval_fast(const Phys &ph, const FastConst &fc, const Grids &gr,
                                  const ShellArgs &sa, const RayGeo &r, uint64_t k,
-                                 FastSample &o) {
+                                 FastSample &o, const double2 *stab = nullptr) {
   // k < 2^31 (validate_los): one 32-bit conversion
   const double dist =
       sa.d_start + (static_cast<double>(static_cast<uint32_t>(k)) + 0.5) * sa.delta;
@@ -551,7 +557,7 @@ __device__ inline bool eval_fast(const Phys &ph, const FastConst &fc, const Grid
   // exp(-2|z| / kpc): the LSA's tanh(z / kpc) and, when the CRE scale
   // height is 1 kpc, the CRE's sech^2(z / z0)
   const double u = pos.z * fc.inv_kpc;
-  const double e_kpc = (o.lsa_in || fc.cre_z_kpc) ? exp_fast(-2. * fabs(u)) : 0.;
+  const double e_kpc = (o.lsa_in || (!CREG && fc.cre_z_kpc)) ? exp_fast(-2. * fabs(u)) : 0.;
   if (o.lsa_in) {
     o.cos_p = pos.x * inv_r;
     o.sin_p = pos.y * inv_r;
@@ -612,22 +618,28 @@ __device__ inline bool eval_fast(const Phys &ph, const FastConst &fc, const Grid
                 B.x * r.l.y - B.y * r.l.x};
   o.bper2 = cr.x * cr.x + cr.y * cr.y + cr.z * cr.z;
   o.bper = sqrt(o.bper2);
-  if (fc.cre_unif) {
-    const Vec3 d{pos.x - ph.obs.x, pos.y - ph.obs.y, pos.z - ph.obs.z};
-    o.prof = (d.x * d.x + d.y * d.y + d.z * d.z > fc.cre_r02) ? 0. : 1.;
+  if constexpr (CREG) {
+    cre_grid_emissivity(ph, gr, pos, o.bper, stab, o.jt, o.jp);
+    o.jt *= fc.kt; // delta i2bt
+    o.jp *= fc.kp;
   } else {
-    // sech^2(z / z0) = 4 e / (1 + e)^2 with e = exp(-2 |z| / z0) <= 1
-    const double e = fc.cre_z_kpc ? e_kpc : exp_fast(-2. * fabs(pos.z * fc.inv_cre_z0));
-    const double d = 1. + e;
-    o.prof = exp_fast((fc.R0 - o.rr) * fc.inv_cre_r0) * (4. * e) * rcp_f64(d * d);
+    if (fc.cre_unif) {
+      const Vec3 d{pos.x - ph.obs.x, pos.y - ph.obs.y, pos.z - ph.obs.z};
+      o.prof = (d.x * d.x + d.y * d.y + d.z * d.z > fc.cre_r02) ? 0. : 1.;
+    } else {
+      // sech^2(z / z0) = 4 e / (1 + e)^2 with e = exp(-2 |z| / z0) <= 1
+      const double e = fc.cre_z_kpc ? e_kpc : exp_fast(-2. * fabs(pos.z * fc.inv_cre_z0));
+      const double d = 1. + e;
+      o.prof = exp_fast((fc.R0 - o.rr) * fc.inv_cre_r0) * (4. * e) * rcp_f64(d * d);
+    }
+    double w;
+    if (PW1)
+      w = o.prof * o.bper2;
+    else
+      w = o.prof * o.bper * pow(fc.a_coef / o.bper, fc.pw_e);
+    o.jt = w * fc.kt;
+    o.jp = w * fc.kp;
   }
-  double w;
-  if (PW1)
-    w = o.prof * o.bper2;
-  else
-    w = o.prof * o.bper * pow(fc.a_coef / o.bper, fc.pw_e);
-  o.jt = w * fc.kt;
-  o.jp = w * fc.kp;
   // cos / sin of twice the IAU angle (integrator.cc:257-265)
   o.x = -dot0(r.eph, B);
   o.y = -dot0(r.eth, B);
