@@ -4,10 +4,12 @@
 //
 // Per sample, over the nE - 1 energy bins: the mean x of the bin's ends (above
 // 100 the bin is skipped), the mean of flux / beta at its ends, F(x) and G(x)
-// (hamx_sync.h), the midpoint sums, then the fore factor.  Bound by the three
-// pipes together -- FP64, LDS (the coefficients) and the vector memory path
-// (the flux) -- so each bin's share of each is kept small: about 60 FP64
-// instructions, 8 16-byte LDS reads, 4 16-byte loads.
+// (hamx_sync.h), the midpoint sums, then the fore factor.  Bound by FP64
+// instructions (about half of the issue slots) and by the latency of the flux
+// loads at three waves per SIMD; four waves spill (1.8 -> 2.3 ms).  Measured on
+// 3 shells up to nside 64, 40x40x8 cells with 32 energies, ms per pass:
+// literal form in the generic march 5.03; this file's 3.65; tables by scalar
+// loads 2.9; loads ahead of the kernels 2.7; four wavefronts per ray 1.88.
 //
 // * x = x_fact c_i and ln x = ln x_fact + ln c_i, with c_i and its logarithm
 //   tabulated on the host; J_tot and J_pol share x (their x_fact differ in
@@ -41,8 +43,13 @@ __device__ inline void cre_grid_emissivity(const Phys &ph, const Grids &gr, cons
   if (ab == 0. || !grid_cell(gr.g_cre, pos, c))
     return; // no field: every bin's x is infinite; outside the grid: no flux
   const uint32_t nE = static_cast<uint32_t>(gr.cre_nE);
-  const double *tc = gr.cre_tab + kCreC * nE, *tl = gr.cre_tab + kCreLnC * nE;
-  const double *td = gr.cre_tab + kCreHalfDE * nE, *tb = gr.cre_tab + kCreInvBeta * nE;
+  // in the constant address space (written before the launch, read by every
+  // lane at one index): scalar loads, where a generic pointer's would be vector
+  // loads, the march's stores after them possibly aliasing
+  typedef const __attribute__((address_space(4))) double *ConstTab;
+  const ConstTab tab = (ConstTab)gr.cre_tab;
+  const ConstTab tc = tab + kCreC * nE, tl = tab + kCreLnC * nE;
+  const ConstTab td = tab + kCreHalfDE * nE, tb = tab + kCreInvBeta * nE;
   const double xf = ph.xft_num / (ph.three_qe * ab);
   const double lx = log_pos(xf);
   // the first pair of bins that any lane keeps (uniform: the energy loop then
@@ -50,47 +57,66 @@ __device__ inline void cre_grid_emissivity(const Phys &ph, const Grids &gr, cons
   uint32_t q = 0;
   while (2 * q + 2 < nE && !__ballot(xf * tc[2 * q + 2 < nE - 1 ? 2 * q + 1 : nE - 2] <= 100.))
     ++q;
+  if (2 * q + 1 >= nE)
+    return; // uniform: no bin is kept
   const uint64_t sz = nE, sy = gr.g_cre.nz * sz, sx = gr.g_cre.ny * sy;
-  const double *f0 = gr.cre + c.idx * sz, *f1 = f0 + sy, *f2 = f0 + sx, *f3 = f2 + sy;
+  const double *f0 = gr.cre + c.idx * sz;
+  const double *fp[4] = {f0, f0 + sy, f0 + sx, f0 + sx + sy};
   const double x1 = 1. - c.xd, y1 = 1. - c.yd, z1 = 1. - c.zd;
-  const double w0 = x1 * y1, w1 = x1 * c.yd, w2 = c.xd * y1, w3 = c.xd * c.yd;
-  const double wa[4] = {w0 * z1, w1 * z1, w2 * z1, w3 * z1};
-  const double wb[4] = {w0 * c.zd, w1 * c.zd, w2 * c.zd, w3 * c.zd};
-  const double *fp[4] = {f0, f1, f2, f3};
-  double Jt = 0., Jp = 0.;
-  auto bin = [&](uint32_t i, double flux2) { // flux2: the sum over the bin's ends
-    const double x = xf * tc[i];
-    double F, G;
-    sync_fg(stab, lx + tl[i], x, F, G);
-    const double m = !(x > 100.) ? flux2 * td[i] : 0.;
-    Jt = fma(!(x > 100.) ? F : 0., m, Jt);
-    Jp = fma(!(x > 100.) ? G : 0., m, Jp);
-  };
-  double last = 0.;
-  bool have = false;
-  for (uint32_t e = 2 * q; e < nE; e += 2) {
-    double g0 = 0., g1 = 0.;
-    if (e + 1 < nE) {
+  const double w[4] = {x1 * y1, x1 * c.yd, c.xd * y1, c.xd * c.yd};
+  const double wa[4] = {w[0] * z1, w[1] * z1, w[2] * z1, w[3] * z1};
+  const double wb[4] = {w[0] * c.zd, w[1] * c.zd, w[2] * c.zd, w[3] * c.zd};
+  // energies e and e + 1 from every corner; with an odd nE the last energy is
+  // the second of the pair before it
+  FluxPair ra[4], rb[4];
+  auto load = [&](uint32_t e) {
+    const uint32_t at = e + 1 < nE ? e : nE - 2;
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const FluxPair a = *reinterpret_cast<const FluxPair *>(fp[k] + e);
-        const FluxPair b = *reinterpret_cast<const FluxPair *>(fp[k] + sz + e);
-        g0 = fma(b.a, wb[k], fma(a.a, wa[k], g0));
-        g1 = fma(b.b, wb[k], fma(a.b, wa[k], g1));
-      }
-      g1 *= tb[e + 1];
-    } else {
-#pragma unroll
-      for (int k = 0; k < 4; ++k)
-        g0 = fma(fp[k][sz + e], wb[k], fma(fp[k][e], wa[k], g0));
+    for (int k = 0; k < 4; ++k) {
+      ra[k] = *reinterpret_cast<const FluxPair *>(fp[k] + at);
+      rb[k] = *reinterpret_cast<const FluxPair *>(fp[k] + sz + at);
     }
-    g0 *= tb[e];
-    if (have)
-      bin(e - 1, last + g0);
+  };
+  double g0, g1;
+  auto lerp = [&](uint32_t e) {
+    const uint32_t at = e + 1 < nE ? e : nE - 2;
+    g0 = g1 = 0.;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      g0 = fma(rb[k].a, wb[k], fma(ra[k].a, wa[k], g0));
+      g1 = fma(rb[k].b, wb[k], fma(ra[k].b, wa[k], g1));
+    }
+    g0 *= tb[at];
+    g1 *= tb[at + 1];
+  };
+  // F and G of a bin times half its width, 0 where it is skipped
+  auto kernels = [&](uint32_t i, double &F, double &G) {
+    const double x = xf * tc[i];
+    sync_fg(stab, lx + tl[i], x, F, G);
+    const double m = td[i];
+    F = x > 100. ? 0. : F * m;
+    G = x > 100. ? 0. : G * m;
+  };
+  double F, G;
+  load(2 * q);
+  kernels(2 * q, F, G);
+  lerp(2 * q);
+  double Jt = F * (g0 + g1), Jp = G * (g0 + g1), last = g1;
+  // the loads of a step are in flight while its two bins' kernels, which do
+  // not depend on them, are evaluated
+  for (uint32_t e = 2 * q + 2; e < nE; e += 2) {
+    double F2 = 0., G2 = 0.;
+    load(e);
+    kernels(e - 1, F, G);
     if (e + 1 < nE)
-      bin(e, g0 + g1);
+      kernels(e, F2, G2);
+    lerp(e);
+    const double first = e + 1 < nE ? g0 : g1;
+    Jt = fma(F, last + first, Jt);
+    Jp = fma(G, last + first, Jp);
+    Jt = fma(F2, g0 + g1, Jt);
+    Jp = fma(G2, g0 + g1, Jp);
     last = g1;
-    have = true;
   }
   const double fore = ph.fore_num * ab / ph.fore_den;
   jt = Jt * fore;

@@ -350,6 +350,86 @@ k_los_fast(Phys ph, FastConst fc, Grids gr, ShellArgs sa) {
   }
 }
 
+// The same march with the four wavefronts of a workgroup on one ray, 256
+// consecutive samples per step (`rays` rays per workgroup, one after another,
+// set up one per lane): the running Faraday depth adds the earlier
+// wavefronts' sums of the step, handed over in LDS.
+constexpr int kRayMax = 4;
+template <bool GRIDS, bool PW1, int MODELS, bool CREG>
+__global__ __launch_bounds__(256) __attribute__((
+    amdgpu_waves_per_eu(MODELS == kAllModels || CREG ? 3 : 4))) void
+k_los_ray(Phys ph, FastConst fc, Grids gr, ShellArgs sa, int rays) {
+  __shared__ double2 stab[CREG ? kSyncTab : 1];
+  __shared__ RayGeo slots[kRayMax];
+  // a step's (a ray's) sums, in turn in either half: one barrier per step
+  // (ray) keeps a half from being rewritten while it may still be read
+  __shared__ double part[2][4], sums[2][4][4];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const uint64_t p0 = static_cast<uint64_t>(blockIdx.x) * rays;
+  const int nr = sa.hs.npix - p0 < static_cast<uint64_t>(rays)
+                     ? static_cast<int>(sa.hs.npix - p0)
+                     : rays;
+  if constexpr (CREG)
+    load_sync_tab(stab);
+  if (static_cast<int>(threadIdx.x) < nr)
+    ray_setup(ph, sa, p0 + threadIdx.x, slots[threadIdx.x]);
+  __syncthreads();
+  const double two_l2 = 2. * ph.lambda_sq;
+  int turn = 0;
+  for (int j = 0; j < nr; ++j) {
+    const uint64_t ipix = p0 + j;
+    if (masked_out(ph, sa, ipix, threadIdx.x == 0))
+      continue; // uniform
+    const RayGeo r = slots[j];
+    double dm = 0., I = 0., Q = 0., U = 0., fd_carry = 0.;
+    for (uint64_t base = r.k_lo; base < r.k_hi; base += 256, turn ^= 1) {
+      const uint64_t k = base + threadIdx.x;
+      FastSample o;
+      bool valid = false;
+      if (k < r.k_hi)
+        valid = eval_fast<GRIDS, PW1, MODELS, CREG>(ph, fc, gr, sa, r, k, o, stab);
+      const double incl = wave_incl_scan(valid ? o.fdk : 0., lane);
+      if (lane == 63)
+        part[turn][wave] = incl;
+      __syncthreads();
+      double fd_here = fd_carry + incl;
+#pragma unroll
+      for (int w = 0; w < 4; ++w) {
+        const double t = part[turn][w];
+        fd_here += w < wave ? t : 0.;
+        fd_carry += t;
+      }
+      if (valid) {
+        double sph, cph;
+        sincos_fast(two_l2 * (r.fd_inner + fd_here), sph, cph);
+        I += o.jt;
+        Q += (cph * o.c2i - sph * o.s2i) * o.jp;
+        U += (sph * o.c2i + cph * o.s2i) * o.jp;
+        dm += o.te;
+      }
+    }
+    dm = wave_sum(dm);
+    I = wave_sum(I);
+    Q = wave_sum(Q);
+    U = wave_sum(U);
+    double(&out)[4][4] = sums[j & 1];
+    if (lane == 0) {
+      out[wave][0] = dm;
+      out[wave][1] = I;
+      out[wave][2] = Q;
+      out[wave][3] = U;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      double t[4];
+      for (int m = 0; m < 4; ++m)
+        t[m] = (out[0][m] + out[1][m]) + (out[2][m] + out[3][m]);
+      // a shell thinner than one step: no finite delta
+      store_ray(ph, sa, ipix, sa.step ? t[0] * sa.delta : 0., fd_carry, t[1], t[2], t[3]);
+    }
+  }
+}
+
 template <bool PACKED, bool CREG, bool HEAVY>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CREG ? 3 : 2))) void
 k_los_thread(Phys ph, Grids gr, ShellArgs sa) {
@@ -973,11 +1053,28 @@ int los_forward_impl(hamx_ctx *ctx, const hamx_los_desc *d, const hamx_fields *f
     ProfMark pm = prof_begin(ctx);
     if (fast) {
       const FastConst fc = make_fast(d, ph, sa.delta, pw1);
+      // Rays per workgroup of k_los_ray, 0 for k_los_fast.  A shell of up to
+      // 3072 rays (nside 16) leaves k_los_fast's two rays per wavefront with
+      // one or two wavefronts per SIMD, so its time is one ray's chain of
+      // steps (us, k_los_fast / k_los_ray: nside 4, 8, 16 with YMW16 167, 152,
+      // 231 / 38, 47, 96; nside 8, 16 with random grids 57, 58 / 22, 52;
+      // from nside 32 on its partly filled steps cost more: 88 / 123 over 600
+      // steps).  A CRE flux grid puts its work on the few rays near the plane
+      // and gains at every size (nside 16, 32, 64: 390, 496, 1446 / 233, 461,
+      // 912), two rays per workgroup from nside 32 on.
+      const int rays = npix <= 3072 ? 1 : creg ? 2 : 0;
+      const bool ray = rays > 0;
       const unsigned blocks =
-          static_cast<unsigned>((npix + 4 * kFastRays - 1) / (4 * kFastRays));
+          static_cast<unsigned>(ray ? (npix + rays - 1) / rays : (npix + 4 * kFastRays - 1) / (4 * kFastRays));
 #define HAMX_LAUNCH_FAST(G, P, M, C)                                                       \
-  hipLaunchKernelGGL((k_los_fast<G, P, M, C>), dim3(blocks), dim3(256), 0, ctx->stream, ph, fc, \
-                     gr, sa)
+  do {                                                                                     \
+    if (ray)                                                                               \
+      hipLaunchKernelGGL((k_los_ray<G, P, M, C>), dim3(blocks), dim3(256), 0, ctx->stream, \
+                         ph, fc, gr, sa, rays);                                            \
+    else                                                                                   \
+      hipLaunchKernelGGL((k_los_fast<G, P, M, C>), dim3(blocks), dim3(256), 0, ctx->stream, \
+                         ph, fc, gr, sa);                                                  \
+  } while (0)
 #define HAMX_LAUNCH_FAST_M(G, P)                                                           \
   do {                                                                                     \
     if (models == kLsaUnif)                                                                \
