@@ -177,6 +177,15 @@ int hamx_open(int device, hamx_ctx **out) {
     delete ctx;
     return HAMX_ERR_DEVICE;
   }
+  void *flag = nullptr;
+  if (hipHostMalloc(&flag, 64, hipHostMallocDefault) != hipSuccess) {
+    (void)hipGetLastError();
+    (void)hipStreamDestroy(ctx->stream);
+    delete ctx;
+    return HAMX_ERR_NOMEM;
+  }
+  ctx->nonfinite = static_cast<int *>(flag);
+  *ctx->nonfinite = 0;
   static_scratch_init(ctx);
   *out = ctx;
   return HAMX_OK;
@@ -195,8 +204,8 @@ void hamx_close(hamx_ctx *ctx) {
   for (int i = 0; i < hamx_ctx::kSlots; ++i)
     if (ctx->ws[i])
       (void)hipFree(ctx->ws[i]);
-  if (ctx->pinned)
-    (void)hipHostFree(ctx->pinned);
+  if (ctx->nonfinite)
+    (void)hipHostFree(ctx->nonfinite);
   if (ctx->stream)
     (void)hipStreamDestroy(ctx->stream);
   delete ctx;

@@ -36,9 +36,9 @@ struct hamx_ctx {
   // Host copy of small per-call tables uploaded asynchronously; it lives
   // until the next call so the copy never reads freed memory.
   std::vector<double> host_tab;
-  // Pinned host staging buffer for host-resident outputs.
-  void *pinned = nullptr;
-  size_t pinned_bytes = 0;
+  // Set to 1 by a march that meets a non-finite ray: pinned host memory that
+  // kernels write and the host reads after synchronising (hamx_open makes it).
+  int *nonfinite = nullptr;
 };
 
 namespace hamx {
@@ -95,7 +95,6 @@ enum Slot : int {
   kSlotCreTab,    // energy tables of the CRE grid emissivities
   kSlotSyncIO,    // hamx_sync_kernels staging (x, F, G)
   kSlotCreOut,    // hamx_cre_write_grid output staging
-  kSlotFlag,      // hamx_los_forward's non-finite output flag
   kSlotRndHalf,   // half spectra of the random-field generators
   kSlotRndPart,   // partial sums of the generators' variance
   kSlotCount

@@ -180,19 +180,34 @@ __device__ inline bool eval_sample(const Phys &ph, const Grids &gr,
 }
 
 // Shell-map epilogue: temp_convert of I/Q/U and the stores
-// (integrator.cc:99-115).
+// (integrator.cc:99-115).  A NaN or an infinity in an input grid or parameter
+// reaches a ray's values (the reference's debug build asserts isfinite on
+// B_par, B_per, te and the phase, integrator.cc:192,195,202,223; its release
+// build carries the NaN): the flag is raised here, where they are at hand (the
+// HEALPix interpolation of the accumulation skips a NaN as an undefined pixel).
 __device__ inline void store_ray(const Phys &ph, const ShellArgs &sa,
                                  uint64_t ipix, double dm, double fd, double I,
                                  double Q, double U) {
-  if (ph.do_dm)
+  bool ok = true;
+  if (ph.do_dm) {
     sa.t_dm[ipix] = dm;
-  if (ph.do_sync) {
-    sa.t_is[ipix] = I * ph.tc_em1 * ph.tc_em1 / ph.tc_den;
-    sa.t_qs[ipix] = Q * ph.tc_em1 * ph.tc_em1 / ph.tc_den;
-    sa.t_us[ipix] = U * ph.tc_em1 * ph.tc_em1 / ph.tc_den;
+    ok = ok && isfinite(dm);
   }
-  if (ph.do_fd || ph.do_sync)
+  if (ph.do_sync) {
+    I = I * ph.tc_em1 * ph.tc_em1 / ph.tc_den;
+    Q = Q * ph.tc_em1 * ph.tc_em1 / ph.tc_den;
+    U = U * ph.tc_em1 * ph.tc_em1 / ph.tc_den;
+    sa.t_is[ipix] = I;
+    sa.t_qs[ipix] = Q;
+    sa.t_us[ipix] = U;
+    ok = ok && isfinite(I) && isfinite(Q) && isfinite(U);
+  }
+  if (ph.do_fd || ph.do_sync) {
     sa.t_fd[ipix] = fd;
+    ok = ok && isfinite(fd);
+  }
+  if (!ok)
+    __hip_atomic_store(sa.nonfinite, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // Masked-out pixel (integrator.cc:63-70): every observable of the shell is
@@ -473,7 +488,9 @@ struct AccPairs {
 };
 
 // dst += src (same nside) or dst += interpolate(src, pixel centre of dst)
-// for up to 5 map pairs sharing the two resolutions (hamdis.h:698-721).
+// for up to 5 map pairs sharing the two resolutions (hamdis.h:698-721).  SET
+// (the first shell) starts dst from zero instead of reading it.
+template <bool SET>
 __global__ __launch_bounds__(256) void k_accumulate(AccPairs p, Healpix hd,
                                                     Healpix hsrc) {
   const uint64_t i = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -481,7 +498,7 @@ __global__ __launch_bounds__(256) void k_accumulate(AccPairs p, Healpix hd,
     return;
   if (hd.npix == hsrc.npix) {
     for (int m = 0; m < p.n; ++m)
-      p.dst[m][i] = p.dst[m][i] + p.src[m][i];
+      p.dst[m][i] = (SET ? 0. : p.dst[m][i]) + p.src[m][i];
     return;
   }
   double theta, phi;
@@ -500,7 +517,7 @@ __global__ __launch_bounds__(256) void k_accumulate(AccPairs p, Healpix hd,
       }
     }
     const double v = (wtot == 0.0) ? cgs::undef : res / wtot;
-    p.dst[m][i] = p.dst[m][i] + v;
+    p.dst[m][i] = (SET ? 0. : p.dst[m][i]) + v;
   }
 }
 
@@ -882,29 +899,6 @@ extern "C" int hamx_los_samples(const hamx_los_desc *d, uint64_t *samples) {
 }
 
 namespace hamx {
-namespace {
-// A NaN or an infinity in an input grid or parameter reaches the shell maps
-// (the reference's debug build asserts isfinite on B_par, B_per, te and the
-// phase, integrator.cc:192,195,202,223; its release build carries the NaN):
-// flag[0] becomes 1 when any of the given values is not finite.
-struct FiniteArgs {
-  const double *m[5];
-  uint64_t n[5];
-  int k;
-};
-
-__global__ __launch_bounds__(256) void k_nonfinite(FiniteArgs a, double *flag) {
-  const uint64_t stride = static_cast<uint64_t>(gridDim.x) * blockDim.x;
-  bool bad = false;
-  for (int j = 0; j < a.k; ++j)
-    for (uint64_t i = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-         i < a.n[j]; i += stride)
-      bad |= !isfinite(a.m[j][i]);
-  if (bad)
-    flag[0] = 1.;
-}
-} // namespace
-
 int los_forward_impl(hamx_ctx *ctx, const hamx_los_desc *d, const hamx_fields *fields,
                      hamx_maps *out, uint32_t flags, double *ckpt, double *shell_fd,
                      Arena *ar) {
@@ -998,18 +992,12 @@ int los_forward_impl(hamx_ctx *ctx, const hamx_los_desc *d, const hamx_fields *f
     HAMX_TRY(scratch_get(ctx, ar, kSlotMaskShell, tb, &q));
     mask_shell = static_cast<double *>(q);
   }
-  HAMX_TRY(scratch_get(ctx, ar, kSlotFlag, sizeof(double), &q));
-  double *nonfinite = static_cast<double *>(q);
-  HAMX_TRY(fill_f64(ctx, nonfinite, 1, 0.));
-  // every buffer is in place: zero the output maps
-  if (o_dm)
-    HAMX_TRY(fill_f64(ctx, o_dm, h_dm.npix, 0.));
-  if (o_is) {
-    HAMX_TRY(fill_f64(ctx, o_is, h_sync.npix, 0.));
-    HAMX_TRY(fill_f64(ctx, o_qs, h_sync.npix, 0.));
-    HAMX_TRY(fill_f64(ctx, o_us, h_sync.npix, 0.));
-  }
-  if (o_fd)
+  // every buffer is in place.  The first shell starts the output maps, all but
+  // the FD map of a pass that does not fill it (an nside 8 pass: six fills, a
+  // check of the shell maps, an accumulation and a copy of the flag fewer, 76 ->
+  // 32 us a call).
+  *ctx->nonfinite = 0;
+  if (o_fd && !d->do_fd)
     HAMX_TRY(fill_f64(ctx, o_fd, h_fd.npix, 0.));
 
   const int sched = d->schedule == HAMX_SCHED_THREAD ? HAMX_SCHED_THREAD : HAMX_SCHED_WAVE;
@@ -1040,14 +1028,27 @@ int los_forward_impl(hamx_ctx *ctx, const hamx_los_desc *d, const hamx_fields *f
     sa.t_is = t_is;
     sa.t_qs = t_qs;
     sa.t_us = t_us;
+    sa.nonfinite = ctx->nonfinite;
     const uint64_t npix = sa.hs.npix;
+    // the first shell's maps at an output's own nside are that output
+    if (s == 0) {
+      if (d->do_dm && h_dm.npix == npix)
+        sa.t_dm = o_dm;
+      if (d->do_sync && h_sync.npix == npix) {
+        sa.t_is = o_is;
+        sa.t_qs = o_qs;
+        sa.t_us = o_us;
+      }
+      if (d->do_fd && !shell_fd && h_fd.npix == npix)
+        sa.t_fd = o_fd;
+    }
     if (mask_piv) {
       hipLaunchKernelGGL(k_mask_dup, dim3(static_cast<unsigned>((npix + 255) / 256)), dim3(256),
                          0, ctx->stream, mask_shell, sa.hs, mask_piv, h_mask);
       HAMX_HIP(ctx, hipGetLastError());
       sa.mask = mask_shell;
     }
-    if (ckpt && d->do_fd) // FD map before shell s, for the adjoint
+    if (ckpt && d->do_fd && s > 0) // FD map before shell s, for the adjoint
       HAMX_HIP(ctx, hipMemcpyAsync(ckpt + s * h_fd.npix, o_fd, h_fd.npix * sizeof(double),
                                    hipMemcpyDeviceToDevice, ctx->stream));
     ProfMark pm = prof_begin(ctx);
@@ -1168,32 +1169,24 @@ int los_forward_impl(hamx_ctx *ctx, const hamx_los_desc *d, const hamx_fields *f
     prof_end(ctx, pm,
              fast ? "los_fast" : (sched == HAMX_SCHED_WAVE ? "los_wave" : "los_thread"), s,
              npix * sa.step);
-    {
-      // every ray's observables finite (checked here: the HEALPix
-      // interpolation of the accumulation skips a NaN as an undefined pixel)
-      FiniteArgs fa;
-      std::memset(&fa, 0, sizeof(fa));
-      for (const double *m : {static_cast<const double *>(sa.t_dm),
-                              static_cast<const double *>(sa.t_fd),
-                              static_cast<const double *>(sa.t_is),
-                              static_cast<const double *>(sa.t_qs),
-                              static_cast<const double *>(sa.t_us)})
-        if (m) {
-          fa.m[fa.k] = m;
-          fa.n[fa.k++] = npix;
-        }
-      const unsigned fb = static_cast<unsigned>(std::min<uint64_t>((npix + 255) / 256, 1024));
-      hipLaunchKernelGGL(k_nonfinite, dim3(fb), dim3(256), 0, ctx->stream, fa, nonfinite);
-      HAMX_HIP(ctx, hipGetLastError());
-    }
     // accumulate shell maps into the outputs (integrator.cc:122-132)
+    auto add = [](AccPairs &pairs, double *dst, const double *src) {
+      if (dst == src)
+        return; // written in place
+      pairs.dst[pairs.n] = dst;
+      pairs.src[pairs.n++] = src;
+    };
     auto acc = [&](AccPairs &pairs, const Healpix &hd) -> int {
       if (pairs.n == 0)
         return HAMX_OK;
       const unsigned blocks = static_cast<unsigned>((hd.npix + 255) / 256);
       ProfMark am = prof_begin(ctx);
-      hipLaunchKernelGGL(k_accumulate, dim3(blocks), dim3(256), 0, ctx->stream,
-                         pairs, hd, sa.hs);
+      if (s == 0)
+        hipLaunchKernelGGL(k_accumulate<true>, dim3(blocks), dim3(256), 0, ctx->stream, pairs,
+                           hd, sa.hs);
+      else
+        hipLaunchKernelGGL(k_accumulate<false>, dim3(blocks), dim3(256), 0, ctx->stream, pairs,
+                           hd, sa.hs);
       HAMX_HIP(ctx, hipGetLastError());
       prof_end(ctx, am, "accumulate", s, hd.npix);
       return HAMX_OK;
@@ -1201,26 +1194,22 @@ int los_forward_impl(hamx_ctx *ctx, const hamx_los_desc *d, const hamx_fields *f
     AccPairs pr;
     std::memset(&pr, 0, sizeof(pr));
     if (d->do_sync) {
-      pr.dst[0] = o_is; pr.src[0] = t_is;
-      pr.dst[1] = o_qs; pr.src[1] = t_qs;
-      pr.dst[2] = o_us; pr.src[2] = t_us;
-      pr.n = 3;
-      if (d->do_dm && d->nside_dm == d->nside_sync) {
-        pr.dst[pr.n] = o_dm; pr.src[pr.n] = t_dm; ++pr.n;
-      }
-      if (d->do_fd && d->nside_fd == d->nside_sync) {
-        pr.dst[pr.n] = o_fd; pr.src[pr.n] = sa.t_fd; ++pr.n;
-      }
+      add(pr, o_is, sa.t_is);
+      add(pr, o_qs, sa.t_qs);
+      add(pr, o_us, sa.t_us);
+      if (d->do_dm && d->nside_dm == d->nside_sync)
+        add(pr, o_dm, sa.t_dm);
+      if (d->do_fd && d->nside_fd == d->nside_sync)
+        add(pr, o_fd, sa.t_fd);
       HAMX_TRY(acc(pr, h_sync));
     }
     if (d->do_dm && !(d->do_sync && d->nside_dm == d->nside_sync)) {
       AccPairs p2;
       std::memset(&p2, 0, sizeof(p2));
-      p2.dst[0] = o_dm; p2.src[0] = t_dm; p2.n = 1;
+      add(p2, o_dm, sa.t_dm);
       if (d->do_fd && d->nside_fd == d->nside_dm &&
-          !(d->do_sync && d->nside_fd == d->nside_sync)) {
-        p2.dst[1] = o_fd; p2.src[1] = sa.t_fd; p2.n = 2;
-      }
+          !(d->do_sync && d->nside_fd == d->nside_sync))
+        add(p2, o_fd, sa.t_fd);
       HAMX_TRY(acc(p2, h_dm));
     }
     const bool fd_done = (d->do_sync && d->nside_fd == d->nside_sync) ||
@@ -1228,15 +1217,10 @@ int los_forward_impl(hamx_ctx *ctx, const hamx_los_desc *d, const hamx_fields *f
     if (d->do_fd && !fd_done) {
       AccPairs p3;
       std::memset(&p3, 0, sizeof(p3));
-      p3.dst[0] = o_fd; p3.src[0] = sa.t_fd; p3.n = 1;
+      add(p3, o_fd, sa.t_fd);
       HAMX_TRY(acc(p3, h_fd));
     }
   }
-
-  // ---- the shells' non-finite flag
-  double host_flag = 0.;
-  HAMX_HIP(ctx, hipMemcpyAsync(&host_flag, nonfinite, sizeof(double), hipMemcpyDeviceToHost,
-                               ctx->stream));
 
   // ---- results to the caller
   auto copy_out = [&](double *user, const double *dev, const Healpix &h) -> int {
@@ -1256,7 +1240,7 @@ int los_forward_impl(hamx_ctx *ctx, const hamx_los_desc *d, const hamx_fields *f
   if (d->do_fd || d->do_sync)
     HAMX_TRY(copy_out(out->fd, o_fd, h_fd));
   HAMX_HIP(ctx, hipStreamSynchronize(ctx->stream));
-  if (host_flag != 0.)
+  if (*const_cast<volatile int *>(ctx->nonfinite) != 0) // raised by the marches
     return set_err(ctx, HAMX_ERR_ARG,
                    "non-finite values on the lines of sight: an input grid or parameter "
                    "holds a NaN or an infinity");
@@ -1276,16 +1260,15 @@ extern "C" int hamx_los_forward(hamx_ctx *ctx, const hamx_los_desc *d,
 namespace hamx {
 namespace {
 
-// The scratch of hamx_los_forward_static: the five shell maps, the mask at
-// the shell's nside (for shells up to nside HAMX_STATIC_MAX_NSIDE) and the
-// non-finite output flag.  Every GPU the library runs on holds its own copy
-// until the process ends.  In host code `scratch` names a host-side stand-in,
-// not device memory: kernels and copies take the device address looked up by
-// static_scratch_init.
+// The scratch of hamx_los_forward_static: the five shell maps and the mask at
+// the shell's nside (for shells up to nside HAMX_STATIC_MAX_NSIDE).  Every GPU
+// the library runs on holds its own copy until the process ends.  In host code
+// `scratch` names a host-side stand-in, not device memory: kernels and copies
+// take the device address looked up by static_scratch_init.
 static_assert(HAMX_STATIC_SCRATCH_BYTES >=
                   6 * (12ull * HAMX_STATIC_MAX_NSIDE * HAMX_STATIC_MAX_NSIDE * sizeof(double) +
                        256) + 512,
-              "static scratch below six maps at HAMX_STATIC_MAX_NSIDE and the flag");
+              "static scratch below six maps at HAMX_STATIC_MAX_NSIDE");
 static __device__ __align__(256) double scratch[HAMX_STATIC_SCRATCH_BYTES / sizeof(double)];
 
 constexpr int kMaxDevices = 64;

@@ -76,6 +76,7 @@ struct ShellArgs {
   const double *fd_map; // accumulated FD of inner shells (NULL: zero cache)
   Healpix hfd;
   double *t_dm, *t_fd, *t_is, *t_qs, *t_us; // shell maps, nside_s
+  int *nonfinite; // set to 1 where a ray's values are not finite
 };
 
 struct RayGeo {
