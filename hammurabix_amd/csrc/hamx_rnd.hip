@@ -207,6 +207,34 @@ __device__ inline uint64_t sym_index(const BoxArgs &a, uint64_t idx) {
   return is * a.ny * a.nz + js * a.nz + ls;
 }
 
+// A spectrum's three bands (brnd_es.cc:34-49, brnd_mhd.cc:211-262) as amplitudes
+// at x = |k|^2: low x below k1, mid between k1 and k0, high above k0.  With
+// k1 > k0 the low and the high band overlap and their powers add.
+struct KBands {
+  KEdge k0, k1;
+  double low;
+  KPower mid, high;
+  // bits of the bands that x lies in: 1 low, 2 mid, 4 high
+  __device__ int of(double x) const {
+    return (x <= k1.lt ? 1 : 0) | (x > k0.le ? 4 : (x > k1.le && x <= k0.lt) ? 2 : 0);
+  }
+  __device__ double amp(int bands, double x, double lnx, const KPower &hi) const {
+    const double lo = bands & 1 ? low * x : 0.;
+    const double v = bands & 6 ? (bands & 4 ? hi : mid).at(lnx) : 0.;
+    return lo != 0. && v != 0. ? sqrt(lo * lo + v * v) : lo + v;
+  }
+};
+
+static KBands k_bands(double k0, double k1, double a1) {
+  KBands b;
+  b.k0 = k_edge(k0);
+  b.k1 = k_edge(k1);
+  b.low = std::sqrt(std::pow(k0 / k1, a1)) / (k1 * k1 * k1);
+  b.mid = KPower{std::pow(k0, 0.5 * a1), -0.25 * (a1 + 2.)};
+  b.high = KPower{0., 0.};
+  return b;
+}
+
 // ---------------------------------------------------- variance (two stage) --
 // toolkit::variance over the first n doubles (toolkit.h:48-78): mean, then
 // the mean squared deviation.  Stage 1: per-block partial sums; stage 2: one
@@ -279,11 +307,7 @@ struct EsArgs {
   BoxArgs b;
   Vec3 obs;
   double rms, rho, r0, z0;
-  // Brnd_es::spectrum (brnd_es.cc:34-49) as amplitudes of a mode's components:
-  // low x below k1, mid between k1 and k0, high above k0
-  KEdge k0, k1;
-  double low;
-  KPower mid, high;
+  KBands bands; // of a mode's components (es_sigma)
   int breg_model;
   int jf12; // Brnd_jf12: its energy profile and literal constants
   double jp[13];
@@ -294,26 +318,20 @@ struct EsArgs {
 };
 
 // The standard deviation of the components of a mode at x = |k|^2
-// (brnd_es.cc:34-49,127-133): the square root of the band's power
+// (brnd_es.cc:34-49,127-133): the square root of
 //   third rms^2 dk3 / (4 pi k^2) {(k0/k1)^a1 (k/k1)^6, (k/k0)^-a1, (k/k0)^-a0}
-// with the constants folded on the host (es_bands).  With k1 > k0 the low and
-// the high band overlap and their powers add.
+// with the constants folded on the host.
 __device__ inline double es_sigma(const EsArgs &a, double x) {
-  const double lo = x <= a.k1.lt ? a.low * x : 0.;
-  const bool hi = x > a.k0.le, mid = x > a.k1.le && x <= a.k0.lt;
-  double v = 0.;
-  if (hi || mid)
-    v = (hi ? a.high : a.mid).at(log_pos(x));
-  return lo != 0. && v != 0. ? sqrt(lo * lo + v * v) : lo + v;
+  const int in = a.bands.of(x);
+  return a.bands.amp(in, x, in & 6 ? log_pos(x) : 0., a.bands.high);
 }
 
 static void es_bands(EsArgs &a, const hamx_es_desc *d) {
-  const double p = a.third * d->rms * d->rms * a.b.dk3 / (4. * cgs::pi);
-  a.k0 = k_edge(d->k0);
-  a.k1 = k_edge(d->k1);
-  a.low = std::sqrt(p * std::pow(d->k0 / d->k1, d->a1)) / (d->k1 * d->k1 * d->k1);
-  a.mid = KPower{std::sqrt(p) * std::pow(d->k0, 0.5 * d->a1), -0.25 * (d->a1 + 2.)};
-  a.high = KPower{std::sqrt(p) * std::pow(d->k0, 0.5 * d->a0), -0.25 * (d->a0 + 2.)};
+  const double p = std::sqrt(a.third * d->rms * d->rms * a.b.dk3 / (4. * cgs::pi));
+  a.bands = k_bands(d->k0, d->k1, d->a1);
+  a.bands.low *= p;
+  a.bands.mid.coef *= p;
+  a.bands.high = KPower{p * std::pow(d->k0, 0.5 * d->a0), -0.25 * (d->a0 + 2.)};
 }
 
 // Brnd_jf12::spatial_profile (brnd_jf12.cc:54-114): the squared disk (JF12
@@ -682,45 +700,38 @@ __global__ __launch_bounds__(256) void k_dft_rescale(const double2 *tk, double *
 // by one backward transform per complex array; no energy-profile rescale.
 struct MhdArgs {
   BoxArgs b;
-  double pa0, pf0, ps0, k0, k1, aa0, af0, as0, a1, beta, ma;
+  // amplitudes sqrt(2 P dk3) of the three modes, spectrum_a / _f / _s
+  // (brnd_mhd.cc:211-262): the shared low and mid bands times ca, cf, cs, and
+  // each mode's own power above k0
+  KBands bands;
+  double ca, cf, cs;
+  KPower ha, hf, hs;
+  int same_as;   // the slow mode's power is the Alfven mode's
+  double beta;
+  double half_ma; // ma^(-4/3) / 2 (the literal exponents of brnd_mhd.cc)
 };
 
-// Brnd_mhd::spectrum_a / _f / _s (brnd_mhd.cc:211-262): one form, the mode
-// choosing its index a0 and norm p0.
-__device__ inline double mhd_spectrum(const MhdArgs &a, double k, double a0, double p0) {
-  const double unit = 0.25 / (cgs::pi * k * k);
-  const double band1 = static_cast<double>(k < a.k1);
-  const double band2 = static_cast<double>(k > a.k1) * static_cast<double>(k < a.k0);
-  const double band3 = static_cast<double>(k > a.k0);
-  const double P = band1 * pow(a.k0 / a.k1, a.a1) * pow(k / a.k1, 6.0) +
-                   band2 / pow(k / a.k0, a.a1) + band3 / pow(k / a.k0, a0);
-  return P * p0 * unit;
-}
-
-// dynamo, h_s, h_f, F_a = F_s (bfield.h:388-412, brnd_mhd.cc:181-209)
+// dynamo, h_s, h_f (bfield.h:388-412).  As written: h_f jumps to 0 at c = 0
+// exactly, and 1 - sq + beta / 2 cancels to rounding for small c, so c and
+// these keep the operations (and the rounding) of the reference.
 __device__ inline double mhd_dynamo(double beta, double c) {
   return 1 + 0.25 * beta * beta + beta * (1. - 2. * c * c);
 }
-__device__ inline double mhd_h_s(double beta, double c) {
-  const double sq = sqrt(mhd_dynamo(beta, c));
+__device__ inline double mhd_h_s(double beta, double sq, double c) {
   const double dpp = 1 + sq + 0.5 * beta;
   const double dmm = 1 - sq - 0.5 * beta;
   const double dmp = 1 - sq + 0.5 * beta;
   const double den = 1 / (dmp * (c * c + dpp * dpp * (1 - c * c) / (dmm * dmm)));
   return isfinite(den) ? 2. * c * c * den * static_cast<double>(den > 0) : 0.;
 }
-__device__ inline double mhd_h_f(double beta, double c) {
+__device__ inline double mhd_h_f(double beta, double sq, double c) {
   if (c == 0)
     return 0;
-  const double sq = sqrt(mhd_dynamo(beta, c));
   const double dpp = 1 + sq + 0.5 * beta;
   const double dpm = 1 + sq - 0.5 * beta;
   const double dmp = 1 - sq + 0.5 * beta;
   const double den = 1 / (dpp * (c * c + dmp * dmp * (1 - c * c) / (dpm * dpm)));
   return isfinite(den) ? 2. * c * c * den : 0.;
-}
-__device__ inline double mhd_aniso(double ma, double c) {
-  return exp(-1. * pow(ma, -1.33333333) * fabs(c) / pow(1 - c * c, 0.33333333));
 }
 
 // Hamvec::versor and crossprod (hamvec.h:176-205)
@@ -737,19 +748,6 @@ __device__ inline Vec3 versor3(const Vec3 &v) {
 __device__ inline Vec3 cross3(const Vec3 &a, const Vec3 &b) {
   return Vec3{a.y * b.z - a.z * b.y, a.z * b.x - a.x * b.z, a.x * b.y - a.y * b.x};
 }
-// Brnd_mhd::e_plus / e_minus (brnd_mhd.cc:169-179): normalised unless
-// their squared length is below 1e-12
-__device__ inline Vec3 unit_or_small(const Vec3 &t) {
-  double l2 = 0.;
-  l2 += t.x * t.x;
-  l2 += t.y * t.y;
-  l2 += t.z * t.z;
-  if (l2 < 1e-12)
-    return t;
-  const double l = sqrt(l2);
-  return Vec3{t.x / l, t.y / l, t.z / l};
-}
-
 // The regular field at the observer (breg->read_field(observer)).
 __global__ void k_mhd_bobs(EsArgs a, double *out) {
   if (blockIdx.x != 0 || threadIdx.x != 0)
@@ -774,43 +772,73 @@ __global__ void k_mhd_bobs(EsArgs a, double *out) {
 // fast/slow power share of the modes along the field.
 constexpr uint32_t kMhdGaussStream = 3, kMhdShareStream = 4;
 
-// The field amplitude of mode (i, j, l), flat index idx (brnd_mhd.cc:54-137);
-// bh is the regular field's versor at the observer.
-__device__ inline Vec3 mhd_mode(const MhdArgs &a, uint64_t seed, const Vec3 &bh, uint64_t idx,
-                                uint64_t i, uint64_t j, uint64_t l) {
-  if (idx == 0)
-    return Vec3{0., 0., 0.};
-  const Vec3 k{wavenum(i, a.b.nx, a.b.lx), wavenum(j, a.b.ny, a.b.ly),
-               wavenum(l, a.b.nz, a.b.lz)};
-  const double ks = length0(k);
+// A mode's spectrum (brnd_mhd.cc:54-137): the amplitudes of the Alfven, fast
+// and slow modes without h_f and h_s.  It varies smoothly with k, unlike
+// those, so a mode and its mirror share it.
+struct MhdPower {
+  double a, f, s;
+};
+
+// x = |k|^2, bands = a.bands.of(x), c the cosine to the regular field.
+__device__ inline MhdPower mhd_power(const MhdArgs &a, double x, int bands, double c) {
+  const double lnx = bands & 6 ? log_pos(x) : 0.;
+  // sqrt of exp(-ma^(-4/3) |c| / (1 - c^2)^(1/3))
+  const double third = exp_fast(-0.33333333 * log_pos(fmax(1. - c * c, 1e-300)));
+  const double an = exp_fast(fmax(-a.half_ma * fabs(c) * third, -745.));
+  const double pa = a.bands.amp(bands, x, lnx, a.ha);
+  return MhdPower{a.ca * pa * an, a.cf * a.bands.amp(bands, x, lnx, a.hf),
+                  a.cs * (a.same_as ? pa : a.bands.amp(bands, x, lnx, a.hs)) * an};
+}
+
+// A mode's versors e_plus and e_minus (brnd_mhd.cc:169-179) and the square
+// roots of h_f and h_s; `generic` false for modes (nearly) along the regular
+// field bh: e_plus is normalised unless its squared length is below 1e-12, and
+// then fails the generic branch's dot(e_plus, e_plus) > 1e-6.
+struct MhdShape {
+  Vec3 ep, em;
+  double c, hf, hs;
+  bool generic;
+};
+
+__device__ inline MhdShape mhd_shape(const MhdArgs &a, const Vec3 &bh, const Vec3 &k) {
+  MhdShape m{};
   const Vec3 kh = versor3(k);
   const Vec3 kxb = cross3(kh, bh);
-  Vec3 ep = unit_or_small(kxb);
-  Vec3 em = unit_or_small(cross3(kxb, kh));
-  const double dk3 = a.b.dk3;
+  const double l2 = kxb.x * kxb.x + kxb.y * kxb.y + kxb.z * kxb.z;
+  m.generic = !(l2 < 1e-12);
+  m.c = m.generic ? dot0(bh, kh) : 1.;
+  const double sq = sqrt(mhd_dynamo(a.beta, m.c));
+  m.hf = sqrt_pos(mhd_h_f(a.beta, sq, m.c));
+  if (m.generic) {
+    const double il = rsqrt_f64(l2);
+    m.ep = Vec3{kxb.x * il, kxb.y * il, kxb.z * il};
+    m.em = cross3(m.ep, kh);
+    m.hs = sqrt_pos(mhd_h_s(a.beta, sq, m.c));
+  }
+  return m;
+}
+
+// The field of mode (i, j, l), flat index idx != 0, with wave vector k.
+__device__ inline Vec3 mhd_field(uint64_t seed, const MhdShape &m, const MhdPower &p,
+                                 const Vec3 &k, double x, uint64_t idx, bool pole) {
   double g0, g1, g2, g3;
   gauss_pair(seed, kMhdGaussStream, 2 * idx, g0, g1);
-  if (dot0(ep, ep) > 1e-6) {
-    const double ang = dot0(bh, kh);
-    const double Pa = mhd_spectrum(a, ks, a.aa0, a.pa0) * mhd_aniso(a.ma, ang) * dk3;
-    const double Pf = mhd_spectrum(a, ks, a.af0, a.pf0) * mhd_h_f(a.beta, ang) * dk3;
-    const double Ps = mhd_spectrum(a, ks, a.as0, a.ps0) * mhd_aniso(a.ma, ang) *
-                      mhd_h_s(a.beta, ang) * dk3;
+  if (m.generic) {
     gauss_pair(seed, kMhdGaussStream, 2 * idx + 1, g2, g3);
-    const double Ap = g0 * sqrt(2. * Pa);
-    const double Am = g1 * sqrt(2. * Pf) + g2 * sqrt(2. * Ps);
-    return Vec3{ep.x * Ap + em.x * Am, ep.y * Ap + em.y * Am, ep.z * Ap + em.z * Am};
+    const double Ap = g0 * p.a, Am = g1 * (p.f * m.hf) + g2 * (p.s * m.hs);
+    return Vec3{m.ep.x * Ap + m.em.x * Am, m.ep.y * Ap + m.em.y * Am,
+                m.ep.z * Ap + m.em.z * Am};
   }
-  const double Pf = mhd_spectrum(a, ks, a.af0, a.pf0) * mhd_h_f(a.beta, 1) * dk3;
-  if (i == 0 && j == 0) {
+  Vec3 ep{0., 0., 0.}, em{0., 0., 0.}; // along the field: below 1e-6 before
+  if (pole) {                          // i == 0 and j == 0
     ep.x = k.x;
     em.y = k.y;
   } else {
-    const double kp = sqrt(k.x * k.x + k.y * k.y);
+    const double ks = sqrt(x), kp = sqrt(k.x * k.x + k.y * k.y);
     ep = Vec3{k.x * k.z / (ks * kp), k.y * k.z / (ks * kp), -kp / ks};
     em = Vec3{-k.y / kp, k.x / kp, 0.};
   }
-  const double Af = g0 * sqrt(2. * Pf);
+  const double Af = g0 * (p.f * m.hf);
   const double share = philox_uniform(seed, kMhdShareStream, idx);
   return Vec3{ep.x * Af * share + em.x * Af * (1. - share),
               ep.y * Af * share + em.y * Af * (1. - share),
@@ -825,7 +853,14 @@ __global__ __launch_bounds__(256) void k_mhd_draw(double2 *c0, double2 *c1, MhdA
        idx < a.b.n; idx += stride) {
     uint64_t i, j, l;
     box_ijl(a.b, idx, i, j, l);
-    const Vec3 bk = mhd_mode(a, seed, bh, idx, i, j, l);
+    const Vec3 k{wavenum(i, a.b.nx, a.b.lx), wavenum(j, a.b.ny, a.b.ly),
+                 wavenum(l, a.b.nz, a.b.lz)};
+    const double x = k.x * k.x + k.y * k.y + k.z * k.z;
+    Vec3 bk{0., 0., 0.};
+    if (idx != 0) {
+      const MhdShape m = mhd_shape(a, bh, k);
+      bk = mhd_field(seed, m, mhd_power(a, x, a.bands.of(x), m.c), k, x, idx, i == 0 && j == 0);
+    }
     c0[idx] = double2{bk.x, bk.y};
     c1[idx] = double2{bk.y, bk.z};
   }
@@ -1043,17 +1078,18 @@ int brnd_mhd(hamx_ctx *ctx, const hamx_mhd_desc *d, uint64_t seed, double *bx, d
   MhdArgs a;
   std::memset(&a, 0, sizeof(a));
   a.b = box_args(d->box);
-  a.pa0 = d->pa0;
-  a.pf0 = d->pf0;
-  a.ps0 = d->ps0;
-  a.k0 = d->k0;
-  a.k1 = d->k1;
-  a.aa0 = d->aa0;
-  a.af0 = d->af0;
-  a.as0 = d->as0;
-  a.a1 = d->a1;
+  const double c = 2. * a.b.dk3 / (4. * cgs::pi);
+  a.bands = k_bands(d->k0, d->k1, d->a1);
+  a.ca = std::sqrt(c * d->pa0);
+  a.cf = std::sqrt(c * d->pf0);
+  a.cs = std::sqrt(c * d->ps0);
+  auto above = [&](double e) { return KPower{std::pow(d->k0, 0.5 * e), -0.25 * (e + 2.)}; };
+  a.ha = above(d->aa0);
+  a.hf = above(d->af0);
+  a.hs = above(d->as0);
+  a.same_as = d->aa0 == d->as0;
   a.beta = d->beta;
-  a.ma = d->ma;
+  a.half_ma = 0.5 * std::pow(d->ma, -1.33333333);
   const uint64_t n = a.b.n;
   HalfPlan hp;
   int rc;

@@ -28,7 +28,7 @@
 // at a time over two complex arrays), 72 instead of 280 for mhd, 72 instead of
 // 144 for te.  Measured per realisation, whole-array steps -> these (with the
 // engine and table work below): es 256x256x64 726 -> 304 us, es 512x512x128
-// 7.05 -> 2.24 ms, te 800x800x160 7.90 -> 2.71 ms, mhd 135x121x98 344 -> 197 us.  Distance from a 64-bit
+// 7.05 -> 2.24 ms, te 800x800x160 7.90 -> 2.71 ms, mhd 135x121x98 344 -> 122 us.  Distance from a 64-bit
 // reference 1.0e-15 -> 1.2e-15 to 3e-15: the rounding errors of a vertex and
 // its mirror now coincide instead of averaging in the extraction.
 //
@@ -396,7 +396,11 @@ __global__ __launch_bounds__(NT) void k_es_gs_x(HalfArrays H, EsArgs a, HalfArgs
 }
 
 // Brnd_mhd's modes, their even part (the only part the extraction keeps) and
-// x(+).
+// x(+).  k and -k share the spectrum, so a pair evaluates it once, except where
+// an index is half its axis length (the wave number keeps its sign at the
+// mirror) or the two |k|, which may differ in rounding, lie in different bands.  Bound by FP64 instructions: mhd
+// 135x121x98 149 -> 62 us with that, the spectra as powers of |k|^2 and no
+// library pow.
 template <uint32_t TILE, uint32_t NT, int MODE>
 __global__ __launch_bounds__(NT) void k_mhd_x(HalfArrays H, MhdArgs a, uint64_t seed,
                                               const double *__restrict__ bobs, HalfArgs h,
@@ -412,16 +416,36 @@ __global__ __launch_bounds__(NT) void k_mhd_x(HalfArrays H, MhdArgs a, uint64_t 
   const uint32_t col = col0 + c;
   const bool on = col < h.ncol;
   const uint32_t j = col / h.nh, l = col - j * h.nh;
+  const uint32_t js = mirror_of(j, h.ny), ls = mirror_of(l, h.nz);
+  Vec3 k{0., wavenum(j, h.ny, a.b.ly), wavenum(l, h.nz, a.b.lz)};
+  Vec3 ks{0., wavenum(js, h.ny, a.b.ly), wavenum(ls, h.nz, a.b.lz)};
+  const bool edge = 2 * j == h.ny || 2 * l == h.nz;
+  double *kx = reinterpret_cast<double *>(lds) +
+               2 * (L.len * P + (fft_lds_tw<TILE, MODE>() ? L.len : 0));
+  for (uint32_t t = threadIdx.x; t < n; t += NT)
+    kx[t] = wavenum(t, n, a.b.lx);
+  __syncthreads();
 #pragma unroll 1
   for (uint32_t t = t0; t < n; t += dt) {
+    const uint32_t ts = mirror_of(t, n);
+    const uint64_t idx = (static_cast<uint64_t>(t) * h.ny + j) * h.nz + l;
+    const uint64_t sym = (static_cast<uint64_t>(ts) * h.ny + js) * h.nz + ls;
     Vec3 f{0., 0., 0.};
-#pragma unroll 1
-    for (int m = 0; on && m < 2; ++m) {
-      const uint32_t mi = m ? mirror_of(t, n) : t, mj = m ? mirror_of(j, h.ny) : j;
-      const uint32_t ml = m ? mirror_of(l, h.nz) : l;
-      const uint64_t idx = (static_cast<uint64_t>(mi) * h.ny + mj) * h.nz + ml;
-      const Vec3 b = mhd_mode(a, seed, bh, idx, mi, mj, ml);
-      f = Vec3{f.x + b.x, f.y + b.y, f.z + b.z};
+    if (on && idx != 0) {
+      k.x = kx[t];
+      ks.x = kx[ts];
+      const double x = k.x * k.x + k.y * k.y + k.z * k.z;
+      const double xs = ks.x * ks.x + ks.y * ks.y + ks.z * ks.z;
+      const int in = a.bands.of(x), ins = a.bands.of(xs);
+      MhdShape m = mhd_shape(a, bh, k);
+      const bool generic = m.generic;
+      MhdPower p = mhd_power(a, x, in, m.c);
+      f = mhd_field(seed, m, p, k, x, idx, t == 0 && j == 0);
+      m = mhd_shape(a, bh, ks);
+      if (edge || 2 * t == n || in != ins || !generic || !m.generic)
+        p = mhd_power(a, xs, ins, m.c);
+      const Vec3 s = mhd_field(seed, m, p, ks, xs, sym, t == 0 && j == 0);
+      f = Vec3{f.x + s.x, f.y + s.y, f.z + s.z};
     }
     lds[t * P + c] = make_double2(0.5 * f.x, 0.5 * f.y);
     lds[t * P + C + c] = make_double2(0.5 * f.z, 0.);
@@ -717,8 +741,8 @@ inline int half_mhd_x(hamx_ctx *ctx, const HalfPlan &p, const HalfArrays &H, con
   with_tile(tile, p.lx.mode, [&](auto T, auto NT, auto M) {
     hipLaunchKernelGGL((k_mhd_x<decltype(T)::value, decltype(NT)::value, decltype(M)::value>),
                        dim3(xcd_grid((h.ncol + (1u << cs) - 1) >> cs)), dim3(decltype(NT)::value),
-                       fft_lds_bytes(p.lx, 2u << cs, tile), ctx->stream, H, a, seed, bobs, h,
-                       p.lx, cs);
+                       fft_lds_bytes(p.lx, 2u << cs, tile) + p.lx.n * sizeof(double),
+                       ctx->stream, H, a, seed, bobs, h, p.lx, cs);
   });
   HAMX_HIP(ctx, hipGetLastError());
   return HAMX_OK;
