@@ -256,17 +256,15 @@ struct S32 {
   int cx, cy, cz; // the cell's lower corner
 };
 
-__device__ inline void lerp_plane_f4(const float4 *__restrict__ f, uint64_t i0, uint64_t sy,
-                                     float zd, float yd, float4 &w) {
+// The four corners c of a cell's lower or upper x plane at (yd, zd).
+__device__ inline void lerp_plane_f4(const float4 *c, float zd, float yd, float4 &w) {
   // FP32 sample arithmetic: a * b + c may fuse (more accurate, fewer instructions)
   #pragma clang fp contract(fast)
-  const float4 a0 = f[i0], a1 = f[i0 + 1];
-  const float4 b0 = f[i0 + sy], b1 = f[i0 + sy + 1];
   const float z1 = 1.f - zd, y1 = 1.f - yd;
-  w.x = (a0.x * z1 + a1.x * zd) * y1 + (b0.x * z1 + b1.x * zd) * yd;
-  w.y = (a0.y * z1 + a1.y * zd) * y1 + (b0.y * z1 + b1.y * zd) * yd;
-  w.z = (a0.z * z1 + a1.z * zd) * y1 + (b0.z * z1 + b1.z * zd) * yd;
-  w.w = (a0.w * z1 + a1.w * zd) * y1 + (b0.w * z1 + b1.w * zd) * yd;
+  w.x = (c[0].x * z1 + c[1].x * zd) * y1 + (c[2].x * z1 + c[3].x * zd) * yd;
+  w.y = (c[0].y * z1 + c[1].y * zd) * y1 + (c[2].y * z1 + c[3].y * zd) * yd;
+  w.z = (c[0].z * z1 + c[1].z * zd) * y1 + (c[2].z * z1 + c[3].z * zd) * yd;
+  w.w = (c[0].w * z1 + c[1].w * zd) * y1 + (c[2].w * z1 + c[3].w * zd) * yd;
 }
 
 // sin and cos of an FP32 angle |r| <= pi/4: the Taylor series to the terms
@@ -376,6 +374,25 @@ __device__ inline bool eval_f32(const BInst &in, const BShell &sh, const RayGeo 
   // in FP64 with the FP64 direction, the LSA part as b0 (FP64) times its
   // unit vector, and te as n0 (FP64) plus the FP32 grid value
   double bpar = 0., te_d = 0.;
+  // The cell's eight corners are loaded ahead of the LSA field, whose hundred
+  // instructions cover the loads; lanes outside the grid load cell 0.
+  o.cell_ok = false;
+  Cell cell;
+  float4 cn[8];
+  bool any_cell = false;
+  if (GRIDS) {
+    o.cell_ok = grid_cell_scaled(in, pos, cell, o.cx, o.cy, o.cz);
+    any_cell = __any(o.cell_ok);
+    if (any_cell) {
+      if (!o.cell_ok)
+        cell.idx = 0;
+      const float4 *g = static_cast<const float4 *>(in.packed) + cell.idx;
+      const uint64_t sy = in.geo.nz, sx = in.geo.ny * in.geo.nz;
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        cn[i] = g[(i >> 2) * sx + ((i >> 1) & 1) * sy + (i & 1)];
+    }
+  }
   // WMAP-LSA window (breg_lsa.cc:9-26)
   o.lsa_in = !(rr2 > (400. * cgs::kpc * cgs::kpc) || rr2 < (9. * cgs::kpc * cgs::kpc));
   if (o.lsa_in) {
@@ -411,20 +428,15 @@ __device__ inline bool eval_f32(const BInst &in, const BShell &sh, const RayGeo 
   o.te_in = geo.te_in;
   if (o.te_in)
     te_d = c.n0d;
-  o.cell_ok = false;
-  if (GRIDS) {
-    Cell cell;
-    if (grid_cell_scaled(in, pos, cell, o.cx, o.cy, o.cz)) {
-      o.cell_ok = true;
-      const float4 *g = static_cast<const float4 *>(in.packed);
-      const uint64_t sy = in.geo.nz, sx = in.geo.ny * in.geo.nz;
-      float4 w1, w2;
-      o.idx = cell.idx;
-      o.zd = static_cast<float>(cell.zd);
-      o.yd = static_cast<float>(cell.yd);
-      o.xd = static_cast<float>(cell.xd);
-      lerp_plane_f4(g, cell.idx, sy, o.zd, o.yd, w1);
-      lerp_plane_f4(g, cell.idx + sx, sy, o.zd, o.yd, w2);
+  if (GRIDS && any_cell) {
+    o.idx = cell.idx;
+    o.zd = static_cast<float>(cell.zd);
+    o.yd = static_cast<float>(cell.yd);
+    o.xd = static_cast<float>(cell.xd);
+    float4 w1, w2;
+    lerp_plane_f4(cn, o.zd, o.yd, w1);
+    lerp_plane_f4(cn + 4, o.zd, o.yd, w2);
+    if (o.cell_ok) {
       const float x1 = 1.f - o.xd;
       const float gx = w1.x * x1 + w2.x * o.xd;
       const float gy = w1.y * x1 + w2.y * o.xd;
@@ -749,6 +761,15 @@ __device__ void adj_ray_f64(const BInst &in, int s, uint64_t ipix, int lane, voi
 // adding them to the gradient grid when the ray leaves the cell (a straight
 // ray meets each cell in one run of samples).  No cross-lane reduction,
 // LDS atomic or wavefront barrier is left in the sample loop.
+//
+// Bound by VALU issue (conversions and transcendentals at a quarter rate
+// included): about 450 instructions a step, 100 of them for the cells' sums.
+// Without the grid's atomics the sweep takes the same time, without the
+// flush list's merge 4 % less; three wavefronts a SIMD (a cache of 384 slots,
+// 28 registers spilled) are no faster than two.  Six instances at nside
+// 64 .. 256, 256x256x64 grids: 22.6 -> 20.6 ms by corners ordered along the
+// ray, the cell's loads ahead of the field model and selects in place of
+// short branches.
 
 
 // Per-wavefront LDS merge of the lanes' gradient flushes.  The 64 rays of a
@@ -867,93 +888,126 @@ __device__ inline void flush_list_drain(const VtxCache &c, float *__restrict__ g
   wave_lds_sync(); // read before the list is written again
 }
 
-// One vertex sum of a lane that takes part in a list step: to the list at
-// `pos`, or straight to the grid when there is no cache (vertex indices
-// beyond 32 bits).
-__device__ inline void list_put(const VtxCache &c, float *__restrict__ g, uint32_t pos,
-                                uint64_t v, float4 a) {
-  if (c.tag) {
-    c.ltag[pos] = static_cast<uint32_t>(v);
-    c.lval[pos] = a;
-  } else {
-    grid_add4(g, v, a);
-  }
-}
-
-// Called by the whole wavefront: the lanes with `part` each get `per` flush
-// list entries; returns the lane's first entry (meaningful where part).
-// The list is drained first when the entries would not fit.
-__device__ inline uint32_t list_reserve(const VtxCache &c, float *__restrict__ g, bool part,
-                                        uint32_t per, uint32_t &nlist, int lane,
-                                        uint64_t &mask) {
+// Called by the whole wavefront: the lanes with `part` each get 4 flush list
+// entries; returns the lane's first entry, a multiple of 4 (meaningful where
+// part).  The list is drained first when the entries would not fit.
+__device__ inline uint32_t list_reserve4(const VtxCache &c, float *__restrict__ g, bool part,
+                                         uint32_t &nlist, int lane, uint64_t &mask) {
   mask = __ballot(part);
   if (mask == 0 || c.tag == nullptr)
     return 0;
-  const uint32_t total = per * static_cast<uint32_t>(__popcll(mask));
+  const uint32_t total = 4 * static_cast<uint32_t>(__popcll(mask)); // <= kFlushCap
   if (nlist + total > kFlushCap) {
     flush_list_drain(c, g, nlist, lane);
     nlist = 0;
   }
-  const uint32_t pos =
-      nlist + per * static_cast<uint32_t>(__popcll(mask & ((1ull << lane) - 1ull)));
+  const uint32_t below = __builtin_amdgcn_mbcnt_hi(
+      static_cast<uint32_t>(mask >> 32),
+      __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(mask), 0u));
+  const uint32_t pos = nlist + 4 * below;
   nlist += total;
   return pos;
 }
 
-// acc (8 corners x {x, y, z, te}) of the lanes with `part` -> the flush list
-// as the 8 vertices of cell `cell`, then acc = 0 there.  Whole wavefront.
-__device__ inline void list_cell_f32(float (&acc)[32], bool part, uint64_t cell,
-                                     float *__restrict__ g, uint64_t sx, uint64_t sy,
-                                     const VtxCache &vc, uint32_t &nlist, int lane) {
-  uint64_t mask;
-  const uint32_t pos = list_reserve(vc, g, part, 8, nlist, lane, mask);
-  if (mask == 0 || !part)
-    return;
+// The corner sums of the cell that a lane's ray is in, ordered along the
+// ray: bit 4 (x), 2 (y), 1 (z) of a corner's number is set for the vertex
+// that lies ahead on that axis, so a crossing always leaves the corners with
+// the bit clear, whatever the ray's direction.
+struct LaneCell {
+  float acc[32];     // 8 corners x {x, y, z, te}
+  int c[3];          // the cell's lower vertex (c[0] < 0: none yet)
+  bool up[3];        // the ray's cells go up the axis
+};
+
+// Vertex `cn` of the lane's cell.
+template <typename T>
+__device__ inline T cell_vertex(const LaneCell &q, const GridGeo &g, int cn) {
+  const T x = static_cast<T>(q.c[0] + (((cn >> 2) & 1) == q.up[0])),
+          y = static_cast<T>(q.c[1] + (((cn >> 1) & 1) == q.up[1])),
+          z = static_cast<T>(q.c[2] + ((cn & 1) == q.up[2]));
+  return (x * static_cast<T>(g.ny) + y) * static_cast<T>(g.nz) + z;
+}
+
+// The 4 corners FIRST, FIRST | B, FIRST | A, FIRST | A | B (A > B: the two
+// axes of a face) of the lane's cell: to the flush list at pos, or straight
+// to the grid when there is no cache (vertex indices beyond 32 bits).
+template <int FIRST, int A, int B>
+__device__ inline void list_face(const LaneCell &q, const GridGeo &geo, float *__restrict__ g,
+                                 const VtxCache &vc, uint32_t pos) {
+  constexpr int cn[4] = {FIRST, FIRST | B, FIRST | A, FIRST | A | B};
+  if (vc.tag) {
+    const uint32_t nz = static_cast<uint32_t>(geo.nz);
+    const uint32_t v = cell_vertex<uint32_t>(q, geo, FIRST);
+    const uint32_t sa = A == 4 ? nz * static_cast<uint32_t>(geo.ny) : nz, sb = B == 2 ? nz : 1u;
+    const uint32_t da = q.up[A == 4 ? 0 : 1] ? sa : 0u - sa,
+                   db = q.up[B == 2 ? 1 : 2] ? sb : 0u - sb;
+    *reinterpret_cast<uint4 *>(vc.ltag + pos) = make_uint4(v, v + db, v + da, v + da + db);
 #pragma unroll
-  for (int c = 0; c < 8; ++c) {
-    const uint64_t v = cell + (c >> 2) * sx + ((c >> 1) & 1) * sy + (c & 1);
-    list_put(vc, g, pos + c,
-             v, make_float4(acc[4 * c], acc[4 * c + 1], acc[4 * c + 2], acc[4 * c + 3]));
+    for (int i = 0; i < 4; ++i)
+      vc.lval[pos + i] = make_float4(q.acc[4 * cn[i]], q.acc[4 * cn[i] + 1],
+                                     q.acc[4 * cn[i] + 2], q.acc[4 * cn[i] + 3]);
+  } else {
 #pragma unroll
-    for (int m = 0; m < 4; ++m)
-      acc[4 * c + m] = 0.f;
+    for (int i = 0; i < 4; ++i)
+      grid_add4(g, cell_vertex<uint64_t>(q, geo, cn[i]),
+                make_float4(q.acc[4 * cn[i]], q.acc[4 * cn[i] + 1], q.acc[4 * cn[i] + 2],
+                            q.acc[4 * cn[i] + 3]));
   }
 }
 
-// The rays of the lanes with `part` move from `cell` to its neighbour along
-// one axis (BIT: 4 x, 2 y, 1 z in the corner numbering 4a + 2b + c),
-// upwards when `up`: the 4 corners they leave behind go to the flush list,
-// the 4 shared with the new cell move to their place in it, the new cell's
-// far corners start at 0, and `cell` becomes the new cell.  Whole wavefront.
-template <int BIT>
-__device__ inline void list_shift_f32(float (&acc)[32], bool part, bool up, uint64_t &cell,
-                                      float *__restrict__ g, uint64_t sx, uint64_t sy,
-                                      const VtxCache &vc, uint32_t &nlist, int lane) {
+// All 8 corners of the lanes with `part` -> the flush list, then acc = 0
+// there.  Whole wavefront.
+__device__ inline void list_cell_f32(LaneCell &q, bool part, const GridGeo &geo,
+                                     float *__restrict__ g, const VtxCache &vc, uint32_t &nlist,
+                                     int lane) {
   uint64_t mask;
-  const uint32_t pos = list_reserve(vc, g, part, 4, nlist, lane, mask);
+  uint32_t pos = list_reserve4(vc, g, part, nlist, lane, mask);
+  if (mask == 0)
+    return;
+  if (part)
+    list_face<0, 2, 1>(q, geo, g, vc, pos);
+  pos = list_reserve4(vc, g, part, nlist, lane, mask);
+  if (part) {
+    list_face<4, 2, 1>(q, geo, g, vc, pos);
+#pragma unroll
+    for (int i = 0; i < 32; ++i)
+      q.acc[i] = 0.f;
+  }
+}
+
+// The rays of the lanes with `part` move to the next cell along one axis
+// (BIT: 4 x, 2 y, 1 z): the 4 corners behind go to the flush list, those
+// ahead take their place, the new cell's corners ahead start at 0.  Whole
+// wavefront.  A few of the 64 lanes cross at a step, but nearly every step
+// has one that does, so this is paid by each step: with corners ordered by
+// the grid's axes it took three selects a sum (up or down) and 64-bit vertex
+// arithmetic.
+template <int BIT>
+__device__ inline void list_shift_f32(LaneCell &q, bool part, const GridGeo &geo,
+                                      float *__restrict__ g, const VtxCache &vc, uint32_t &nlist,
+                                      int lane) {
+  constexpr int axis = BIT == 4 ? 0 : (BIT == 2 ? 1 : 2);
+  uint64_t mask;
+  const uint32_t pos = list_reserve4(vc, g, part, nlist, lane, mask);
   if (mask == 0 || !part)
     return;
-  int j = 0;
+  if (BIT == 4)
+    list_face<0, 2, 1>(q, geo, g, vc, pos);
+  else if (BIT == 2)
+    list_face<0, 4, 1>(q, geo, g, vc, pos);
+  else
+    list_face<0, 4, 2>(q, geo, g, vc, pos);
 #pragma unroll
-  for (int lo = 0; lo < 8; ++lo) {
-    if (lo & BIT)
+  for (int c = 0; c < 8; ++c) {
+    if (c & BIT)
       continue;
-    const int hi = lo | BIT;
-    const uint64_t vlo = cell + (lo >> 2) * sx + ((lo >> 1) & 1) * sy + (lo & 1);
-    const uint64_t vhi = cell + (hi >> 2) * sx + ((hi >> 1) & 1) * sy + (hi & 1);
-    float left[4];
 #pragma unroll
     for (int m = 0; m < 4; ++m) {
-      left[m] = up ? acc[4 * lo + m] : acc[4 * hi + m];
-      const float kept = up ? acc[4 * hi + m] : acc[4 * lo + m];
-      acc[4 * lo + m] = up ? kept : 0.f;
-      acc[4 * hi + m] = up ? 0.f : kept;
+      q.acc[4 * c + m] = q.acc[4 * (c | BIT) + m];
+      q.acc[4 * (c | BIT) + m] = 0.f;
     }
-    list_put(vc, g, pos + j, up ? vlo : vhi, make_float4(left[0], left[1], left[2], left[3]));
-    ++j;
   }
-  const uint64_t st = BIT == 4 ? sx : (BIT == 2 ? sy : 1);
-  cell = up ? cell + st : cell - st;
+  q.c[axis] += q.up[axis] ? 1 : -1;
 }
 
 template <bool GRIDS, bool PW1>
@@ -999,12 +1053,17 @@ __device__ void adj_lanes_f32(const BInst &in, int s, uint64_t ipix, bool live,
     vc.tag = nullptr;
   double p0 = 0., p1 = 0., p2 = 0., p3 = 0., p4 = 0., p5 = 0., q0 = 0.;
   double after = 0., dacc = 0.; // FD and R contributions of the samples beyond
-  float acc[32];
+  LaneCell q;
 #pragma unroll
   for (int i = 0; i < 32; ++i)
-    acc[i] = 0.f;
-  uint64_t cur = ~0ull; // cell whose corner sums acc holds
-  int ccx = 0, ccy = 0, ccz = 0;
+    q.acc[i] = 0.f;
+  q.c[0] = q.c[1] = q.c[2] = -2; // no cell's neighbour
+  // the sweep runs towards the observer: the ray's cell goes up an axis
+  // where its direction points down it (a straight ray's cell only ever
+  // moves one way along an axis: every rounding on the way to it is monotonic)
+  q.up[0] = r.l.x * in.gsx < 0.;
+  q.up[1] = r.l.y * in.gsy < 0.;
+  q.up[2] = r.l.z * in.gsz < 0.;
   // the union of the lanes' step ranges, far end first
   const uint64_t k_end = wave_max_u64(live ? r.k_hi : 0ull);
   const uint64_t k_beg = wave_min_u64(live ? r.k_lo : ~0ull);
@@ -1048,24 +1107,21 @@ __device__ void adj_lanes_f32(const BInst &in, int s, uint64_t ipix, bool live,
       dbx = ft * lf.x;
       dby = ft * lf.y;
       dbz = ft * lf.z;
-      if (o.bper2 > 0.f) {
-        const float coef = dLdw * 2.f * in.f.hexp * o.w * __builtin_amdgcn_rcpf(o.bper2);
-        dbx += coef * (o.bx - o.b_par * lf.x);
-        dby += coef * (o.by - o.b_par * lf.y);
-        dbz += coef * (o.bz - o.b_par * lf.z);
-        // ln |B_perp| in Gauss: the B grid and b0 are in muG here
-        const double lnb = 0.5 * static_cast<double>(__logf(o.bper2)) - 13.815510557964274;
-        p4 += static_cast<double>(o.w) *
-              (AIL + static_cast<double>(alpha_p) + 0.5 * lnb * static_cast<double>(dLdw));
-      }
-      if (o.n2 > 0.f) {
-        const float cc = dipa * __builtin_amdgcn_rcpf(o.n2);
-        dbx += cc * (o.y * ephf.x - o.x * ethf.x);
-        dby += cc * (o.y * ephf.y - o.x * ethf.y);
-        dbz += cc * (o.y * ephf.z - o.x * ethf.z);
-      }
-      if (o.te_in)
-        p5 += dte;
+      const bool perp = o.bper2 > 0.f;
+      const float bp2 = perp ? o.bper2 : 1.f, wp = perp ? o.w : 0.f;
+      const float coef = dLdw * 2.f * in.f.hexp * wp * __builtin_amdgcn_rcpf(bp2);
+      dbx += coef * (o.bx - o.b_par * lf.x);
+      dby += coef * (o.by - o.b_par * lf.y);
+      dbz += coef * (o.bz - o.b_par * lf.z);
+      // ln |B_perp| in Gauss: the B grid and b0 are in muG here
+      const double lnb = 0.5 * static_cast<double>(__logf(bp2)) - 13.815510557964274;
+      p4 += static_cast<double>(wp) *
+            (AIL + static_cast<double>(alpha_p) + 0.5 * lnb * static_cast<double>(dLdw));
+      const float cc = (o.n2 > 0.f ? dipa : 0.f) * __builtin_amdgcn_rcpf(o.n2 > 0.f ? o.n2 : 1.f);
+      dbx += cc * (o.y * ephf.x - o.x * ethf.x);
+      dby += cc * (o.y * ephf.y - o.x * ethf.y);
+      dbz += cc * (o.y * ephf.z - o.x * ethf.z);
+      p5 += o.te_in ? dte : 0.;
       if (o.lsa_in) {
         const float u = o.sps * o.cos_p - o.cps * o.sin_p;
         const float v = o.sps * o.sin_p + o.cps * o.cos_p;
@@ -1082,45 +1138,39 @@ __device__ void adj_lanes_f32(const BInst &in, int s, uint64_t ipix, bool live,
       // corner sums of the cell (face steps one axis at a time: every
       // intermediate cell lies between two valid cells, so is valid)
       const bool in_cell = valid && o.cell_ok;
-      const bool moves = in_cell && cur != ~0ull && o.idx != cur;
-      int dx = 0, dy = 0, dz = 0;
-      if (moves) {
-        dx = o.cx - ccx;
-        dy = o.cy - ccy;
-        dz = o.cz - ccz;
-      }
-      const bool near = dx >= -1 && dx <= 1 && dy >= -1 && dy <= 1 && dz >= -1 && dz <= 1;
-      uint64_t c = cur;
-      list_shift_f32<4>(acc, moves && near && dx != 0, dx > 0, c, ggrid, sx, sy, vc, nlist,
-                        lane);
-      list_shift_f32<2>(acc, moves && near && dy != 0, dy > 0, c, ggrid, sx, sy, vc, nlist,
-                        lane);
-      list_shift_f32<1>(acc, moves && near && dz != 0, dz > 0, c, ggrid, sx, sy, vc, nlist,
-                        lane);
-      list_cell_f32(acc, moves && !near, cur, ggrid, sx, sy, vc, nlist, lane);
+      const int dx = o.cx - q.c[0], dy = o.cy - q.c[1], dz = o.cz - q.c[2];
+      const bool moves = in_cell && q.c[0] >= 0;
+      // one step the ray's way at most, along each axis
+      const bool near = static_cast<uint32_t>(q.up[0] ? dx : -dx) <= 1u &&
+                        static_cast<uint32_t>(q.up[1] ? dy : -dy) <= 1u &&
+                        static_cast<uint32_t>(q.up[2] ? dz : -dz) <= 1u;
+      list_shift_f32<4>(q, moves && near && dx != 0, in.geo, ggrid, vc, nlist, lane);
+      list_shift_f32<2>(q, moves && near && dy != 0, in.geo, ggrid, vc, nlist, lane);
+      list_shift_f32<1>(q, moves && near && dz != 0, in.geo, ggrid, vc, nlist, lane);
+      list_cell_f32(q, moves && !near, in.geo, ggrid, vc, nlist, lane);
       if (in_cell) {
-        if (o.idx != cur) {
-          cur = o.idx;
-          ccx = o.cx;
-          ccy = o.cy;
-          ccz = o.cz;
-        }
+        q.c[0] = o.cx;
+        q.c[1] = o.cy;
+        q.c[2] = o.cz;
         const float gte = static_cast<float>(dte);
-        const float wx[2] = {1.f - o.xd, o.xd}, wy[2] = {1.f - o.yd, o.yd},
-                    wz[2] = {1.f - o.zd, o.zd};
+        const float x1 = 1.f - o.xd, y1 = 1.f - o.yd, z1 = 1.f - o.zd;
+        // {behind, ahead}
+        const float wx[2] = {q.up[0] ? x1 : o.xd, q.up[0] ? o.xd : x1},
+                    wy[2] = {q.up[1] ? y1 : o.yd, q.up[1] ? o.yd : y1},
+                    wz[2] = {q.up[2] ? z1 : o.zd, q.up[2] ? o.zd : z1};
 #pragma unroll
         for (int cn = 0; cn < 8; ++cn) {
           const float w = wx[cn >> 2] * wy[(cn >> 1) & 1] * wz[cn & 1];
-          acc[4 * cn + 0] += w * dbx;
-          acc[4 * cn + 1] += w * dby;
-          acc[4 * cn + 2] += w * dbz;
-          acc[4 * cn + 3] += w * gte;
+          q.acc[4 * cn + 0] += w * dbx;
+          q.acc[4 * cn + 1] += w * dby;
+          q.acc[4 * cn + 2] += w * dbz;
+          q.acc[4 * cn + 3] += w * gte;
         }
       }
     }
   }
   if (GRIDS && ggrid) {
-    list_cell_f32(acc, cur != ~0ull, cur, ggrid, sx, sy, vc, nlist, lane);
+    list_cell_f32(q, q.c[0] >= 0, in.geo, ggrid, vc, nlist, lane);
     if (vc.tag) {
       flush_list_drain(vc, ggrid, nlist, lane);
       vtx_cache_flush(vc, ggrid, lane);
@@ -1226,7 +1276,7 @@ __device__ void do_item(const LevelArgs &a, uint64_t item, int lane, void *slab,
 // selects the reverse-mode sweep.
 template <int PREC, bool GRIDS, bool PW1, bool REV>
 __global__ __launch_bounds__(256)
-__attribute__((amdgpu_waves_per_eu(PREC == HAMX_PREC_F32 && !REV ? 3 : 1))) void k_batch_march(
+__attribute__((amdgpu_waves_per_eu(PREC == HAMX_PREC_F32 ? (REV ? 2 : 3) : 1))) void k_batch_march(
     LevelArgs a) {
   const int lane = threadIdx.x & 63;
   const uint32_t wave = threadIdx.x >> 6, wpb = blockDim.x >> 6;
