@@ -57,7 +57,8 @@ struct AdjShell {
 };
 
 template <bool GRIDS, bool PW1, bool MODELS>
-__global__ __launch_bounds__(256) void k_los_adj(Phys ph, FastConst fc, AdjConst ac,
+__global__ __launch_bounds__(256)
+__attribute__((amdgpu_waves_per_eu(MODELS ? 1 : 3))) void k_los_adj(Phys ph, FastConst fc, AdjConst ac,
                                                  Grids gr, ShellArgs sa, AdjShell as) {
   // kAdjRays consecutive rays per wavefront (set up one per lane), and a
   // per-wavefront cell cache that merges their grid-gradient contributions

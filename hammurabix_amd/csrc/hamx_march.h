@@ -283,29 +283,41 @@ constexpr int kAdjRays = 2;
 // costs about 30 times a plain 64-lane LDS store or load (measured on
 // gfx950), so the 32 corner values of a chunk's samples are merged without
 // atomics: every lane stores its values into a per-wavefront staging area
-// (16 values at a time), and the lanes then sum each run of samples that
-// share a cell transposed, one lane per (value, run), 4 runs at a time.
+// (kStageRows values at a time), and the lanes then sum each run of samples
+// that share a cell transposed, one lane per (value, run), 8 runs at a time;
+// what a run needs (its lanes, slot and cell) stands in a small LDS table.
+// Bound by the chain of LDS round trips and FP64 issue at few wavefronts:
+// 16 rows, run bounds found by scalar loops and one staged load at a time
+// left two wavefronts a SIMD (48 % VALU issue); 8 rows, the table and 4 loads
+// in flight leave three, and the adjoint of a 256x256x64 three-shell map of
+// nside 128 went from 5.27 to 3.90 ms (loads in flight alone 4.69, the table
+// 4.36, 8 rows with three wavefronts 3.90; two wavefronts with 50 slots 4.55).
 // Each run's sums go once into the run's slot of a per-wavefront cell
 // cache (plain stores: one wavefront owns its cache and, within a chunk,
 // each slot serves one run), or straight to the grid when an earlier run
 // of the chunk holds the slot.  A cell reaches the grid (32 global atomics)
 // when its slot is taken by another cell and at the end of the wavefront.
-constexpr int kStageSlots = 40; // the most that keeps two 4-wave workgroups per CU
+constexpr int kStageSlots = 28; // the most that keeps three 4-wave workgroups per CU (even: 16-byte records)
+constexpr int kStageRows = 8;  // values staged at a time
+constexpr int kStageAhead = 4; // staged loads in flight
 constexpr int kStageStride = 65; // doubles per staged row: 64 lanes + 1, so rows start in different banks
 
 struct StagedCache {
   unsigned long long *key; // cell held by each slot (~0: empty)
   double *val;             // kStageSlots x 32 values
-  double *stage;           // 16 rows x kStageStride
+  double *stage;           // kStageRows rows x kStageStride
+  uint4 *run;              // the chunk's runs: {first | last + 1 << 8 | fresh << 16 |
+                           // direct << 17, slot, cell}
 };
 
 constexpr int staged_cache_bytes() {
-  return kStageSlots * (8 + 32 * 8) + 16 * kStageStride * 8;
+  return 64 * 16 + kStageSlots * (8 + 32 * 8) + kStageRows * kStageStride * 8;
 }
 
 __device__ inline StagedCache staged_at(void *base) {
   StagedCache c;
-  c.key = static_cast<unsigned long long *>(base);
+  c.run = static_cast<uint4 *>(base);
+  c.key = reinterpret_cast<unsigned long long *>(c.run + 64);
   c.val = reinterpret_cast<double *>(c.key + kStageSlots);
   c.stage = c.val + 32 * kStageSlots;
   return c;
@@ -397,7 +409,6 @@ __device__ inline void scatter_staged(const StagedCache &c, double *__restrict__
   const bool mine = head && has && !((direct >> lane) & 1ull);
   const bool fresh = mine && held != key;           // the run claims its slot
   const bool evict = fresh && held != ~0ull;        // ... from another cell
-  const unsigned long long fresh_runs = __ballot(fresh);
   unsigned long long ev_slots = 0;
   for (unsigned long long t = __ballot(evict); t; t &= t - 1)
     ev_slots |= 1ull << __builtin_amdgcn_readlane(s_own, __ffsll(t) - 1);
@@ -405,59 +416,57 @@ __device__ inline void scatter_staged(const StagedCache &c, double *__restrict__
   wave_lds_sync();
   if (fresh)
     c.key[s_own] = key;
-  // this lane's corner values (0 without a sample), 16 per half: corners
-  // 4 half .. 4 half + 3 (the x = half plane), formed just before they are
-  // staged so that only half of them hold registers
-  const double wy[2] = {1. - yd, yd}, wz[2] = {1. - zd, zd};
-  const int vi = lane & 15, grp = lane >> 4;
+  if (head && has) {
+    const unsigned long long later = heads & ~((2ull << lane) - 1ull);
+    const uint32_t end = later ? static_cast<uint32_t>(__ffsll(later) - 1) : 64u;
+    c.run[__popcll(runs & ((1ull << lane) - 1ull))] =
+        make_uint4(static_cast<uint32_t>(lane) | end << 8 | (fresh ? 1u << 16 : 0u) |
+                       (mine ? 0u : 1u << 17),
+                   static_cast<uint32_t>(s_own), static_cast<uint32_t>(key),
+                   static_cast<uint32_t>(key >> 32));
+  }
+  // this lane's corner values (0 without a sample), kStageRows at a time,
+  // formed just before they are staged so that only these hold registers
+  const double wx[2] = {has ? 1. - xd : 0., has ? xd : 0.}, wy[2] = {1. - yd, yd},
+               wz[2] = {1. - zd, zd};
+  constexpr int kGroups = 64 / kStageRows; // runs per round
+  const int vi = lane % kStageRows, grp = lane / kStageRows;
+  const int nrun = __popcll(runs);
+  const double *row = c.stage + vi * kStageStride;
 #pragma unroll
-  for (int half = 0; half < 2; ++half) {
-    const double wxh = has ? (half ? xd : 1. - xd) : 0.;
-    wave_lds_sync(); // the previous half's loads are done before the rows are rewritten
+  for (int part = 0; part < 32 / kStageRows; ++part) {
+    wave_lds_sync(); // the previous part's loads are done before the rows are rewritten
 #pragma unroll
-    for (int cq = 0; cq < 4; ++cq) {
-      const double w = wxh * wy[cq >> 1] * wz[cq & 1];
-      c.stage[(4 * cq + 0) * kStageStride + lane] = w * g0;
-      c.stage[(4 * cq + 1) * kStageStride + lane] = w * g1;
-      c.stage[(4 * cq + 2) * kStageStride + lane] = w * g2;
-      c.stage[(4 * cq + 3) * kStageStride + lane] = w * g3;
+    for (int i = 0; i < kStageRows / 4; ++i) {
+      const int cn = part * (kStageRows / 4) + i;
+      const double w = wx[cn >> 2] * wy[(cn >> 1) & 1] * wz[cn & 1];
+      c.stage[(4 * i + 0) * kStageStride + lane] = w * g0;
+      c.stage[(4 * i + 1) * kStageStride + lane] = w * g1;
+      c.stage[(4 * i + 2) * kStageStride + lane] = w * g2;
+      c.stage[(4 * i + 3) * kStageStride + lane] = w * g3;
     }
     wave_lds_sync();
-    for (unsigned long long t = runs; t;) { // uniform: 4 runs per round
-      int a[4], b[4], len = 0;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        a[j] = b[j] = 0;
-        if (t) {
-          a[j] = __ffsll(t) - 1;
-          t &= t - 1;
-          const unsigned long long later = heads & ~((2ull << a[j]) - 1ull);
-          b[j] = later ? __ffsll(later) - 1 : 64;
-          len = max(len, b[j] - a[j]);
-        }
-      }
-      // the run of this lane's 16-lane group (run heads are uniform)
-      unsigned long long cl[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        cl[j] = lane_u64(key, a[j]);
-      const int ra = grp == 0 ? a[0] : grp == 1 ? a[1] : grp == 2 ? a[2] : a[3];
-      const int rb = grp == 0 ? b[0] : grp == 1 ? b[1] : grp == 2 ? b[2] : b[3];
-      const unsigned long long cell = grp == 0 ? cl[0] : grp == 1 ? cl[1] : grp == 2 ? cl[2] : cl[3];
+    for (int r = grp; r < nrun; r += kGroups) {
+      const uint4 d = c.run[r];
+      const int rb = static_cast<int>((d.x >> 8) & 0xffu);
+      // kStageAhead loads in flight: one at a time, each sample of the
+      // longest run waited for its own LDS round trip
       double sum = 0.;
-      for (int k = 0; k < len; ++k) {
-        const int i = ra + k;
-        if (i < rb)
-          sum += c.stage[vi * kStageStride + i];
+      for (int k = static_cast<int>(d.x & 0xffu); k < rb; k += kStageAhead) {
+        double v[kStageAhead];
+#pragma unroll
+        for (int j = 0; j < kStageAhead; ++j)
+          v[j] = row[min(k + j, 63)];
+#pragma unroll
+        for (int j = 0; j < kStageAhead; ++j)
+          sum += k + j < rb ? v[j] : 0.;
       }
-      if (rb > ra) {
-        const int val = 16 * half + vi;
-        if ((direct >> ra) & 1ull) {
-          staged_grid_add(g, cell, val, sum, sx, sy);
-        } else {
-          double *q = c.val + 32 * staged_hash(cell) + val;
-          *q = ((fresh_runs >> ra) & 1ull) ? sum : *q + sum;
-        }
+      const int val = kStageRows * part + vi;
+      if ((d.x >> 17) & 1u) {
+        staged_grid_add(g, static_cast<unsigned long long>(d.w) << 32 | d.z, val, sum, sx, sy);
+      } else {
+        double *q = c.val + 32 * d.y + val;
+        *q = ((d.x >> 16) & 1u) ? sum : *q + sum;
       }
     }
   }
