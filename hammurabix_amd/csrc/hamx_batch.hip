@@ -256,15 +256,17 @@ struct S32 {
   int cx, cy, cz; // the cell's lower corner
 };
 
-// The four corners c of a cell's lower or upper x plane at (yd, zd).
-__device__ inline void lerp_plane_f4(const float4 *c, float zd, float yd, float4 &w) {
-  // FP32 sample arithmetic: a * b + c may fuse (more accurate, fewer instructions)
-  #pragma clang fp contract(fast)
-  const float z1 = 1.f - zd, y1 = 1.f - yd;
-  w.x = (c[0].x * z1 + c[1].x * zd) * y1 + (c[2].x * z1 + c[3].x * zd) * yd;
-  w.y = (c[0].y * z1 + c[1].y * zd) * y1 + (c[2].y * z1 + c[3].y * zd) * yd;
-  w.z = (c[0].z * z1 + c[1].z * zd) * y1 + (c[2].z * z1 + c[3].z * zd) * yd;
-  w.w = (c[0].w * z1 + c[1].w * zd) * y1 + (c[2].w * z1 + c[3].w * zd) * yd;
+// a (1 - t) + b t with t1 = 1 - t, fused one way whatever surrounds it (left
+// to the compiler, the rounded product was the one or the other with the
+// order of loads and branches around it).
+__device__ inline float lerp_f32(float a, float b, float t, float t1) {
+  return __builtin_fmaf(t1, a, t * b);
+}
+
+__device__ inline float4 lerp_f4(const float4 &a, const float4 &b, float t) {
+  const float t1 = 1.f - t;
+  return make_float4(lerp_f32(a.x, b.x, t, t1), lerp_f32(a.y, b.y, t, t1),
+                     lerp_f32(a.z, b.z, t, t1), lerp_f32(a.w, b.w, t, t1));
 }
 
 // sin and cos of an FP32 angle |r| <= pi/4: the Taylor series to the terms
@@ -433,20 +435,17 @@ __device__ inline bool eval_f32(const BInst &in, const BShell &sh, const RayGeo 
     o.zd = static_cast<float>(cell.zd);
     o.yd = static_cast<float>(cell.yd);
     o.xd = static_cast<float>(cell.xd);
-    float4 w1, w2;
-    lerp_plane_f4(cn, o.zd, o.yd, w1);
-    lerp_plane_f4(cn + 4, o.zd, o.yd, w2);
+    const float4 w = lerp_f4(lerp_f4(lerp_f4(cn[0], cn[1], o.zd), lerp_f4(cn[2], cn[3], o.zd), o.yd),
+                             lerp_f4(lerp_f4(cn[4], cn[5], o.zd), lerp_f4(cn[6], cn[7], o.zd), o.yd),
+                             o.xd);
     if (o.cell_ok) {
-      const float x1 = 1.f - o.xd;
-      const float gx = w1.x * x1 + w2.x * o.xd;
-      const float gy = w1.y * x1 + w2.y * o.xd;
-      const float gz = w1.z * x1 + w2.z * o.xd;
+      const float gx = w.x, gy = w.y, gz = w.z;
       bx += gx;
       by += gy;
       bz += gz;
       bpar += static_cast<double>(gx) * r.l.x + static_cast<double>(gy) * r.l.y +
               static_cast<double>(gz) * r.l.z;
-      te_d += static_cast<double>(w1.w * x1 + w2.w * o.xd);
+      te_d += static_cast<double>(w.w);
     }
   }
   o.te_raw = static_cast<float>(te_d); // the clamp decision keeps te_d's sign
