@@ -700,7 +700,7 @@ def main():
             "accumulate_ms_per_step": acc_ms / args.steps,
             "random_field_generation_ms": gen_ms,
             "es_generator_ms": es_ms,
-            "es_generator_algorithmic_GBps": 800 * n / (es_ms * 1e-3) / 1e9,
+            "es_generator_algorithmic_GBps": 248 * n / (es_ms * 1e-3) / 1e9,
             "maps_finite": finite,
             "map_gradient_evals_per_s": 1.0 / mg_s,
             "map_gradient_ms": mg_s * 1e3,
