@@ -36,7 +36,7 @@ struct hamx_ctx {
   // Host copy of small per-call tables uploaded asynchronously; it lives
   // until the next call so the copy never reads freed memory.
   std::vector<double> host_tab;
-  // Set to 1 by a march that meets a non-finite ray: pinned host memory that
+  // Set to 1 where a ray's values are not finite: pinned host memory that
   // kernels write and the host reads after synchronising (hamx_open makes it).
   int *nonfinite = nullptr;
 };

@@ -183,8 +183,14 @@ __device__ inline bool eval_sample(const Phys &ph, const Grids &gr,
 // (integrator.cc:99-115).  A NaN or an infinity in an input grid or parameter
 // reaches a ray's values (the reference's debug build asserts isfinite on
 // B_par, B_per, te and the phase, integrator.cc:192,195,202,223; its release
-// build carries the NaN): the flag is raised here, where they are at hand (the
-// HEALPix interpolation of the accumulation skips a NaN as an undefined pixel).
+// build carries the NaN).  FLAG (k_los_ray, whose small shells cost their
+// launches) raises the pass's flag here, where they are at hand; behind the
+// other marches k_nonfinite reads the shell maps, 17 us for three shells up to
+// nside 256: the flag's pointer, held over their sample loops in two more
+// scalar registers, cost them 105 us in spilled scalars read back (a pass of
+// 256x256x64 random grids 5.47 -> 5.34 ms, an analytic one at nside 32 261 ->
+// 246 us without it).
+template <bool FLAG>
 __device__ inline void store_ray(const Phys &ph, const ShellArgs &sa,
                                  uint64_t ipix, double dm, double fd, double I,
                                  double Q, double U) {
@@ -206,18 +212,19 @@ __device__ inline void store_ray(const Phys &ph, const ShellArgs &sa,
     sa.t_fd[ipix] = fd;
     ok = ok && isfinite(fd);
   }
-  if (!ok)
+  if (FLAG && !ok)
     __hip_atomic_store(sa.nonfinite, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // Masked-out pixel (integrator.cc:63-70): every observable of the shell is
 // zero.  True when the caller should return.
+template <bool FLAG>
 __device__ inline bool masked_out(const Phys &ph, const ShellArgs &sa, uint64_t ipix,
                                   bool writer) {
   if (!sa.mask || sa.mask[ipix] == 1.0)
     return false;
   if (writer)
-    store_ray(ph, sa, ipix, 0., 0., 0., 0., 0.);
+    store_ray<FLAG>(ph, sa, ipix, 0., 0., 0., 0., 0.);
   return true;
 }
 
@@ -240,7 +247,7 @@ k_los_wave(Phys ph, Grids gr, ShellArgs sa) {
       static_cast<uint64_t>(blockIdx.x) * (blockDim.x >> 6) + (threadIdx.x >> 6);
   if (ipix >= sa.hs.npix)
     return; // uniform per wavefront
-  if (masked_out(ph, sa, ipix, lane == 0))
+  if (masked_out<false>(ph, sa, ipix, lane == 0))
     return; // uniform per wavefront
   RayGeo r;
   ray_setup(ph, sa, ipix, r);
@@ -276,7 +283,7 @@ k_los_wave(Phys ph, Grids gr, ShellArgs sa) {
   Q = wave_sum(Q);
   U = wave_sum(U);
   if (lane == 0)
-    store_ray(ph, sa, ipix, dm, fd, I, Q, U);
+    store_ray<false>(ph, sa, ipix, dm, fd, I, Q, U);
 }
 
 // ---------------------------------------------------- specialised march --
@@ -332,7 +339,7 @@ k_los_fast(Phys ph, FastConst fc, Grids gr, ShellArgs sa) {
   const double two_l2 = 2. * ph.lambda_sq;
   for (uint64_t j = 0; j < nr; ++j) {
     const uint64_t ipix = p0 + j;
-    if (masked_out(ph, sa, ipix, lane == 0))
+    if (masked_out<false>(ph, sa, ipix, lane == 0))
       continue; // uniform per wavefront
     const RayGeo r = slots[wave][j];
     double dm = 0., I = 0., Q = 0., U = 0., fd_carry = 0.;
@@ -361,7 +368,7 @@ k_los_fast(Phys ph, FastConst fc, Grids gr, ShellArgs sa) {
     Q = wave_sum(Q);
     U = wave_sum(U);
     if (lane == 0)
-      store_ray(ph, sa, ipix, dm, fd_carry, I, Q, U);
+      store_ray<false>(ph, sa, ipix, dm, fd_carry, I, Q, U);
   }
 }
 
@@ -393,7 +400,7 @@ k_los_ray(Phys ph, FastConst fc, Grids gr, ShellArgs sa, int rays) {
   int turn = 0;
   for (int j = 0; j < nr; ++j) {
     const uint64_t ipix = p0 + j;
-    if (masked_out(ph, sa, ipix, threadIdx.x == 0))
+    if (masked_out<true>(ph, sa, ipix, threadIdx.x == 0))
       continue; // uniform
     const RayGeo r = slots[j];
     double dm = 0., I = 0., Q = 0., U = 0., fd_carry = 0.;
@@ -440,7 +447,7 @@ k_los_ray(Phys ph, FastConst fc, Grids gr, ShellArgs sa, int rays) {
       for (int m = 0; m < 4; ++m)
         t[m] = (out[0][m] + out[1][m]) + (out[2][m] + out[3][m]);
       // a shell thinner than one step: no finite delta
-      store_ray(ph, sa, ipix, sa.step ? t[0] * sa.delta : 0., fd_carry, t[1], t[2], t[3]);
+      store_ray<true>(ph, sa, ipix, sa.step ? t[0] * sa.delta : 0., fd_carry, t[1], t[2], t[3]);
     }
   }
 }
@@ -456,7 +463,7 @@ k_los_thread(Phys ph, Grids gr, ShellArgs sa) {
   const uint64_t ipix = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   if (ipix >= sa.hs.npix)
     return;
-  if (masked_out(ph, sa, ipix, true))
+  if (masked_out<false>(ph, sa, ipix, true))
     return;
   RayGeo r;
   ray_setup(ph, sa, ipix, r);
@@ -476,7 +483,7 @@ k_los_thread(Phys ph, Grids gr, ShellArgs sa) {
       U += sin(2. * qui) * s.jp;
     }
   }
-  store_ray(ph, sa, ipix, dm, fd, I, Q, U);
+  store_ray<false>(ph, sa, ipix, dm, fd, I, Q, U);
 }
 
 // ------------------------------------------------------------- accumulate --
@@ -899,6 +906,28 @@ extern "C" int hamx_los_samples(const hamx_los_desc *d, uint64_t *samples) {
 }
 
 namespace hamx {
+namespace {
+// Raises the pass's flag where a shell map holds a value that is not finite (the
+// HEALPix interpolation of the accumulation skips a NaN as an undefined pixel).
+struct FiniteArgs {
+  const double *m[5];
+  int k;
+  uint64_t n;
+  int *flag;
+};
+
+__global__ __launch_bounds__(256) void k_nonfinite(FiniteArgs a) {
+  const uint64_t stride = static_cast<uint64_t>(gridDim.x) * blockDim.x;
+  bool bad = false;
+  for (int j = 0; j < a.k; ++j)
+    for (uint64_t i = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < a.n;
+         i += stride)
+      bad |= !isfinite(a.m[j][i]);
+  if (bad)
+    __hip_atomic_store(a.flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+} // namespace
+
 int los_forward_impl(hamx_ctx *ctx, const hamx_los_desc *d, const hamx_fields *fields,
                      hamx_maps *out, uint32_t flags, double *ckpt, double *shell_fd,
                      Arena *ar) {
@@ -1051,6 +1080,7 @@ int los_forward_impl(hamx_ctx *ctx, const hamx_los_desc *d, const hamx_fields *f
     if (ckpt && d->do_fd && s > 0) // FD map before shell s, for the adjoint
       HAMX_HIP(ctx, hipMemcpyAsync(ckpt + s * h_fd.npix, o_fd, h_fd.npix * sizeof(double),
                                    hipMemcpyDeviceToDevice, ctx->stream));
+    bool scan = true; // the march leaves the flag to k_nonfinite
     ProfMark pm = prof_begin(ctx);
     if (fast) {
       const FastConst fc = make_fast(d, ph, sa.delta, pw1);
@@ -1065,6 +1095,7 @@ int los_forward_impl(hamx_ctx *ctx, const hamx_los_desc *d, const hamx_fields *f
       // 912), two rays per workgroup from nside 32 on.
       const int rays = npix <= 3072 ? 1 : creg ? 2 : 0;
       const bool ray = rays > 0;
+      scan = !ray;
       const unsigned blocks =
           static_cast<unsigned>(ray ? (npix + rays - 1) / rays : (npix + 4 * kFastRays - 1) / (4 * kFastRays));
 #define HAMX_LAUNCH_FAST(G, P, M, C)                                                       \
@@ -1169,6 +1200,22 @@ int los_forward_impl(hamx_ctx *ctx, const hamx_los_desc *d, const hamx_fields *f
     prof_end(ctx, pm,
              fast ? "los_fast" : (sched == HAMX_SCHED_WAVE ? "los_wave" : "los_thread"), s,
              npix * sa.step);
+    if (scan) {
+      FiniteArgs fa;
+      std::memset(&fa, 0, sizeof(fa));
+      for (const double *m : {static_cast<const double *>(sa.t_dm),
+                              static_cast<const double *>(sa.t_fd),
+                              static_cast<const double *>(sa.t_is),
+                              static_cast<const double *>(sa.t_qs),
+                              static_cast<const double *>(sa.t_us)})
+        if (m)
+          fa.m[fa.k++] = m;
+      fa.n = npix;
+      fa.flag = ctx->nonfinite;
+      const unsigned fb = static_cast<unsigned>(std::min<uint64_t>((npix + 255) / 256, 1024));
+      hipLaunchKernelGGL(k_nonfinite, dim3(fb), dim3(256), 0, ctx->stream, fa);
+      HAMX_HIP(ctx, hipGetLastError());
+    }
     // accumulate shell maps into the outputs (integrator.cc:122-132)
     auto add = [](AccPairs &pairs, double *dst, const double *src) {
       if (dst == src)
@@ -1240,7 +1287,7 @@ int los_forward_impl(hamx_ctx *ctx, const hamx_los_desc *d, const hamx_fields *f
   if (d->do_fd || d->do_sync)
     HAMX_TRY(copy_out(out->fd, o_fd, h_fd));
   HAMX_HIP(ctx, hipStreamSynchronize(ctx->stream));
-  if (*const_cast<volatile int *>(ctx->nonfinite) != 0) // raised by the marches
+  if (*const_cast<volatile int *>(ctx->nonfinite) != 0)
     return set_err(ctx, HAMX_ERR_ARG,
                    "non-finite values on the lines of sight: an input grid or parameter "
                    "holds a NaN or an infinity");

@@ -333,3 +333,24 @@ def test_lsa_angles_beyond_a_quarter_turn(ctx, angles):
     d.breg[1] = math.radians(psi0)
     d.breg[3] = math.radians(chi0)
     assert_parity(gpu_maps(ctx, d), write_grid(d), label=f"lsa {psi0}/{chi0}")
+
+
+@pytest.mark.parametrize("schedule", [capi.HAMX_SCHED_AUTO, capi.HAMX_SCHED_WAVE,
+                                      capi.HAMX_SCHED_THREAD])
+@pytest.mark.parametrize("nside_out", [32, 8])
+def test_nan_on_a_large_shell_is_an_error(ctx, schedule, nside_out):
+    """The same on a shell whose march leaves the check to a scan of the shell
+    maps, written to the output or interpolated (which skips a NaN): one
+    vertex, far enough out that few of the 12288 rays meet its cells."""
+    print("case: nan on a large shell", schedule, nside_out, flush=True)
+    par = Param(text=configs.random_forward(shell_num=1, nside_sim=32, nside_out=nside_out,
+                                            oc_r_res=0.2, grid=(32, 32, 16)))
+    d = par.los_desc(schedule=schedule)
+    b, te, box = random_grids((32, 32, 16), seed=22)
+    bad = tuple(a.copy() for a in b)
+    bad[2][(26 * 32 + 10) * 16 + 5] = np.nan
+    kw = dict(brnd_box=box, ternd=te, ternd_box=box)
+    with pytest.raises(HamxError) as e:
+        gpu_maps(ctx, d, brnd=bad, **kw)
+    assert e.value.code == capi.HAMX_ERR_ARG and "non-finite" in str(e.value)
+    assert_parity(gpu_maps(ctx, d, brnd=b, **kw), write_grid(d, brnd=b, **kw), label="after-nan")
