@@ -28,9 +28,7 @@
 // at a time over two complex arrays), 72 instead of 280 for mhd, 72 instead of
 // 144 for te.  Measured per realisation, whole-array steps -> these (with the
 // engine and table work below): es 256x256x64 726 -> 304 us, es 512x512x128
-// 7.05 -> 2.24 ms, te 800x800x160 7.90 -> 2.71 ms, mhd 135x121x98 344 -> 122 us.  Distance from a 64-bit
-// reference 1.0e-15 -> 1.2e-15 to 3e-15: the rounding errors of a vertex and
-// its mirror now coincide instead of averaging in the extraction.
+// 7.05 -> 2.24 ms, te 800x800x160 7.90 -> 2.71 ms, mhd 135x121x98 344 -> 122 us.
 //
 // Half arrays: H[i][j][k], i <= nx/2, all j, k <= nz/2.  Two real lines share
 // one complex transform: X + i U in one, V in the other.
@@ -353,9 +351,13 @@ __device__ inline void store_half_columns(const double2 *lds, const HalfArrays &
 }
 
 // x(-), Gram-Schmidt (brnd_es.cc:211-259) of the real even k-space vector,
-// the even part of the result, x(+).  The vector is the same at k and -k; the
-// results differ only where an index is half its axis length, whose wave
-// number keeps its sign at the mirror.
+// the even part of the result, x(+).  The vector is the same at k and -k, the
+// results are not: a wave number beyond half its axis is i/L - n/L, which
+// carries the rounding of n/L that its mirror's does not, and at half the axis it
+// keeps its sign.  Each wave vector gives a result of its own and both enter the
+// even part (with k's alone es 512x512x128 was 2.2e-15 to 3.0e-15 from a 64-bit
+// reference, with both it is 1.0e-15, as the whole-array steps).  The wave numbers
+// along x are formed once per workgroup, in LDS behind the engine's tables.
 template <uint32_t TILE, uint32_t NT, int MODE>
 __global__ __launch_bounds__(NT) void k_es_gs_x(HalfArrays H, EsArgs a, HalfArgs h, FftLine L,
                                                 uint32_t cs) {
@@ -369,26 +371,25 @@ __global__ __launch_bounds__(NT) void k_es_gs_x(HalfArrays H, EsArgs a, HalfArgs
   const uint32_t col = col0 + c;
   const bool on = col < h.ncol;
   load_half_columns<TILE, NT>(lds, H, h, cs, col, on);
+  double *kx = reinterpret_cast<double *>(lds) +
+               2 * (L.len * P + (fft_lds_tw<TILE, MODE>() ? L.len : 0));
+  for (uint32_t t = threadIdx.x; t < n; t += NT)
+    kx[t] = wavenum(t, n, a.b.lx);
   __syncthreads();
   fft_lines<-1, TILE, NT, MODE>(lds, twl, L, cs + 1, P);
   const uint32_t j = col / h.nh, l = col - j * h.nh;
   const uint32_t js = mirror_of(j, h.ny), ls = mirror_of(l, h.nz);
   Vec3 k{0., wavenum(j, h.ny, a.b.ly), wavenum(l, h.nz, a.b.lz)};
   Vec3 ks{0., wavenum(js, h.ny, a.b.ly), wavenum(ls, h.nz, a.b.lz)};
-  const bool edge = 2 * j == h.ny || 2 * l == h.nz;
 #pragma unroll 1
   for (uint32_t t = t0; t < n; t += dt) {
     double2 &z = lds[t * P + c], &zv = lds[t * P + C + c];
     const Vec3 b{z.x, z.y, zv.x};
-    k.x = wavenum(t, n, a.b.lx);
-    Vec3 f = es_gs(a, k, b);
-    if (edge || 2 * t == n) {
-      ks.x = wavenum(mirror_of(t, n), n, a.b.lx);
-      const Vec3 fs = es_gs(a, ks, b);
-      f = Vec3{0.5 * (f.x + fs.x), 0.5 * (f.y + fs.y), 0.5 * (f.z + fs.z)};
-    }
-    z = make_double2(cgs::sqrtwo * f.x, cgs::sqrtwo * f.y);
-    zv = make_double2(cgs::sqrtwo * f.z, 0.);
+    k.x = kx[t];
+    ks.x = kx[mirror_of(t, n)];
+    const Vec3 f = es_gs(a, k, b), fs = es_gs(a, ks, b);
+    z = make_double2(cgs::sqrtwo * (0.5 * (f.x + fs.x)), cgs::sqrtwo * (0.5 * (f.y + fs.y)));
+    zv = make_double2(cgs::sqrtwo * (0.5 * (f.z + fs.z)), 0.);
   }
   __syncthreads();
   fft_lines<1, TILE, NT, MODE>(lds, twl, L, cs + 1, P);
@@ -726,7 +727,8 @@ inline int half_gs_x(hamx_ctx *ctx, const HalfPlan &p, const HalfArrays &H, cons
   with_tile(tile, p.lx.mode, [&](auto T, auto NT, auto M) {
     hipLaunchKernelGGL((k_es_gs_x<decltype(T)::value, decltype(NT)::value, decltype(M)::value>),
                        dim3(xcd_grid((h.ncol + (1u << cs) - 1) >> cs)), dim3(decltype(NT)::value),
-                       fft_lds_bytes(p.lx, 2u << cs, tile), ctx->stream, H, a, h, p.lx, cs);
+                       fft_lds_bytes(p.lx, 2u << cs, tile) + p.lx.n * sizeof(double),
+                       ctx->stream, H, a, h, p.lx, cs);
   });
   HAMX_HIP(ctx, hipGetLastError());
   return HAMX_OK;
