@@ -397,11 +397,11 @@ __global__ __launch_bounds__(NT) void k_es_gs_x(HalfArrays H, EsArgs a, HalfArgs
 }
 
 // Brnd_mhd's modes, their even part (the only part the extraction keeps) and
-// x(+).  k and -k share the spectrum, so a pair evaluates it once, except where
-// an index is half its axis length (the wave number keeps its sign at the
-// mirror) or the two |k|, which may differ in rounding, lie in different bands.  Bound by FP64 instructions: mhd
-// 135x121x98 149 -> 62 us with that, the spectra as powers of |k|^2 and no
-// library pow.
+// x(+).  A mode and its mirror are evaluated each with its own wave vector (see
+// k_es_gs_x; one spectrum for both, 121 instead of 125 us a realisation of
+// 135x121x98, was 2.9e-15 instead of 6.5e-16 from a 64-bit reference).  Bound by
+// FP64 instructions: mhd 135x121x98 149 -> 66 us with the spectra as powers of
+// |k|^2 and no library pow.
 template <uint32_t TILE, uint32_t NT, int MODE>
 __global__ __launch_bounds__(NT) void k_mhd_x(HalfArrays H, MhdArgs a, uint64_t seed,
                                               const double *__restrict__ bobs, HalfArgs h,
@@ -420,7 +420,6 @@ __global__ __launch_bounds__(NT) void k_mhd_x(HalfArrays H, MhdArgs a, uint64_t 
   const uint32_t js = mirror_of(j, h.ny), ls = mirror_of(l, h.nz);
   Vec3 k{0., wavenum(j, h.ny, a.b.ly), wavenum(l, h.nz, a.b.lz)};
   Vec3 ks{0., wavenum(js, h.ny, a.b.ly), wavenum(ls, h.nz, a.b.lz)};
-  const bool edge = 2 * j == h.ny || 2 * l == h.nz;
   double *kx = reinterpret_cast<double *>(lds) +
                2 * (L.len * P + (fft_lds_tw<TILE, MODE>() ? L.len : 0));
   for (uint32_t t = threadIdx.x; t < n; t += NT)
@@ -437,15 +436,11 @@ __global__ __launch_bounds__(NT) void k_mhd_x(HalfArrays H, MhdArgs a, uint64_t 
       ks.x = kx[ts];
       const double x = k.x * k.x + k.y * k.y + k.z * k.z;
       const double xs = ks.x * ks.x + ks.y * ks.y + ks.z * ks.z;
-      const int in = a.bands.of(x), ins = a.bands.of(xs);
       MhdShape m = mhd_shape(a, bh, k);
-      const bool generic = m.generic;
-      MhdPower p = mhd_power(a, x, in, m.c);
-      f = mhd_field(seed, m, p, k, x, idx, t == 0 && j == 0);
+      f = mhd_field(seed, m, mhd_power(a, x, a.bands.of(x), m.c), k, x, idx, t == 0 && j == 0);
       m = mhd_shape(a, bh, ks);
-      if (edge || 2 * t == n || in != ins || !generic || !m.generic)
-        p = mhd_power(a, xs, ins, m.c);
-      const Vec3 s = mhd_field(seed, m, p, ks, xs, sym, t == 0 && j == 0);
+      const Vec3 s = mhd_field(seed, m, mhd_power(a, xs, a.bands.of(xs), m.c), ks, xs, sym,
+                               t == 0 && j == 0);
       f = Vec3{f.x + s.x, f.y + s.y, f.z + s.z};
     }
     lds[t * P + c] = make_double2(0.5 * f.x, 0.5 * f.y);

@@ -99,12 +99,16 @@ def test_dft_profile_routes(ctx, z0):
     compare(ctx.ternd_dft, load_oracle().orc_ternd_dft, d, 6, shape, 1)
 
 
-@pytest.mark.parametrize("shape", SHAPES)
-def test_mhd(ctx, shape):
+def mhd(shape):
     d = fill(capi.HamxMhdDesc(), shape)
     d.pa0 = d.pf0 = d.ps0 = 1e-12
     d.k0, d.k1, d.aa0, d.af0, d.as0, d.a1, d.beta, d.ma = 0.3, 0.1, 1.7, 1.5, 1.7, 0.0, 0.1, 0.5
-    compare(ctx.brnd_mhd, load_oracle().orc_brnd_mhd, d, 7, shape, 3)
+    return d
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+def test_mhd(ctx, shape):
+    compare(ctx.brnd_mhd, load_oracle().orc_brnd_mhd, mhd(shape), 7, shape, 3)
 
 
 # Wave numbers beyond half of an axis carry the rounding of n/L: on an axis of
@@ -119,3 +123,9 @@ WAVE = [(4096, 4, 6), (6, 4000, 4), (4, 6, 1000)]
 def test_es_takes_each_wave_vector(ctx, shape):
     print("case: es wave vectors", shape, flush=True)
     compare(ctx.brnd_es, load_oracle().orc_brnd_es, es(shape, 1.3), 5, shape, 3, bound=6e-15)
+
+
+@pytest.mark.parametrize("shape", WAVE)
+def test_mhd_takes_each_wave_vector(ctx, shape):
+    print("case: mhd wave vectors", shape, flush=True)
+    compare(ctx.brnd_mhd, load_oracle().orc_brnd_mhd, mhd(shape), 5, shape, 3, bound=6e-15)
