@@ -176,11 +176,23 @@ static KEdge k_edge(double k) {
   return KEdge{last(true), std::isinf(k) && k > 0 ? INFINITY : last(false)};
 }
 
-// A power of |k| as coef * x^e, x = |k|^2: one logarithm and one exponential.
+// A power of |k| as coef * y^e, y = |k|^2 / kn^2: one logarithm and one
+// exponential.  kn is the spectrum's k0, so that the logarithm, whose rounding
+// the exponent multiplies, is small for the modes that carry the power (in
+// units of 1/kpc instead the standard deviations were 2.3e-16 off, weighted by
+// power; now 1.5e-16).
 struct KPower {
   double coef, e;
-  __device__ double at(double lnx) const { return coef * exp_fast(e * lnx); }
+  __device__ double at(double lny) const { return coef * exp_fast(e * lny); }
 };
+
+static double k_norm(double k0) { return k0 > 1e-100 && k0 < 1e100 ? k0 : 1.; }
+
+// (|k| / k0)^(-a / 2) / |k|
+static KPower k_power(double k0, double a) {
+  const double kn = k_norm(k0);
+  return KPower{std::pow(k0 / kn, 0.5 * a) / kn, -0.25 * (a + 2.)};
+}
 
 // Vertex position (brnd_es.cc:165-173: vertex spacing L/(n-1)).
 __device__ inline Vec3 vertex_pos(const BoxArgs &a, uint64_t i, uint64_t j,
@@ -212,15 +224,16 @@ __device__ inline uint64_t sym_index(const BoxArgs &a, uint64_t idx) {
 // k1 > k0 the low and the high band overlap and their powers add.
 struct KBands {
   KEdge k0, k1;
+  double inv_kn2; // y = x inv_kn2
   double low;
   KPower mid, high;
   // bits of the bands that x lies in: 1 low, 2 mid, 4 high
   __device__ int of(double x) const {
     return (x <= k1.lt ? 1 : 0) | (x > k0.le ? 4 : (x > k1.le && x <= k0.lt) ? 2 : 0);
   }
-  __device__ double amp(int bands, double x, double lnx, const KPower &hi) const {
+  __device__ double amp(int bands, double x, double lny, const KPower &hi) const {
     const double lo = bands & 1 ? low * x : 0.;
-    const double v = bands & 6 ? (bands & 4 ? hi : mid).at(lnx) : 0.;
+    const double v = bands & 6 ? (bands & 4 ? hi : mid).at(lny) : 0.;
     return lo != 0. && v != 0. ? sqrt(lo * lo + v * v) : lo + v;
   }
 };
@@ -230,7 +243,8 @@ static KBands k_bands(double k0, double k1, double a1) {
   b.k0 = k_edge(k0);
   b.k1 = k_edge(k1);
   b.low = std::sqrt(std::pow(k0 / k1, a1)) / (k1 * k1 * k1);
-  b.mid = KPower{std::pow(k0, 0.5 * a1), -0.25 * (a1 + 2.)};
+  b.inv_kn2 = 1. / (k_norm(k0) * k_norm(k0));
+  b.mid = k_power(k0, a1);
   b.high = KPower{0., 0.};
   return b;
 }
@@ -323,7 +337,7 @@ struct EsArgs {
 // with the constants folded on the host.
 __device__ inline double es_sigma(const EsArgs &a, double x) {
   const int in = a.bands.of(x);
-  return a.bands.amp(in, x, in & 6 ? log_pos(x) : 0., a.bands.high);
+  return a.bands.amp(in, x, in & 6 ? log_pos(x * a.bands.inv_kn2) : 0., a.bands.high);
 }
 
 static void es_bands(EsArgs &a, const hamx_es_desc *d) {
@@ -331,7 +345,8 @@ static void es_bands(EsArgs &a, const hamx_es_desc *d) {
   a.bands = k_bands(d->k0, d->k1, d->a1);
   a.bands.low *= p;
   a.bands.mid.coef *= p;
-  a.bands.high = KPower{p * std::pow(d->k0, 0.5 * d->a0), -0.25 * (d->a0 + 2.)};
+  a.bands.high = k_power(d->k0, d->a0);
+  a.bands.high.coef *= p;
 }
 
 // Brnd_jf12::spatial_profile (brnd_jf12.cc:54-114): the squared disk (JF12
@@ -637,13 +652,14 @@ struct DftArgs {
   Vec3 obs;
   double rms, r0, z0;
   KEdge k0;
+  double inv_kn2;
   KPower amp; // above k0
 };
 
 // The standard deviation of the components of a mode at x = |k|^2, the
 // square root of rms (k / k0)^a0 dk3 / (4 pi k^2) (ternd_dft.cc:17-24,71-78).
 __device__ inline double dft_sigma(const DftArgs &a, double x) {
-  return x <= a.k0.lt ? 0. : a.amp.at(log_pos(x));
+  return x <= a.k0.lt ? 0. : a.amp.at(log_pos(x * a.inv_kn2));
 }
 
 __global__ __launch_bounds__(256) void k_dft_draw(double2 *tk, DftArgs a,
@@ -781,13 +797,13 @@ struct MhdPower {
 
 // x = |k|^2, bands = a.bands.of(x), c the cosine to the regular field.
 __device__ inline MhdPower mhd_power(const MhdArgs &a, double x, int bands, double c) {
-  const double lnx = bands & 6 ? log_pos(x) : 0.;
+  const double lny = bands & 6 ? log_pos(x * a.bands.inv_kn2) : 0.;
   // sqrt of exp(-ma^(-4/3) |c| / (1 - c^2)^(1/3))
   const double third = exp_fast(-0.33333333 * log_pos(fmax(1. - c * c, 1e-300)));
   const double an = exp_fast(fmax(-a.half_ma * fabs(c) * third, -745.));
-  const double pa = a.bands.amp(bands, x, lnx, a.ha);
-  return MhdPower{a.ca * pa * an, a.cf * a.bands.amp(bands, x, lnx, a.hf),
-                  a.cs * (a.same_as ? pa : a.bands.amp(bands, x, lnx, a.hs)) * an};
+  const double pa = a.bands.amp(bands, x, lny, a.ha);
+  return MhdPower{a.ca * pa * an, a.cf * a.bands.amp(bands, x, lny, a.hf),
+                  a.cs * (a.same_as ? pa : a.bands.amp(bands, x, lny, a.hs)) * an};
 }
 
 // A mode's versors e_plus and e_minus (brnd_mhd.cc:169-179) and the square
@@ -1083,10 +1099,9 @@ int brnd_mhd(hamx_ctx *ctx, const hamx_mhd_desc *d, uint64_t seed, double *bx, d
   a.ca = std::sqrt(c * d->pa0);
   a.cf = std::sqrt(c * d->pf0);
   a.cs = std::sqrt(c * d->ps0);
-  auto above = [&](double e) { return KPower{std::pow(d->k0, 0.5 * e), -0.25 * (e + 2.)}; };
-  a.ha = above(d->aa0);
-  a.hf = above(d->af0);
-  a.hs = above(d->as0);
+  a.ha = k_power(d->k0, d->aa0);
+  a.hf = k_power(d->k0, d->af0);
+  a.hs = k_power(d->k0, d->as0);
   a.same_as = d->aa0 == d->as0;
   a.beta = d->beta;
   a.half_ma = 0.5 * std::pow(d->ma, -1.33333333);
@@ -1164,8 +1179,9 @@ extern "C" int hamx_ternd_dft(hamx_ctx *ctx, const hamx_dft_desc *d, uint64_t se
   a.obs = Vec3{d->observer[0], d->observer[1], d->observer[2]};
   a.rms = d->rms;
   a.k0 = k_edge(d->k0);
-  a.amp = KPower{std::sqrt(d->rms * a.b.dk3 / (4. * cgs::pi)) * std::pow(d->k0, -0.5 * d->a0),
-                 0.25 * (d->a0 - 2.)};
+  a.inv_kn2 = 1. / (k_norm(d->k0) * k_norm(d->k0));
+  a.amp = k_power(d->k0, -d->a0);
+  a.amp.coef *= std::sqrt(d->rms * a.b.dk3 / (4. * cgs::pi));
   a.r0 = d->r0;
   a.z0 = d->z0;
   const uint64_t n = a.b.n;

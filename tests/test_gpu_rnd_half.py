@@ -129,3 +129,29 @@ def test_es_takes_each_wave_vector(ctx, shape):
 def test_mhd_takes_each_wave_vector(ctx, shape):
     print("case: mhd wave vectors", shape, flush=True)
     compare(ctx.brnd_mhd, load_oracle().orc_brnd_mhd, mhd(shape), 5, shape, 3, bound=6e-15)
+
+
+@pytest.mark.parametrize("gen", ["es", "dft", "mhd"])
+def test_spectra_far_from_one_per_kpc(ctx, gen):
+    """Spectra of boxes 1e20 times as large: |k| enters relative to k0, so the
+    rounding of its logarithm (1.4e-14 once multiplied by the exponent, were it
+    taken in 1/kpc) leaves the sums' 3e-15 alone."""
+    shape, big = (24, 20, 16), 1e20
+    orc = load_oracle()
+    if gen == "es":
+        d = es(shape, 1.0)
+        d.k0, d.k1, d.a0, d.a1 = 0.12 / big, 0.06 / big, 3.7, 0.5
+        call, ref, outs = ctx.brnd_es, orc.orc_brnd_es, 3
+    elif gen == "dft":
+        d = fill(capi.HamxDftDesc(), shape)
+        d.rms, d.k0, d.a0, d.r0, d.z0 = 1e-3, 0.02 / big, -3.7, 8 * CGS.kpc, 1 * CGS.kpc
+        call, ref, outs = ctx.ternd_dft, orc.orc_ternd_dft, 1
+    else:
+        d = mhd(shape)
+        d.k0, d.k1, d.aa0, d.af0, d.as0 = 0.3 / big, 0.1 / big, 3.7, 3.5, 3.7
+        call, ref, outs = ctx.brnd_mhd, orc.orc_brnd_mhd, 3
+    for f in ("x_min", "x_max", "y_min", "y_max", "z_min", "z_max"):
+        setattr(d.box, f, getattr(d.box, f) * big)
+    if gen != "mhd":
+        d.r0, d.z0 = d.r0 * big, d.z0 * big
+    compare(call, ref, d, 8, shape, outs, bound=6e-15)
