@@ -809,7 +809,8 @@ __device__ inline MhdPower mhd_power(const MhdArgs &a, double x, int bands, doub
 // A mode's versors e_plus and e_minus (brnd_mhd.cc:169-179) and the square
 // roots of h_f and h_s; `generic` false for modes (nearly) along the regular
 // field bh: e_plus is normalised unless its squared length is below 1e-12, and
-// then fails the generic branch's dot(e_plus, e_plus) > 1e-6.
+// then fails the generic branch's dot(e_plus, e_plus) > 1e-6.  Its components,
+// and e_minus's, stay as they are there.
 struct MhdShape {
   Vec3 ep, em;
   double c, hf, hs;
@@ -825,12 +826,11 @@ __device__ inline MhdShape mhd_shape(const MhdArgs &a, const Vec3 &bh, const Vec
   m.c = m.generic ? dot0(bh, kh) : 1.;
   const double sq = sqrt(mhd_dynamo(a.beta, m.c));
   m.hf = sqrt_pos(mhd_h_f(a.beta, sq, m.c));
-  if (m.generic) {
-    const double il = rsqrt_f64(l2);
-    m.ep = Vec3{kxb.x * il, kxb.y * il, kxb.z * il};
-    m.em = cross3(m.ep, kh);
+  const double il = m.generic ? rsqrt_f64(l2) : 1.;
+  m.ep = Vec3{kxb.x * il, kxb.y * il, kxb.z * il};
+  m.em = cross3(m.ep, kh);
+  if (m.generic)
     m.hs = sqrt_pos(mhd_h_s(a.beta, sq, m.c));
-  }
   return m;
 }
 
@@ -845,8 +845,8 @@ __device__ inline Vec3 mhd_field(uint64_t seed, const MhdShape &m, const MhdPowe
     return Vec3{m.ep.x * Ap + m.em.x * Am, m.ep.y * Ap + m.em.y * Am,
                 m.ep.z * Ap + m.em.z * Am};
   }
-  Vec3 ep{0., 0., 0.}, em{0., 0., 0.}; // along the field: below 1e-6 before
-  if (pole) {                          // i == 0 and j == 0
+  Vec3 ep = m.ep, em = m.em;
+  if (pole) { // i == 0 and j == 0
     ep.x = k.x;
     em.y = k.y;
   } else {

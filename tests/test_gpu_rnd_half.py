@@ -155,3 +155,16 @@ def test_spectra_far_from_one_per_kpc(ctx, gen):
     if gen != "mhd":
         d.r0, d.z0 = d.r0 * big, d.z0 * big
     compare(call, ref, d, 8, shape, outs, bound=6e-15)
+
+
+@pytest.mark.parametrize("half", [True, False])
+@pytest.mark.parametrize("tilt", [0.0, 3e-7, 3e-6])
+def test_mhd_along_the_field(ctx, tilt, half):
+    """Modes along a regular field that is off the z axis by less than 1e-6 (their
+    versors' small components stay), exactly on it, or by enough to count as
+    across it; half-space passes and whole-array steps."""
+    shape = (6, 4, 10) if half else (3, 2, 1100)
+    d = mhd(shape)
+    d.breg_model = capi.HAMX_BREG_CART
+    d.breg[0:3] = [tilt * 2e-6, -0.4 * tilt * 2e-6, 2e-6]
+    compare(ctx.brnd_mhd, load_oracle().orc_brnd_mhd, d, 9, shape, 3)
