@@ -156,17 +156,17 @@ __device__ inline void sincos_fast(double x, double &s, double &c) {
   }
 }
 
-// sqrt(x) for x >= 0 below 2^1000, within 1 ulp: the v_rsq_f64 estimate and
-// two coupled Newton steps for the root and half its reciprocal, without the
-// library's scaling of tiny arguments (below 2^-1000 the result is 2^-500).
+// sqrt(x) for x below 2^1000, within 1 ulp from 2^-1000 on (less exact in the
+// subnormals), 0 for 0 and NaN below it: the v_rsq_f64 estimate and two coupled
+// Newton steps for the root and half its reciprocal, without the library's
+// scaling of tiny and huge arguments.
 __device__ inline double sqrt_pos(double x) {
-  x = fmax(x, 0x1p-1000);
   const double y = __builtin_amdgcn_rsq(x);
   double g = x * y, h = 0.5 * y;
   const double e = fma(-h, g, 0.5);
   g = fma(g, e, g);
   h = fma(h, e, h);
-  return fma(fma(-g, g, x), h, g);
+  return x == 0. ? x : fma(fma(-g, g, x), h, g);
 }
 
 // sin and cos of 2 pi u for 0 <= u < 1: the quadrant and the angle within it

@@ -168,3 +168,11 @@ def test_mhd_along_the_field(ctx, tilt, half):
     d.breg_model = capi.HAMX_BREG_CART
     d.breg[0:3] = [tilt * 2e-6, -0.4 * tilt * 2e-6, 2e-6]
     compare(ctx.brnd_mhd, load_oracle().orc_brnd_mhd, d, 9, shape, 3)
+
+
+def test_mhd_modes_without_power(ctx):
+    """A fast mode whose h_f is 0 stays exactly 0, however large its norm (here
+    every one, by a plasma beta without an h_f; sqrt(norm) = 1e150)."""
+    d = mhd((12, 10, 8))
+    d.beta, d.pf0 = np.nan, 1e300
+    compare(ctx.brnd_mhd, load_oracle().orc_brnd_mhd, d, 10, (12, 10, 8), 3)
