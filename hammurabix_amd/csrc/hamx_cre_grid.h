@@ -55,7 +55,7 @@ __device__ inline void cre_grid_emissivity(const Phys &ph, const Grids &gr, cons
   // the first pair of bins that any lane keeps (uniform: the energy loop then
   // reads its tables with scalar loads)
   uint32_t q = 0;
-  while (2 * q + 2 < nE && !__ballot(xf * tc[2 * q + 2 < nE - 1 ? 2 * q + 1 : nE - 2] <= 100.))
+  while (2 * q + 2 < nE && !__ballot(xf * tc[2 * q + 1] <= 100.))
     ++q;
   if (2 * q + 1 >= nE)
     return; // uniform: no bin is kept
@@ -89,33 +89,39 @@ __device__ inline void cre_grid_emissivity(const Phys &ph, const Grids &gr, cons
     g0 *= tb[at];
     g1 *= tb[at + 1];
   };
-  // F and G of a bin times half its width, 0 where it is skipped
+  // F and G of a bin times half its width; false where the bin is skipped
   auto kernels = [&](uint32_t i, double &F, double &G) {
     const double x = xf * tc[i];
     sync_fg(stab, lx + tl[i], x, F, G);
     const double m = td[i];
-    F = x > 100. ? 0. : F * m;
-    G = x > 100. ? 0. : G * m;
+    F *= m;
+    G *= m;
+    return !(x > 100.);
+  };
+  double Jt = 0., Jp = 0.;
+  // a skipped bin's flux, which may be infinite or NaN, takes no part
+  auto add = [&](bool on, double F, double G, double flux) {
+    Jt = on ? fma(F, flux, Jt) : Jt;
+    Jp = on ? fma(G, flux, Jp) : Jp;
   };
   double F, G;
   load(2 * q);
-  kernels(2 * q, F, G);
+  bool on = kernels(2 * q, F, G);
   lerp(2 * q);
-  double Jt = F * (g0 + g1), Jp = G * (g0 + g1), last = g1;
+  add(on, F, G, g0 + g1);
+  double last = g1;
   // the loads of a step are in flight while its two bins' kernels, which do
   // not depend on them, are evaluated
   for (uint32_t e = 2 * q + 2; e < nE; e += 2) {
     double F2 = 0., G2 = 0.;
+    bool on2 = false;
     load(e);
-    kernels(e - 1, F, G);
+    on = kernels(e - 1, F, G);
     if (e + 1 < nE)
-      kernels(e, F2, G2);
+      on2 = kernels(e, F2, G2);
     lerp(e);
-    const double first = e + 1 < nE ? g0 : g1;
-    Jt = fma(F, last + first, Jt);
-    Jp = fma(G, last + first, Jp);
-    Jt = fma(F2, g0 + g1, Jt);
-    Jp = fma(G2, g0 + g1, Jp);
+    add(on, F, G, last + (e + 1 < nE ? g0 : g1));
+    add(on2, F2, G2, g0 + g1);
     last = g1;
   }
   const double fore = ph.fore_num * ab / ph.fore_den;

@@ -123,6 +123,51 @@ def test_los_with_cre_grid_matches_oracle(ctx, sched):
     assert np.linalg.norm(ref["is"]) > 0 and np.linalg.norm(ref["qs"]) > 0
 
 
+@pytest.mark.parametrize("sched", [capi.HAMX_SCHED_THREAD, capi.HAMX_SCHED_WAVE,
+                                   capi.HAMX_SCHED_AUTO])
+@pytest.mark.parametrize("bad", [np.inf, np.nan])
+@pytest.mark.parametrize("nE", [16, 17])
+def test_flux_of_skipped_bins_is_not_read(ctx, nE, bad, sched):
+    """Fluxes that are not finite at the energies whose bins every sample skips
+    (x > 100): the lowest ones everywhere, and all of them where the field is
+    all but zero, beside samples of the same wavefront that keep their bins."""
+    par = Param(text=configs.plain_forward(nside_sim=2, nside_out=2, oc_r_res=0.2, freqs=[23.0]))
+    d = par.los_desc(schedule=sched)
+    d.cre_model = capi.HAMX_CRE_GRID
+    d.breg_model = capi.HAMX_BREG_GRID
+    box = capi.HamxBox(41, 4, 4, -20 * KPC, 20 * KPC, -20 * KPC, 20 * KPC, -4 * KPC, 4 * KPC)
+    x = np.linspace(-20, 20, 41)[:, None, None] + np.zeros((41, 4, 4))
+    bz = np.where(x < 0, 2e-5, 1e-16).ravel()
+    breg = (np.zeros_like(bz), np.zeros_like(bz), bz)
+    flux = np.ones((41, 4, 4, nE)) * np.geomspace(1.0, 1e-6, nE)
+    kw = dict(breg=breg, breg_box=box, cre_box=box,
+              cre_E=(0.05 * CGS.GeV, math.log(1e3) / (nE - 1), nE))
+
+    def ref(f):
+        m = write_grid(d, cre=np.ascontiguousarray(f.ravel()), **kw)
+        return m if all(np.all(np.isfinite(v)) for v in m.values()) else None
+
+    flux[x >= 3] = bad  # no bin is kept from x = 1 kpc on
+    assert ref(flux) is not None
+    low = 0
+    while low < nE:  # every energy that no sample reads
+        f = flux.copy()
+        f[..., low] = bad
+        if ref(f) is None:
+            break
+        flux, low = f, low + 1
+    assert 2 < low < nE - 2
+    for skip in (low, low - 1):  # of either parity
+        f = flux.copy()
+        f[x < 3, skip:low] = 1.0
+        want = ref(f)
+        assert np.linalg.norm(want["is"]) > 0
+        got = maps_for(d)
+        ctx.los_forward(d, got, cre=np.ascontiguousarray(f.ravel()), **kw)
+        for k in want:
+            assert rel_l2(got[k], want[k]) <= 1e-10, (k, skip)
+
+
 def test_cre_grid_errors(ctx):
     par = Param(text=configs.plain_forward(nside_sim=4, nside_out=4, oc_r_res=0.5))
     d = par.los_desc()
