@@ -46,14 +46,22 @@ def _trap(weight, x):
     return np.longdouble(x) * H * (f.sum() - f[0] / 2)
 
 
-def target_p(u):
+def sum_p(u):
     x = np.exp(np.longdouble(u))
-    return float(np.log(_trap(W_F, x)) + x)
+    return np.log(_trap(W_F, x)) + x
+
+
+def ratio_r(u):
+    x = np.exp(np.longdouble(u))
+    return _trap(W_G, x) / _trap(W_F, x)
+
+
+def target_p(u):
+    return float(sum_p(u))
 
 
 def target_r(u):
-    x = np.exp(np.longdouble(u))
-    return float(_trap(W_G, x) / _trap(W_F, x))
+    return float(ratio_r(u))
 
 
 def segments():

@@ -2,7 +2,7 @@
 // replacing gsl_sf_synchrotron_1 / _2 (integrator.cc:321,390):
 //   F(x) = x int_x^inf K_5/3(t) dt,   G(x) = x K_2/3(x),   0 < x <= 100.
 // F = exp(P(u) - x) and G = F R(u), with P(u) = ln F + x and R(u) = G / F in
-// u = ln x.  From u = ln 100 down to ln 100 - 18 (x = 1.5e-6) both are degree-7
+// u = ln x.  From u = ln 100 down to ln 100 - 18 (x = 1.5e-6) both are degree-8
 // polynomials on segments of width 1/4 (hamx_sync_fine.h), below that piecewise
 // Chebyshev series (hamx_synchrotron.h: 12 segments of width 4, one Clenshaw
 // loop for both series); below the last segment (x < 1.8e-23) F is its leading
