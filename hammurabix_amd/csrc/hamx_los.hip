@@ -183,13 +183,13 @@ __device__ inline bool eval_sample(const Phys &ph, const Grids &gr,
 // (integrator.cc:99-115).  A NaN or an infinity in an input grid or parameter
 // reaches a ray's values (the reference's debug build asserts isfinite on
 // B_par, B_per, te and the phase, integrator.cc:192,195,202,223; its release
-// build carries the NaN).  FLAG (k_los_ray, whose small shells cost their
-// launches) raises the pass's flag here, where they are at hand; behind the
-// other marches k_nonfinite reads the shell maps, 17 us for three shells up to
-// nside 256: the flag's pointer, held over their sample loops in two more
-// scalar registers, cost them 105 us in spilled scalars read back (a pass of
-// 256x256x64 random grids 5.47 -> 5.34 ms, an analytic one at nside 32 261 ->
-// 246 us without it).
+// build carries the NaN).  FLAG raises the pass's flag here, where they are at
+// hand.  Behind k_los_fast k_nonfinite reads the shell maps instead, 17 us for
+// three shells up to nside 256: the flag's pointer, held over its sample loop in
+// two more scalar registers, cost 105 us in spilled scalars read back (a pass of
+// 256x256x64 random grids 5.47 -> 5.34 ms, an analytic one at nside 32 261 -> 246
+// us without it).  k_los_ray's small shells cost their launches, and the generic
+// marches lose nothing to the flag (15.0 ms a pass, 15.2 with the scan).
 template <bool FLAG>
 __device__ inline void store_ray(const Phys &ph, const ShellArgs &sa,
                                  uint64_t ipix, double dm, double fd, double I,
@@ -247,7 +247,7 @@ k_los_wave(Phys ph, Grids gr, ShellArgs sa) {
       static_cast<uint64_t>(blockIdx.x) * (blockDim.x >> 6) + (threadIdx.x >> 6);
   if (ipix >= sa.hs.npix)
     return; // uniform per wavefront
-  if (masked_out<false>(ph, sa, ipix, lane == 0))
+  if (masked_out<true>(ph, sa, ipix, lane == 0))
     return; // uniform per wavefront
   RayGeo r;
   ray_setup(ph, sa, ipix, r);
@@ -283,7 +283,7 @@ k_los_wave(Phys ph, Grids gr, ShellArgs sa) {
   Q = wave_sum(Q);
   U = wave_sum(U);
   if (lane == 0)
-    store_ray<false>(ph, sa, ipix, dm, fd, I, Q, U);
+    store_ray<true>(ph, sa, ipix, dm, fd, I, Q, U);
 }
 
 // ---------------------------------------------------- specialised march --
@@ -463,7 +463,7 @@ k_los_thread(Phys ph, Grids gr, ShellArgs sa) {
   const uint64_t ipix = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   if (ipix >= sa.hs.npix)
     return;
-  if (masked_out<false>(ph, sa, ipix, true))
+  if (masked_out<true>(ph, sa, ipix, true))
     return;
   RayGeo r;
   ray_setup(ph, sa, ipix, r);
@@ -483,7 +483,7 @@ k_los_thread(Phys ph, Grids gr, ShellArgs sa) {
       U += sin(2. * qui) * s.jp;
     }
   }
-  store_ray<false>(ph, sa, ipix, dm, fd, I, Q, U);
+  store_ray<true>(ph, sa, ipix, dm, fd, I, Q, U);
 }
 
 // ------------------------------------------------------------- accumulate --
@@ -1080,7 +1080,7 @@ int los_forward_impl(hamx_ctx *ctx, const hamx_los_desc *d, const hamx_fields *f
     if (ckpt && d->do_fd && s > 0) // FD map before shell s, for the adjoint
       HAMX_HIP(ctx, hipMemcpyAsync(ckpt + s * h_fd.npix, o_fd, h_fd.npix * sizeof(double),
                                    hipMemcpyDeviceToDevice, ctx->stream));
-    bool scan = true; // the march leaves the flag to k_nonfinite
+    bool scan = false; // the march leaves the flag to k_nonfinite
     ProfMark pm = prof_begin(ctx);
     if (fast) {
       const FastConst fc = make_fast(d, ph, sa.delta, pw1);
