@@ -109,7 +109,7 @@ __attribute__((amdgpu_waves_per_eu(MODELS ? 1 : 3))) void k_los_adj(Phys ph, Fas
     FastSample o;
     bool valid = false;
     if (k < r.k_hi)
-      valid = eval_fast<GRIDS, PW1, MODELS ? kAllModels : kLsaUnif>(ph, fc, gr, sa, r, k, o);
+      valid = eval_fast<GRIDS, PW1, MODELS ? kAnyModels : kLsaUnif>(ph, fc, gr, sa, r, k, o);
     const double incl = wave_incl_scan(valid ? o.fdk : 0., lane);
     const double chunk = wave_last(incl);
     const double fd_here = (fd_total - after - chunk) + incl;

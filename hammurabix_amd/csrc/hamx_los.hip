@@ -56,6 +56,12 @@ struct SampleOut {
   double ipa;  // intrinsic polarisation angle
 };
 
+// Regular fields and electrons compiled into a generic march: the light ones;
+// JF12, Jaffe and YMW16's short form too; those with YMW16's literal form.  Each
+// in kernels of its own (register use: with both forms of YMW16 a pass took 8.1 ms
+// instead of 7.8).
+enum Heavy { kLight = 0, kHeavy = 1, kHeavyLiteral = 2 };
+
 // CRE_ana / CRE_unif spatial profile (cre_ana.cc:11-19, cre_unif.cc)
 __device__ inline double cre_profile(const Phys &ph, const Vec3 &pos) {
   if (ph.cre_model == HAMX_CRE_ANA) {
@@ -74,7 +80,7 @@ __device__ inline double cre_index(const Phys &ph, const Vec3 &pos) {
   return -ph.cre[0] + ph.cre[1] * r + ph.cre[2] * z;
 }
 
-template <bool PACKED, bool CREG, bool HEAVY>
+template <bool PACKED, bool CREG, Heavy HEAVY>
 __device__ inline bool eval_sample(const Phys &ph, const Grids &gr,
                                    const ShellArgs &sa, const RayGeo &r,
                                    uint64_t k, SampleOut &s, const double2 *stab) {
@@ -97,12 +103,14 @@ __device__ inline bool eval_sample(const Phys &ph, const Grids &gr,
   if (ph.breg_model == HAMX_BREG_GRID)
     B = gather3(gr.breg_x, gr.breg_y, gr.breg_z, gr.g_breg, pos);
   else
-    B = breg_eval<HEAVY>(ph.breg_model, ph.breg, pos);
+    B = breg_eval<HEAVY != kLight>(ph.breg_model, ph.breg, pos);
   // regular + random thermal electrons (integrator.cc:197-201)
   double te = 0.;
   if (ph.tereg_model == HAMX_TEREG_UNIF)
     te = tereg_unif(ph.tereg, pos, ph.obs);
-  else if (HEAVY && ph.tereg_model == HAMX_TEREG_YMW16) {
+  else if (HEAVY == kHeavyLiteral && ph.tereg_model == kTeregYmw16Literal)
+    te = tereg_ymw16_eval(ph.tereg, pos.x, pos.y, pos.z);
+  else if (HEAVY == kHeavy && ph.tereg_model == HAMX_TEREG_YMW16) {
     const double r2 = pos.x * pos.x + pos.y * pos.y, inv_r = r2 > 0. ? rsqrt_f64(r2) : 0.;
     te = ymw16_density(ph.ymw, pos.x, pos.y, pos.z, r2 * inv_r, inv_r);
   }
@@ -233,7 +241,7 @@ __device__ inline bool masked_out(const Phys &ph, const ShellArgs &sa, uint64_t 
 // spilled registers) measured 1.7x faster for a JF12 field on the
 // random_forward workload; with the CRE grid's energy loop three waves
 // measured 2.1x faster than one (2.3x slower for JF12, hence per case).
-template <bool PACKED, bool CREG, bool HEAVY>
+template <bool PACKED, bool CREG, Heavy HEAVY>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CREG ? 3 : 2))) void
 k_los_wave(Phys ph, Grids gr, ShellArgs sa) {
   // the synchrotron kernel tables of the CRE grid emissivities, in LDS
@@ -452,7 +460,7 @@ k_los_ray(Phys ph, FastConst fc, Grids gr, ShellArgs sa, int rays) {
   }
 }
 
-template <bool PACKED, bool CREG, bool HEAVY>
+template <bool PACKED, bool CREG, Heavy HEAVY>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CREG ? 3 : 2))) void
 k_los_thread(Phys ph, Grids gr, ShellArgs sa) {
   __shared__ double2 stab[CREG ? kSyncTab : 1];
@@ -650,8 +658,12 @@ Phys make_phys(const hamx_los_desc *d) {
   std::memcpy(ph.breg, d->breg, sizeof(ph.breg));
   std::memcpy(ph.tereg, d->tereg, sizeof(ph.tereg));
   std::memcpy(ph.cre, d->cre, sizeof(ph.cre));
-  if (d->tereg_model == HAMX_TEREG_YMW16)
-    ph.ymw = ymw16_fold(d->tereg);
+  if (d->tereg_model == HAMX_TEREG_YMW16) {
+    if (ymw16_ordinary(d->tereg))
+      ph.ymw = ymw16_fold(d->tereg);
+    else
+      ph.tereg_model = kTeregYmw16Literal;
+  }
   ph.fd_fore = -(cgs::qe * cgs::qe * cgs::qe) / (2. * cgs::pi * cgs::mec2 * cgs::mec2);
   ph.qe3 = cgs::qe * cgs::qe * cgs::qe;
   ph.three_qe = 3. * cgs::qe;
@@ -1031,17 +1043,22 @@ int los_forward_impl(hamx_ctx *ctx, const hamx_los_desc *d, const hamx_fields *f
 
   const int sched = d->schedule == HAMX_SCHED_THREAD ? HAMX_SCHED_THREAD : HAMX_SCHED_WAVE;
   // the specialised kernel covers a constant-index CRE or an imported flux
-  // grid, with synchrotron on and the random grids (if any) packed in one box
+  // grid, with synchrotron on and the random grids (if any) packed in one box; a
+  // YMW16 that needs its literal form goes to the generic march
   const bool creg = d->cre_model == HAMX_CRE_GRID && d->do_sync;
   const bool fast = d->schedule == HAMX_SCHED_AUTO && d->do_sync &&
                     (creg || (ph.idx_const && (d->cre_model == HAMX_CRE_ANA ||
                                                d->cre_model == HAMX_CRE_UNIF))) &&
-                    (packed || !grids_any);
+                    (packed || !grids_any) &&
+                    ph.tereg_model != kTeregYmw16Literal;
   const FastModels models = fast_models(d);
   const bool pw1 = fast && (creg || 0.5 * (ph.idx + 1) == -1.0);
   // models with large evaluators get kernels of their own (register use)
-  const bool heavy = d->breg_model == HAMX_BREG_JF12 || d->breg_model == HAMX_BREG_JAFFE ||
-                     d->tereg_model == HAMX_TEREG_YMW16;
+  const Heavy heavy = ph.tereg_model == kTeregYmw16Literal ? kHeavyLiteral
+                      : d->breg_model == HAMX_BREG_JF12 || d->breg_model == HAMX_BREG_JAFFE ||
+                              d->tereg_model == HAMX_TEREG_YMW16
+                          ? kHeavy
+                          : kLight;
   for (uint32_t s = 0; s < d->n_shell; ++s) {
     ShellArgs sa;
     std::memset(&sa, 0, sizeof(sa));
@@ -1142,59 +1159,36 @@ int los_forward_impl(hamx_ctx *ctx, const hamx_los_desc *d, const hamx_fields *f
 #undef HAMX_LAUNCH_FAST_CREG
 #undef HAMX_LAUNCH_FAST_M
 #undef HAMX_LAUNCH_FAST
-    } else if (sched == HAMX_SCHED_WAVE) {
-      const unsigned blocks = static_cast<unsigned>((npix + 3) / 4);
-#define HAMX_LAUNCH_WAVE(P, C, H)                                                          \
-  hipLaunchKernelGGL((k_los_wave<P, C, H>), dim3(blocks), dim3(256), 0, ctx->stream, ph, gr, sa)
-      if (creg)
-        {
-        if (heavy)
-          HAMX_LAUNCH_WAVE(false, true, true);
-        else
-          HAMX_LAUNCH_WAVE(false, true, false);
-      }
-      else if (packed)
-        {
-        if (heavy)
-          HAMX_LAUNCH_WAVE(true, false, true);
-        else
-          HAMX_LAUNCH_WAVE(true, false, false);
-      }
-      else
-        {
-        if (heavy)
-          HAMX_LAUNCH_WAVE(false, false, true);
-        else
-          HAMX_LAUNCH_WAVE(false, false, false);
-      }
-#undef HAMX_LAUNCH_WAVE
     } else {
-      const unsigned blocks = static_cast<unsigned>((npix + 255) / 256);
-#define HAMX_LAUNCH_THREAD(P, C, H)                                                        \
-  hipLaunchKernelGGL((k_los_thread<P, C, H>), dim3(blocks), dim3(256), 0, ctx->stream, ph, gr, \
-                     sa)
-      if (creg)
-        {
-        if (heavy)
-          HAMX_LAUNCH_THREAD(false, true, true);
-        else
-          HAMX_LAUNCH_THREAD(false, true, false);
-      }
-      else if (packed)
-        {
-        if (heavy)
-          HAMX_LAUNCH_THREAD(true, false, true);
-        else
-          HAMX_LAUNCH_THREAD(true, false, false);
-      }
+      // CRE flux grids gather the random grids where they lie
+#define HAMX_LAUNCH_GENERIC(KERNEL, BLOCKS)                                                \
+  do {                                                                                     \
+    if (creg)                                                                              \
+      HAMX_LAUNCH_HEAVY(KERNEL, BLOCKS, false, true);                                      \
+    else if (packed)                                                                       \
+      HAMX_LAUNCH_HEAVY(KERNEL, BLOCKS, true, false);                                      \
+    else                                                                                   \
+      HAMX_LAUNCH_HEAVY(KERNEL, BLOCKS, false, false);                                     \
+  } while (0)
+#define HAMX_LAUNCH_HEAVY(KERNEL, BLOCKS, P, C)                                            \
+  do {                                                                                     \
+    if (heavy == kHeavyLiteral)                                                            \
+      HAMX_LAUNCH(KERNEL, BLOCKS, P, C, kHeavyLiteral);                                    \
+    else if (heavy == kHeavy)                                                              \
+      HAMX_LAUNCH(KERNEL, BLOCKS, P, C, kHeavy);                                           \
+    else                                                                                   \
+      HAMX_LAUNCH(KERNEL, BLOCKS, P, C, kLight);                                           \
+  } while (0)
+#define HAMX_LAUNCH(KERNEL, BLOCKS, P, C, H)                                               \
+  hipLaunchKernelGGL((KERNEL<P, C, H>), dim3(static_cast<unsigned>(BLOCKS)), dim3(256), 0, \
+                     ctx->stream, ph, gr, sa)
+      if (sched == HAMX_SCHED_WAVE)
+        HAMX_LAUNCH_GENERIC(k_los_wave, (npix + 3) / 4);
       else
-        {
-        if (heavy)
-          HAMX_LAUNCH_THREAD(false, false, true);
-        else
-          HAMX_LAUNCH_THREAD(false, false, false);
-      }
-#undef HAMX_LAUNCH_THREAD
+        HAMX_LAUNCH_GENERIC(k_los_thread, (npix + 255) / 256);
+#undef HAMX_LAUNCH
+#undef HAMX_LAUNCH_HEAVY
+#undef HAMX_LAUNCH_GENERIC
     }
     HAMX_HIP(ctx, hipGetLastError());
     prof_end(ctx, pm,

@@ -20,6 +20,9 @@
 
 namespace hamx {
 
+// Phys::tereg_model of a YMW16 that needs its literal form (ymw16_ordinary).
+constexpr int kTeregYmw16Literal = 1000;
+
 // Constants of one write_grid pass (host-computed in the reference's
 // expression order).
 struct Phys {
@@ -525,8 +528,16 @@ struct FastSample {
 // models (an LSA field with its parameter partials; a uniform TE sphere with
 // n0's) instead of being LSA and the uniform sphere.  JF12, Jaffe and YMW16,
 // whose evaluators take many registers, are compiled in only where the pass
-// has them: kYmw16Models adds YMW16 to the light models, kAllModels all three.
-enum FastModels { kLsaUnif = 0, kLightModels = 1, kYmw16Models = 2, kAllModels = 3 };
+// has them: kYmw16Models adds YMW16 to the light models, kAllModels all three,
+// kAnyModels (the reverse sweep, one kernel for every model) YMW16's literal form
+// too.
+enum FastModels {
+  kLsaUnif = 0,
+  kLightModels = 1,
+  kYmw16Models = 2,
+  kAllModels = 3,
+  kAnyModels = 4
+};
 inline FastModels fast_models(const hamx_los_desc *d) {
   if (d->breg_model == HAMX_BREG_LSA && d->tereg_model == HAMX_TEREG_UNIF)
     return kLsaUnif;
@@ -562,7 +573,7 @@ __device__ inline bool eval_fast(const Phys &ph, const FastConst &fc, const Grid
     if (ph.breg_model == HAMX_BREG_GRID)
       B = gather3(gr.breg_x, gr.breg_y, gr.breg_z, gr.g_breg, pos);
     else
-      B = breg_eval<MODELS == kAllModels>(ph.breg_model, ph.breg, pos);
+      B = breg_eval<(MODELS >= kAllModels)>(ph.breg_model, ph.breg, pos);
   }
   // exp(-2|z| / kpc): the LSA's tanh(z / kpc) and, when the CRE scale
   // height is 1 kpc, the CRE's sech^2(z / z0)
@@ -598,7 +609,9 @@ __device__ inline bool eval_fast(const Phys &ph, const FastConst &fc, const Grid
       te = fc.n0;
   } else {
     o.te_in = false; // no n0 partial
-    if (MODELS >= kYmw16Models && ph.tereg_model == HAMX_TEREG_YMW16)
+    if (MODELS == kAnyModels && ph.tereg_model == kTeregYmw16Literal)
+      te = tereg_ymw16_eval(ph.tereg, pos.x, pos.y, pos.z);
+    else if (MODELS >= kYmw16Models && ph.tereg_model == HAMX_TEREG_YMW16)
       te = ymw16_density(ph.ymw, pos.x, pos.y, pos.z, o.rr, inv_r);
     else if (ph.tereg_model == HAMX_TEREG_GRID)
       te = gather1(gr.tereg, gr.g_tereg, pos);

@@ -3,7 +3,7 @@
 // parameters, cuts and choice between components) in far fewer FP64
 // instructions, which bound the march: with the literal form it took about
 // 4500 VALU instructions per sample inside the limits.  Measured on 3 shells
-// up to nside 128 with 200x200x40 random grids: generic march 12.7 -> 8.0 ms
+// up to nside 128 with 200x200x40 random grids: generic march 12.7 -> 7.8 ms
 // per pass with this evaluator, 4.8 ms in the specialised march.  Within 8e-14
 // of the literal form at any of 8e6 random points (8e-15 rms), the difference
 // largest where the Gum shell's angles cancelled.
@@ -41,6 +41,29 @@ struct Ymw16 {
   double lb_n[2], lb_theta[2], lb_det[2], lb_w[2], lb_h[2];
   double nli, li_rmax, li_rli, inv_wli, li_tmax, inv_dli, li_cos, li_sin;
 };
+
+// The parameters for which the short forms below hold: finite, every scale
+// positive and such that the exponents stay within exp_fast's range (|x| below
+// 1e15), arms of a pitch short of a right angle, a Gum shell with a radius.
+// Others (a scale height of 0 to switch a component off, say) take the literal
+// form, in the generic march: there 1 / cosh(inf), the sign of a negative scale
+// and a component's NaN have their own meaning.
+inline bool ymw16_ordinary(const double *p) {
+  auto in = [p](int i, double lo, double hi) { return p[i] >= lo && p[i] <= hi; };
+  for (int i = 0; i < 73; ++i)
+    if (!in(i, -1e25, 1e25))
+      return false;
+  for (int i : {3, 6, 7, 17, 18, 19, 20, 42, 51, 52, 54, 55, 61, 62, 66, 67, 70}) // lengths
+    if (!in(i, 1e15, 1e24))
+      return false;
+  for (int i : {10, 43, 46, 49, 60, 65, 71}) // factors and angles
+    if (!in(i, 1e-5, 1e5))
+      return false;
+  for (int i = 0; i < 4; ++i)
+    if (!in(27 + i, -1e3, 1e3) || !in(32 + i, -1e2, 1e2) || !in(37 + i, 1e-3, 1e3))
+      return false;
+  return in(56, 1e-3, 1e3);
+}
 
 inline Ymw16 ymw16_fold(const double *p) {
   Ymw16 y;

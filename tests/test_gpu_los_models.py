@@ -5,7 +5,7 @@ oracle: FP64 maps within 1e-10 relative L2 (the plain-path bar)."""
 import numpy as np
 import pytest
 
-from hammurabix_amd import Param, _capi as capi, configs
+from hammurabix_amd import HamxError, Param, _capi as capi, configs
 from hammurabix_amd.units import CGS
 from oracle_lib import write_grid
 from test_gpu_los import assert_parity, gpu_maps, random_grids
@@ -71,3 +71,74 @@ def test_ymw16_through_its_nebulae(ctx):
                                            oc_r_max=1.5, oc_r_res=0.002))
     d = par.los_desc()
     assert_parity(gpu_maps(ctx, d), write_grid(d), label="ymw16 nebulae")
+
+
+def ymw16_near(schedule=capi.HAMX_SCHED_AUTO):
+    """Rays through the nebulae about the Sun and the disks to 12 kpc."""
+    return Param(text=configs.plain_forward(tereg="ymw16", shell_num=2, nside_sim=4, nside_out=4,
+                                            oc_r_max=12., oc_r_res=0.03)).los_desc(schedule=schedule)
+
+
+def compare_ymw16(ctx, d, label):
+    """Parity with the oracle, or refused where its maps are not finite."""
+    with np.errstate(all="ignore"):
+        ref = write_grid(d)
+    print("case:", label, flush=True)
+    if all(np.all(np.isfinite(v)) for v in ref.values()):
+        assert_parity(gpu_maps(ctx, d), ref, label=label)
+    else:
+        with pytest.raises(HamxError, match="non-finite"):
+            gpu_maps(ctx, d)
+
+
+# the scale lengths and angular widths of every component
+YMW16_SCALES = [3, 6, 7, 10, 17, 18, 19, 20, 42, 43, 46, 49, 51, 52, 54, 60, 61, 62, 65, 66, 67,
+                70, 71]
+
+
+@pytest.mark.parametrize("sched", [capi.HAMX_SCHED_AUTO, capi.HAMX_SCHED_WAVE])
+@pytest.mark.parametrize("value", [0.0, 1.0, "negative"])
+def test_ymw16_scales_out_of_range(ctx, value, sched):
+    """A scale of 0 (or 1 cm, 1 degree) turns its component off, wholly or off
+    its own surface; a negative one is its magnitude within its sech^2."""
+    for i in YMW16_SCALES:
+        d = ymw16_near(sched)
+        d.tereg[i] = -d.tereg[i] if value == "negative" else value
+        compare_ymw16(ctx, d, f"ymw16 scale {i} = {value}")
+
+
+@pytest.mark.parametrize("sched", [capi.HAMX_SCHED_AUTO, capi.HAMX_SCHED_WAVE])
+def test_ymw16_arm_across_the_circle(ctx, sched):
+    """Pitch angles to a right angle."""
+    for pitch in (np.pi / 2, -np.pi / 2, 1.5707, 1.4):
+        d = ymw16_near(sched)
+        d.tereg[32], d.tereg[37] = np.tan(pitch), np.cos(pitch)
+        compare_ymw16(ctx, d, f"ymw16 pitch {pitch}")
+    d = ymw16_near(sched)
+    d.tereg[37] = -d.tereg[37]  # the distance from the arm changes sign
+    compare_ymw16(ctx, d, "ymw16 negative cosine")
+    d = ymw16_near(sched)
+    d.tereg[27] = -1e7
+    compare_ymw16(ctx, d, "ymw16 arm out of reach")
+
+
+@pytest.mark.parametrize("value", [np.nan, np.inf])
+def test_ymw16_parameter_not_finite(ctx, value):
+    """Refused where the model's own weighting (0 times what is not chosen)
+    makes the density NaN, accepted where it does not.  (The disk's and the arms'
+    NaN is left out: the oracle takes the larger of the two by std::max, which
+    drops the other one.)"""
+    disk = range(7, 50) if np.isnan(value) else range(44, 50)
+    for i in sorted(set(range(73)) - set(disk) - {0, 3, 4, 50, 52}):
+        d = ymw16_near()
+        d.tereg[i] = value
+        compare_ymw16(ctx, d, f"ymw16 parameter {i} = {value}")
+
+
+@pytest.mark.parametrize("sched", [capi.HAMX_SCHED_AUTO, capi.HAMX_SCHED_WAVE])
+def test_ymw16_gum_shell_out_of_range(ctx, sched):
+    """A Gum shell without radius, inside out or flattened beyond measure."""
+    for a, k in ((0.0, 1.0), (1.0, -1.4), (-1.0, 1.4), (1.0, 0.0), (1e-80, 1.4)):
+        d = ymw16_near(sched)
+        d.tereg[55], d.tereg[56] = a * d.tereg[55], k
+        compare_ymw16(ctx, d, f"ymw16 gum shell {a} {k}")
