@@ -18,7 +18,9 @@
 //     D^2 = (sqrt(S) - a k)^2 S / (k^4 Q + Z).
 // * The Local Bubble's and Loop I's angles are evaluated only where their
 //   other factors leave something: the bubble's components are dropped where
-//   their exponents sum to more than `lb_skip` (below 1e-60 cm^-3).
+//   their exponents sum to more than 150 and what is left of them is below the
+//   disks' density (`lb_floor`), the least that the bubble is compared with;
+//   without disks, where the exponentials are 0.
 #pragma once
 
 #include "hamx_cgs.h"
@@ -37,7 +39,7 @@ struct Ymw16 {
   double ngc, gc_r2, inv_agc2, gc_zmax, m2_hgc;
   double ngn, gum_d2, inv_wgn2, k2g, k4g, akg; // k^2, k^4, a k
   double gum_x, gum_y, gum_z;
-  double j_lb, lb_skip;
+  double j_lb, lb_floor;
   double lb_n[2], lb_theta[2], lb_det[2], lb_w[2], lb_h[2];
   double nli, li_rmax, li_rli, inv_wli, li_tmax, inv_dli, li_cos, li_sin;
 };
@@ -62,7 +64,7 @@ inline bool ymw16_ordinary(const double *p) {
   for (int i = 0; i < 4; ++i)
     if (!in(27 + i, -1e3, 1e3) || !in(32 + i, -1e2, 1e2) || !in(37 + i, 1e-3, 1e3))
       return false;
-  return in(56, 1e-3, 1e3);
+  return in(1, -1e23, 1e23) && in(56, 1e-3, 1e3);
 }
 
 inline Ymw16 ymw16_fold(const double *p) {
@@ -119,9 +121,8 @@ inline Ymw16 ymw16_fold(const double *p) {
   y.k4g = y.k2g * y.k2g;
   y.akg = p[55] * p[56];
   y.j_lb = p[57];
-  // without a thick disk the density can be zero elsewhere and any positive
-  // bubble term decides: drop none then (the exponentials underflow at 745)
-  y.lb_skip = p[5] > 0. ? 150. : 1500.;
+  // both components' sech^2 products at exponents of -150 and below
+  y.lb_floor = 128. * std::exp(-150.) * std::fmax(std::fabs(p[58]), std::fabs(p[63]));
   for (int c = 0; c < 2; ++c) {
     const double *q = p + 58 + 5 * c;
     y.lb_n[c] = q[0];
@@ -227,22 +228,25 @@ __device__ inline double ymw16_density(const Ymw16 &m, double px, double py, dou
   const double Rlb = 110. * cgs::pc;
   const double u = (y - 8.34 * cgs::kpc) * 0.94 - 0.34 * z;
   const double rlb = sqrt_pos(u * u + x * x);
+  const double n_disk = n_thin > n_arm ? n_thin : n_arm;
+  const bool bubble = rlb < Rlb;
+  const double n0 = (bubble ? m.j_lb * n_thick : n_thick) + n_disk;
   double n_lb = 0.;
   if (!(y < 0)) {
-    const double dr = rlb - Rlb;
+    const double dr = rlb - Rlb, skip = n0 > m.lb_floor ? 150. : 1500.;
     double ex[2];
     bool any = false;
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
       ex[c] = 2. * (fabs(dr) / m.lb_w[c] + az / m.lb_h[c]);
-      any = any || !(ex[c] > m.lb_skip);
+      any = any || !(ex[c] > skip);
     }
     if (any) {
       const double l = atan2(x, m.r0 - y) / cgs::rad;
 #pragma unroll
       for (int c = 0; c < 2; ++c) {
         const double dl = fmin(fabs(l + 360. - m.lb_theta[c]), fabs(m.lb_theta[c] - l));
-        if (ex[c] > m.lb_skip ||
+        if (ex[c] > skip ||
             !(dl < 10. * m.lb_det[c] || dr < 10. * m.lb_w[c] || z < 10. * m.lb_h[c]))
           continue;
         n_lb += m.lb_n[c] * sech2_of(exp_fast(-2. * (dl / m.lb_det[c]))) *
@@ -266,9 +270,6 @@ __device__ inline double ymw16_density(const Ymw16 &m, double px, double py, dou
       }
     }
   }
-  const double n_disk = n_thin > n_arm ? n_thin : n_arm;
-  const bool bubble = rlb < Rlb;
-  const double n0 = (bubble ? m.j_lb * n_thick : n_thick) + n_disk;
   if (n_lb > n0 && (bubble || n_lb > n_gum))
     return n_lb;
   if (n_gum > n0)

@@ -122,6 +122,22 @@ def test_ymw16_arm_across_the_circle(ctx, sched):
     compare_ymw16(ctx, d, "ymw16 arm out of reach")
 
 
+@pytest.mark.parametrize("sched", [capi.HAMX_SCHED_AUTO, capi.HAMX_SCHED_WAVE])
+@pytest.mark.parametrize("n1", [0.0, 0.01])
+def test_ymw16_bubble_without_disks(ctx, n1, sched):
+    """Where the disks are 0 any bubble term above 0 decides, here 1e-60 and
+    less against a wide Loop I above a thick disk of 20 pc."""
+    d = ymw16_near(sched)
+    d.tereg[5], d.tereg[6] = n1, 20 * CGS.pc
+    d.tereg[9] = 0.0
+    for i in range(12, 17):
+        d.tereg[i] = 0.0
+    for i in (61, 62, 66, 67):
+        d.tereg[i] = 1.3 * CGS.pc
+    d.tereg[70], d.tereg[71] = 100 * CGS.pc, 300.0
+    compare_ymw16(ctx, d, "ymw16 bubble without disks")
+
+
 @pytest.mark.parametrize("value", [np.nan, np.inf])
 def test_ymw16_parameter_not_finite(ctx, value):
     """Refused where the model's own weighting (0 times what is not chosen)
