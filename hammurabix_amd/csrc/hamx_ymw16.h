@@ -61,6 +61,9 @@ inline bool ymw16_ordinary(const double *p) {
   for (int i : {10, 43, 46, 49, 60, 65, 71}) // factors and angles
     if (!in(i, 1e-5, 1e5))
       return false;
+  for (int i : {45, 48, 59, 64, 72}) // directions, in degrees
+    if (!in(i, -1e6, 1e6))
+      return false;
   for (int i = 0; i < 4; ++i)
     if (!in(27 + i, -1e3, 1e3) || !in(32 + i, -1e2, 1e2) || !in(37 + i, 1e-3, 1e3))
       return false;
