@@ -2179,10 +2179,10 @@ extern "C" int hamx_batch_create(hamx_ctx *ctx, const hamx_batch_inst *inst, uin
       in.f.inv_z0k = static_cast<float>(cgs::kpc / x.los.cre[4]);
     }
     in.f.hexp = static_cast<float>(0.5 * (1. - pw_e));
-    in.r_min2 = x.los.gc_r_min * x.los.gc_r_min;
-    in.r_max2 = x.los.gc_r_max * x.los.gc_r_max;
-    in.te_r02 = x.los.tereg[1] * x.los.tereg[1];
-    in.cre_r02 = x.los.cre[1] * x.los.cre[1];
+    in.r_min2 = limit2(x.los.gc_r_min);
+    in.r_max2 = limit2(x.los.gc_r_max);
+    in.te_r02 = limit2(x.los.tereg[1]);
+    in.cre_r02 = limit2(x.los.cre[1]);
     // grids
     const bool any_grid = x.brnd_x || x.ternd;
     in.grids = any_grid ? 1 : 0;

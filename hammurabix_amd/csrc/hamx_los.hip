@@ -645,8 +645,8 @@ Phys make_phys(const hamx_los_desc *d) {
   ph.obs = Vec3{d->observer[0], d->observer[1], d->observer[2]};
   ph.gc_r_min = d->gc_r_min;
   ph.gc_r_max = d->gc_r_max;
-  ph.gc_r_min2 = d->gc_r_min * d->gc_r_min;
-  ph.gc_r_max2 = d->gc_r_max * d->gc_r_max;
+  ph.gc_r_min2 = limit2(d->gc_r_min);
+  ph.gc_r_max2 = limit2(d->gc_r_max);
   ph.gc_z_min = d->gc_z_min;
   ph.gc_z_max = d->gc_z_max;
   ph.do_dm = d->do_dm != 0;
@@ -736,7 +736,7 @@ FastConst make_fast(const hamx_los_desc *d, const Phys &ph, double delta, bool p
   fc.inv_kpc = 1.0 / (1. * cgs::kpc);
   fc.n0 = d->tereg[0];
   fc.te_r0 = d->tereg[1];
-  fc.te_r02 = d->tereg[1] * d->tereg[1];
+  fc.te_r02 = limit2(d->tereg[1]);
   fc.cre_unif = d->cre_model == HAMX_CRE_UNIF;
   if (creg) { // the flux grid's emissivities take delta i2bt alone
     fc.kt = fc.kp = delta * ph.i2bt;
@@ -745,7 +745,7 @@ FastConst make_fast(const hamx_los_desc *d, const Phys &ph, double delta, bool p
   }
   if (fc.cre_unif) {
     fc.cre_r0 = d->cre[1];
-    fc.cre_r02 = d->cre[1] * d->cre[1];
+    fc.cre_r02 = limit2(d->cre[1]);
   } else {
     fc.R0 = ph.R0;
     fc.inv_cre_r0 = 1.0 / d->cre[3];

@@ -698,6 +698,9 @@ inline double digamma(double x) {
 }
 bool same_box(const hamx_box &a, const hamx_box &b);
 int check_box(hamx_ctx *ctx, const hamx_box &b, const char *what);
+// A limit on a length as one on its square (the length is below no negative
+// limit and above every one).
+inline double limit2(double r) { return r < 0. ? -1. : r * r; }
 inline uint64_t box_size(const hamx_box &b) { return b.nx * b.ny * b.nz; }
 // Integrator::assemble_shell_ref (integrator.cc:231-244)
 void shell_ref(const hamx_los_desc *d, uint32_t s, uint64_t &step, double &d_start,

@@ -158,3 +158,31 @@ def test_ymw16_gum_shell_out_of_range(ctx, sched):
         d = ymw16_near(sched)
         d.tereg[55], d.tereg[56] = a * d.tereg[55], k
         compare_ymw16(ctx, d, f"ymw16 gum shell {a} {k}")
+
+
+@pytest.mark.parametrize("sched", [capi.HAMX_SCHED_AUTO, capi.HAMX_SCHED_WAVE])
+@pytest.mark.parametrize("breg", ["cart", "lsa"])
+@pytest.mark.parametrize("what", ["r_min", "r_max", "te", "cre"])
+def test_negative_limits(ctx, what, breg, sched):
+    """No length is below a negative lower limit; every one is above a negative
+    radius (the specialised march compares squares)."""
+    print("case: negative", what, breg, sched, flush=True)
+    d = Param(text=configs.plain_forward(nside_sim=2, nside_out=2, oc_r_res=0.1)).los_desc(
+        schedule=sched)
+    set_breg(d, breg)
+    if what == "r_min":
+        d.gc_r_min = -12 * CGS.kpc
+    elif what == "r_max":
+        d.gc_r_max = -12 * CGS.kpc
+    elif what == "te":
+        d.tereg[1] = -6 * CGS.kpc
+    else:
+        d.cre_model = capi.HAMX_CRE_UNIF
+        d.cre[0:4] = [3.0, -6 * CGS.kpc, 20.6 * CGS.GeV, 0.0217]
+    ref, got = write_grid(d), gpu_maps(ctx, d)
+    zero = {k for k, v in ref.items() if not np.any(v)}
+    assert zero == {"r_min": set(), "r_max": set(ref), "te": {"dm", "fd"},
+                    "cre": {"is", "qs", "us"}}[what]
+    assert not any(np.any(got[k]) for k in zero)
+    assert_parity({k: got[k] for k in ref if k not in zero},
+                  {k: ref[k] for k in ref if k not in zero}, label=f"negative {what}")
