@@ -123,6 +123,41 @@ def test_los_with_cre_grid_matches_oracle(ctx, sched):
     assert np.linalg.norm(ref["is"]) > 0 and np.linalg.norm(ref["qs"]) > 0
 
 
+@pytest.mark.parametrize("random", [True, False])
+@pytest.mark.parametrize("model", ["lsa", "cart", "jf12"])
+@pytest.mark.parametrize("masked", ["", "pixels", "halves"])
+def test_large_shell_with_cre_grid(ctx, masked, model, random):
+    """A shell of nside 32, two rays to a workgroup (their set-up, their steps and
+    their sums in turn), with none, either or both of them masked."""
+    from test_gpu_los_models import set_breg
+    print("case: cre grid large shell", masked, model, random, flush=True)
+    d = Param(text=configs.random_forward(shell_num=1, nside_sim=32, nside_out=32, oc_r_res=0.31,
+                                          grid=(16, 16, 8), freqs=[1.4])).los_desc()
+    d.cre_model = capi.HAMX_CRE_GRID
+    set_breg(d, model)
+    kw = dict(cre=flux_grid(), cre_box=CRE_BOX, cre_E=(E_MIN, E_FACT, NE))
+    if random:
+        rng = np.random.default_rng(2)
+        n = 16 * 16 * 8
+        box = capi.HamxBox(16, 16, 8, -20 * KPC, 20 * KPC, -20 * KPC, 20 * KPC, -4 * KPC, 4 * KPC)
+        kw.update(brnd=tuple(np.ascontiguousarray(rng.normal(0, 2e-6, n)) for _ in range(3)),
+                  brnd_box=box, ternd=np.ascontiguousarray(rng.normal(0.0, 0.003, n)),
+                  ternd_box=box)
+    if masked:
+        m = np.ones(npix(32))
+        if masked == "pixels":
+            m[np.random.default_rng(3).random(m.size) < 0.4] = 0.0
+        else:
+            m[m.size // 3::2] = 0.0
+        kw.update(mask=m, nside_mask=32)
+    ref = write_grid(d, **kw)
+    got = maps_for(d)
+    ctx.los_forward(d, got, **kw)
+    for k in ref:
+        assert rel_l2(got[k], ref[k]) <= 1e-10, k
+    assert np.linalg.norm(ref["is"]) > 0
+
+
 @pytest.mark.parametrize("sched", [capi.HAMX_SCHED_THREAD, capi.HAMX_SCHED_WAVE,
                                    capi.HAMX_SCHED_AUTO])
 @pytest.mark.parametrize("bad", [np.inf, np.nan])

@@ -31,16 +31,13 @@ def set_breg(d, name):
         d.breg_model = capi.HAMX_BREG_GRID
 
 
-@pytest.mark.parametrize("alpha", [3.0, 2.8])
-@pytest.mark.parametrize("random", [True, False])
-@pytest.mark.parametrize("breg,tereg", [("none", "unif"), ("cart", "none"), ("helix", "unif"),
-                                        ("grid", "grid"), ("lsa", "none"), ("lsa", "ymw16"),
-                                        ("cart", "ymw16"), ("jf12", "unif"), ("jf12", "ymw16")])
-def test_models(ctx, breg, tereg, random, alpha):
-    print("case:", breg, tereg, random, alpha, flush=True)
+MODELS = [("none", "unif"), ("cart", "none"), ("helix", "unif"), ("grid", "grid"), ("lsa", "none"),
+          ("lsa", "ymw16"), ("cart", "ymw16"), ("jf12", "unif"), ("jf12", "ymw16")]
+
+
+def check_models(ctx, breg, tereg, random, alpha, **kw):
     par = Param(text=configs.random_forward(
-        nside_sim=2, nside_out=8, oc_r_res=0.043, grid=(16, 16, 8),
-        tereg="ymw16" if tereg == "ymw16" else "unif"))
+        grid=(16, 16, 8), tereg="ymw16" if tereg == "ymw16" else "unif", **kw))
     d = par.los_desc()
     d.cre[0] = alpha
     set_breg(d, breg)
@@ -56,12 +53,31 @@ def test_models(ctx, breg, tereg, random, alpha):
     elif tereg == "none":
         d.tereg_model = capi.HAMX_TEREG_NONE
     if (breg, random) == ("none", False):
-        return  # no field at all: nothing to compare
+        pytest.skip("no field at all: nothing to compare")
     if tereg == "none" and not random:
         d.do_dm = d.do_fd = 0  # zero maps
     ref = {k: v for k, v in write_grid(d, **grids).items() if np.any(v)}
     got = gpu_maps(ctx, d, **grids)
     assert_parity({k: got[k] for k in ref}, ref, label=f"{breg}/{tereg}")
+
+
+@pytest.mark.parametrize("alpha", [3.0, 2.8])
+@pytest.mark.parametrize("random", [True, False])
+@pytest.mark.parametrize("breg,tereg", MODELS)
+def test_models(ctx, breg, tereg, random, alpha):
+    """Small shells: four wavefronts on a ray."""
+    print("case:", breg, tereg, random, alpha, flush=True)
+    check_models(ctx, breg, tereg, random, alpha, nside_sim=2, nside_out=8, oc_r_res=0.043)
+
+
+@pytest.mark.parametrize("alpha", [3.0, 2.8])
+@pytest.mark.parametrize("random", [True, False])
+@pytest.mark.parametrize("breg,tereg", MODELS)
+def test_models_on_large_shells(ctx, breg, tereg, random, alpha):
+    """Shells from nside 32 on: a wavefront marches two rays in turn."""
+    print("case: large", breg, tereg, random, alpha, flush=True)
+    check_models(ctx, breg, tereg, random, alpha, shell_num=2, nside_sim=32, nside_out=32,
+                 oc_r_res=0.17)
 
 
 def test_ymw16_through_its_nebulae(ctx):
