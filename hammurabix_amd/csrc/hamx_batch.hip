@@ -251,7 +251,6 @@ struct S32 {
   float te_raw;
   bool lsa_in, te_in, cell_ok;
   float cos_p, sin_p, sps, cps, sch, cch, lnr, tnh;
-  uint64_t idx;
   float xd, yd, zd;
   int cx, cy, cz; // the cell's lower corner
 };
@@ -431,7 +430,6 @@ __device__ inline bool eval_f32(const BInst &in, const BShell &sh, const RayGeo 
   if (o.te_in)
     te_d = c.n0d;
   if (GRIDS && any_cell) {
-    o.idx = cell.idx;
     o.zd = static_cast<float>(cell.zd);
     o.yd = static_cast<float>(cell.yd);
     o.xd = static_cast<float>(cell.xd);
@@ -1045,7 +1043,7 @@ __device__ void adj_lanes_f32(const BInst &in, int s, uint64_t ipix, bool live,
     gfd = in.do_fd ? A.g_fd[ipix] : 0.;
     fd_total = in.t_fd[in.fd_off[s] + ipix];
   }
-  const uint64_t sy = in.geo.nz, sx = in.geo.ny * in.geo.nz;
+  const uint64_t sx = in.geo.ny * in.geo.nz;
   float *ggrid = static_cast<float *>(A.ggrid);
   // vertex indices are the cache's 32-bit tags
   if ((in.geo.fx + 1.) * static_cast<double>(sx) >= static_cast<double>(kVtxEmpty))

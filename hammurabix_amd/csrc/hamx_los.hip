@@ -320,16 +320,10 @@ k_los_wave(Phys ph, Grids gr, ShellArgs sa) {
 // measured 8% faster than the unconstrained choice of two.  With YMW16 two /
 // three / four waves measured 5.68 / 4.98 / 4.80 ms per march (3 shells up to
 // nside 128); JF12 4.7 / 4.0 ms with two / three.
-template <bool GRIDS, bool PW1, int MODELS, bool CREG>
-__global__ __launch_bounds__(256) __attribute__((
-    amdgpu_waves_per_eu(MODELS == kAllModels || CREG ? 3 : 4))) void
+template <bool GRIDS, bool PW1, int MODELS>
+__global__ __launch_bounds__(256)
+__attribute__((amdgpu_waves_per_eu(MODELS == kAllModels ? 3 : 4))) void
 k_los_fast(Phys ph, FastConst fc, Grids gr, ShellArgs sa) {
-  // the synchrotron kernels' table of the CRE grid emissivities
-  __shared__ double2 stab[CREG ? kSyncTab : 1];
-  if constexpr (CREG) {
-    load_sync_tab(stab);
-    __syncthreads();
-  }
   // kFastRays consecutive rays per wavefront: their set-up (pointing,
   // versors, FD cache, culled step range) runs one ray per lane into LDS,
   // then the rays are marched one after another, 64 samples per step
@@ -356,7 +350,7 @@ k_los_fast(Phys ph, FastConst fc, Grids gr, ShellArgs sa) {
       FastSample o;
       bool valid = false;
       if (k < r.k_hi)
-        valid = eval_fast<GRIDS, PW1, MODELS, CREG>(ph, fc, gr, sa, r, k, o, stab);
+        valid = eval_fast<GRIDS, PW1, MODELS>(ph, fc, gr, sa, r, k, o);
       const double fdk = valid ? o.fdk : 0.;
       const double incl = wave_incl_scan(fdk, lane);
       const double fd_here = fd_carry + incl;
@@ -384,7 +378,7 @@ k_los_fast(Phys ph, FastConst fc, Grids gr, ShellArgs sa) {
 // consecutive samples per step (`rays` rays per workgroup, one after another,
 // set up one per lane): the running Faraday depth adds the earlier
 // wavefronts' sums of the step, handed over in LDS.
-constexpr int kRayMax = 4;
+constexpr int kRayMax = 2; // with more, a masked ray between two would leave `sums` unguarded
 template <bool GRIDS, bool PW1, int MODELS, bool CREG>
 __global__ __launch_bounds__(256) __attribute__((
     amdgpu_waves_per_eu(MODELS == kAllModels || CREG ? 3 : 4))) void
@@ -675,7 +669,6 @@ Phys make_phys(const hamx_los_desc *d) {
     ph.i2bt = cgs::c_light * cgs::c_light / (2. * cgs::kB * f * f);
     ph.A_num = 2. * cgs::pi * f * cgs::mec;
     ph.xft_num = 4. * cgs::pi * f * cgs::mec * cgs::mec2 * cgs::mec2;
-    ph.xfp_num = 2. * cgs::mec * cgs::mec2 * cgs::mec2 * 2. * cgs::pi * f;
     ph.fore_num = 1.73205081 * cgs::qe * cgs::qe * cgs::qe;
     ph.fore_den = cgs::mec2 * cgs::c_light * cgs::GeV * cgs::m * cgs::m * cgs::sec;
     const double p = cgs::h_planck * f / (cgs::kB * 2.725);
@@ -1115,34 +1108,36 @@ int los_forward_impl(hamx_ctx *ctx, const hamx_los_desc *d, const hamx_fields *f
       scan = !ray;
       const unsigned blocks =
           static_cast<unsigned>(ray ? (npix + rays - 1) / rays : (npix + 4 * kFastRays - 1) / (4 * kFastRays));
-#define HAMX_LAUNCH_FAST(G, P, M, C)                                                       \
+#define HAMX_LAUNCH_RAY(G, P, M, C)                                                        \
+  hipLaunchKernelGGL((k_los_ray<G, P, M, C>), dim3(blocks), dim3(256), 0, ctx->stream, ph, \
+                     fc, gr, sa, rays)
+#define HAMX_LAUNCH_FAST(G, P, M)                                                          \
   do {                                                                                     \
     if (ray)                                                                               \
-      hipLaunchKernelGGL((k_los_ray<G, P, M, C>), dim3(blocks), dim3(256), 0, ctx->stream, \
-                         ph, fc, gr, sa, rays);                                            \
+      HAMX_LAUNCH_RAY(G, P, M, false);                                                     \
     else                                                                                   \
-      hipLaunchKernelGGL((k_los_fast<G, P, M, C>), dim3(blocks), dim3(256), 0, ctx->stream, \
+      hipLaunchKernelGGL((k_los_fast<G, P, M>), dim3(blocks), dim3(256), 0, ctx->stream,   \
                          ph, fc, gr, sa);                                                  \
   } while (0)
 #define HAMX_LAUNCH_FAST_M(G, P)                                                           \
   do {                                                                                     \
     if (models == kLsaUnif)                                                                \
-      HAMX_LAUNCH_FAST(G, P, kLsaUnif, false);                                             \
+      HAMX_LAUNCH_FAST(G, P, kLsaUnif);                                                    \
     else if (models == kLightModels)                                                       \
-      HAMX_LAUNCH_FAST(G, P, kLightModels, false);                                         \
+      HAMX_LAUNCH_FAST(G, P, kLightModels);                                                \
     else if (models == kYmw16Models)                                                       \
-      HAMX_LAUNCH_FAST(G, P, kYmw16Models, false);                                         \
+      HAMX_LAUNCH_FAST(G, P, kYmw16Models);                                                \
     else                                                                                   \
-      HAMX_LAUNCH_FAST(G, P, kAllModels, false);                                           \
+      HAMX_LAUNCH_FAST(G, P, kAllModels);                                                  \
   } while (0)
 #define HAMX_LAUNCH_FAST_CREG(G)                                                           \
   do {                                                                                     \
     if (models == kLsaUnif)                                                                \
-      HAMX_LAUNCH_FAST(G, true, kLsaUnif, true);                                           \
+      HAMX_LAUNCH_RAY(G, true, kLsaUnif, true);                                            \
     else if (models == kLightModels)                                                       \
-      HAMX_LAUNCH_FAST(G, true, kLightModels, true);                                       \
+      HAMX_LAUNCH_RAY(G, true, kLightModels, true);                                        \
     else                                                                                   \
-      HAMX_LAUNCH_FAST(G, true, kAllModels, true);                                         \
+      HAMX_LAUNCH_RAY(G, true, kAllModels, true);                                          \
   } while (0)
       if (creg && packed)
         HAMX_LAUNCH_FAST_CREG(true);
@@ -1159,6 +1154,7 @@ int los_forward_impl(hamx_ctx *ctx, const hamx_los_desc *d, const hamx_fields *f
 #undef HAMX_LAUNCH_FAST_CREG
 #undef HAMX_LAUNCH_FAST_M
 #undef HAMX_LAUNCH_FAST
+#undef HAMX_LAUNCH_RAY
     } else {
       // CRE flux grids gather the random grids where they lie
 #define HAMX_LAUNCH_GENERIC(KERNEL, BLOCKS)                                                \

@@ -46,9 +46,9 @@ struct Phys {
   double idx, g_t1, g_t2, g_p1; // index and its Gamma factors when constant
   double tc_em1, tc_den; // temp_convert: (e^p - 1) and p^2 e^p, integrator.cc:275-279
   // CRE grid emissivities (integrator.cc:296-298,325-327,365-367,379-381):
-  // the x_fact numerators of J_tot and J_pol in their own operation orders,
-  // and the fore factor's 1.73205081 qe^3 and denominator.
-  double xft_num, xfp_num, fore_num, fore_den;
+  // the x_fact numerator of J_tot (J_pol's differs in rounding alone), and the
+  // fore factor's 1.73205081 qe^3 and denominator.
+  double xft_num, fore_num, fore_den;
   Ymw16 ymw; // HAMX_TEREG_YMW16
 };
 
@@ -335,12 +335,6 @@ __device__ inline void staged_init(const StagedCache &c, int lane) {
 __device__ inline int staged_hash(unsigned long long idx) {
   // Fibonacci hash to 32 bits, then multiply-shift onto the slots
   return static_cast<int>(((idx * 0x9E3779B97F4A7C15ull) >> 32) * kStageSlots >> 32);
-}
-
-__device__ inline unsigned long long lane_u64(unsigned long long v, int L) {
-  const uint32_t lo = __builtin_amdgcn_readlane(static_cast<uint32_t>(v), L);
-  const uint32_t hi = __builtin_amdgcn_readlane(static_cast<uint32_t>(v >> 32), L);
-  return (static_cast<unsigned long long>(hi) << 32) | lo;
 }
 
 // Value v (corner v >> 2, component v & 3) of cell `cell` into the grid.

@@ -27,7 +27,9 @@ __device__ inline void load_sync_tab(double2 *dst) {
 }
 
 // Below the short segments: the Chebyshev tables, read where they lie (few
-// samples come here; a call would cost the march its registers).
+// samples come here; a call would cost the march its registers).  Their rows above
+// u = ln 100 - 17, which the short segments took over, are those that the CPU test
+// of the tables reads.
 __device__ inline void sync_fg_low(double u, double x, double &F, double &G) {
   using namespace sync_tab;
   const double dtop = kUTop - u, fine_span = kFineN * kFineW;
