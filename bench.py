@@ -528,8 +528,7 @@ def run_cre_grid(args):
             "march_ms_per_step": march_ms / args.steps,
             "energy_bin_evaluations_per_s": S * (nE - 1) * args.steps / (march_ms * 1e-3),
             "maps_finite": finite,
-            "bound": "FP64 VALU: two logarithms, two exponentials and two Chebyshev sums "
-                     "per energy bin and sample",
+            "bound": "FP64 VALU: one exponential and two polynomials per energy bin and sample",
         },
     }
     if host is not None:

@@ -2,15 +2,16 @@
 // radial_integration (integrator.cc:23-279) as HIP kernels.
 //
 // Per shell s (nside_s, step_s samples at dist_k = d0 + (k + 1/2) delta):
-//   k_los_wave / k_los_thread : march every ray of the shell, producing the
-//       shell maps DM, FD, I, Q, U (I/Q/U temp_convert-ed, integrator.cc:99-115)
+//   k_los_fast / k_los_ray (specialised), k_los_wave / k_los_thread (generic) :
+//       march every ray of the shell, producing the shell maps DM, FD, I, Q, U
+//       (I/Q/U temp_convert-ed, integrator.cc:99-115)
 //   k_accumulate               : add the shell maps into the output maps,
 //       directly or by HEALPix interpolation at the output pixel centres
 //       (hamdis.h:698-721)
 // FD of the inner shells reaches shell s through the accumulated FD map,
 // interpolated at the ray's direction (integrator.cc:78-86).
 //
-// Two march schedules share the per-sample arithmetic:
+// The generic marches' two schedules share the per-sample arithmetic:
 //   wave   : one 64-lane wavefront per ray, lane j evaluating sample
 //            base + j; the running Faraday depth is carried across chunks
 //            and formed inside a chunk by an inclusive wave scan, so every
@@ -24,9 +25,8 @@
 // per-sample checks of integrator.cc:179-186): skipped samples contribute
 // nothing in the reference either.
 //
-// The translation unit is compiled with -ffp-contract=off and keeps the
-// reference's operation order, so the FP64 maps agree with the CPU
-// restatement to rounding.
+// The generic marches keep the reference's operation order, so the FP64 maps agree
+// with the CPU restatement to rounding (products and sums may contract).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

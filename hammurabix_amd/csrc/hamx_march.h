@@ -729,8 +729,10 @@ inline uint64_t shell_offset(const hamx_los_desc *d, uint32_t s) {
 }
 // One write_grid pass (hamx_los_forward); when ckpt is non-null and FD is
 // carried, the accumulated FD map before shell s is copied to
-// ckpt + s * npix(fd map); when shell_fd is non-null each ray's FD over
-// shell s is written to shell_fd + shell_offset(d, s) (device memory).
+// ckpt + s * npix(fd map) for s > 0 (before the first shell there is none: its
+// place is not written and must not be read); when shell_fd is non-null each
+// ray's FD over shell s is written to shell_fd + shell_offset(d, s) (device
+// memory).
 // With an arena every scratch buffer (shell maps, the mask at the shell's
 // nside, output maps the caller left NULL) is carved from it before the
 // first launch, so an arena too small fails before any work is queued.

@@ -28,7 +28,7 @@
 // at a time over two complex arrays), 72 instead of 280 for mhd, 72 instead of
 // 144 for te.  Measured per realisation, whole-array steps -> these (with the
 // engine and table work below): es 256x256x64 726 -> 304 us, es 512x512x128
-// 7.05 -> 2.24 ms, te 800x800x160 7.90 -> 2.71 ms, mhd 135x121x98 344 -> 122 us.
+// 7.05 -> 2.23 ms, te 800x800x160 7.90 -> 2.69 ms, mhd 135x121x98 344 -> 125 us.
 //
 // Half arrays: H[i][j][k], i <= nx/2, all j, k <= nz/2.  Two real lines share
 // one complex transform: X + i U in one, V in the other.
